@@ -55,7 +55,7 @@ PAL_DEBUG_FLAGS_DEFINE(decode_debug_flags)
 
 }  // namespace pal
 
-#include "prefill_tile.h"  // the fused kernel's prefill tiles
+#include "prefill_half_tile.h"  // the fused kernels' prefill tiles (and prefill_tile.h)
 
 namespace pal {
 
@@ -840,7 +840,7 @@ __global__ __launch_bounds__(kGroupThreads) void decode_stream_kernel(const Deco
 // tiles need more than half of the register file themselves.
 constexpr bool shares_cu(int hd) { return hd <= 128; }
 
-template <int HD, int TPP>
+template <int HD>
 constexpr int shared_cu_prefetch() {
   return HD == 128 ? kPrefetch - 1 : kPrefetch;
 }
@@ -956,26 +956,33 @@ __device__ __forceinline__ void fused_decode_body(const DecodeParams& p, FusedDe
   {
     bool any = false;
     const bool vec = (reinterpret_cast<uintptr_t>(p.q2seq) & 15u) == 0;
-    for (int64_t base = 0; base < n_rows; base += 4 * kGroupThreads) {
-      const int64_t r0 = base + 4 * static_cast<int64_t>(tid);
-      if (r0 >= n_rows) continue;
-      uint32_t q[6];
-      q[0] = r0 > 0 ? p.q2seq[r0 - 1] : 0xFFFFFFFFu;
-      if (vec && r0 + 4 <= n_rows) {
-        const u32x4 v = *reinterpret_cast<const u32x4*>(p.q2seq + r0);
-        q[1] = v.x;
-        q[2] = v.y;
-        q[3] = v.z;
-        q[4] = v.w;
-      } else {
+    constexpr int kPasses = 4;  // passes whose loads are in flight together
+    for (int64_t base = 0; base < n_rows; base += kPasses * 4 * kGroupThreads) {
+      uint32_t q[kPasses][6];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) q[1 + k] = r0 + k < n_rows ? p.q2seq[r0 + k] : 0xFFFFFFFFu;
+      for (int u = 0; u < kPasses; ++u) {
+        const int64_t r0 = base + 4 * (static_cast<int64_t>(u) * kGroupThreads + tid);
+        q[u][0] = r0 > 0 && r0 <= n_rows ? p.q2seq[r0 - 1] : 0xFFFFFFFFu;
+        if (vec && r0 + 4 <= n_rows) {
+          const u32x4 v = *reinterpret_cast<const u32x4*>(p.q2seq + r0);
+          q[u][1] = v.x;
+          q[u][2] = v.y;
+          q[u][3] = v.z;
+          q[u][4] = v.w;
+        } else {
+#pragma unroll
+          for (int k = 0; k < 4; ++k) q[u][1 + k] = r0 + k < n_rows ? p.q2seq[r0 + k] : 0xFFFFFFFFu;
+        }
+        q[u][5] = r0 + 4 < n_rows ? p.q2seq[r0 + 4] : 0xFFFFFFFFu;
       }
-      q[5] = r0 + 4 < n_rows ? p.q2seq[r0 + 4] : 0xFFFFFFFFu;
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const int64_t r = r0 + k;
-        if (r < n_rows && (r == 0 || q[k] != q[k + 1]) && (r + 1 == n_rows || q[k + 2] != q[k + 1])) any = true;
+      for (int u = 0; u < kPasses; ++u) {
+        const int64_t r0 = base + 4 * (static_cast<int64_t>(u) * kGroupThreads + tid);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const int64_t r = r0 + k;
+          if (r < n_rows && (r == 0 || q[u][k] != q[u][k + 1]) && (r + 1 == n_rows || q[u][k + 2] != q[u][k + 1])) any = true;
+        }
       }
     }
     if (!__syncthreads_or(any)) {
@@ -1044,27 +1051,54 @@ __device__ __forceinline__ void fused_decode_body(const DecodeParams& p, FusedDe
   fused_claim_rows<DT, HD, TPP, PF, KV8>(p, L, lone_row);
 }
 
-// The fused mixed batch in one launch (head dims up to 128).  Blocks
-// [0, n_dec) are the decode workers of the lone rows (one workgroup per CU,
-// equal static shares of the rows' KV blocks, as in decode_stream_kernel),
-// the other blocks the prefill tiles of the windows of rows.  The decode
-// blocks have the lowest ids, so the dispatcher places them first: they hold
-// one slot on every CU from the start instead of waiting for tiles to drain
-// (equal static shares started late would end late), and the tiles take the
-// other slot, then both once the decode workers are done.  The two roles
-// share one LDS allocation.
+// The fused mixed batch in one launch (head dims up to 128), in two forms.
+//
+// Side by side (fused_kernel): blocks [0, n_dec) are the decode workers of the
+// lone rows (one workgroup per CU, equal static shares of the rows' KV blocks,
+// as in decode_stream_kernel), the other blocks prefill tiles of the windows
+// of rows (prefill_half_tile.h).  Both roles keep to half of a SIMD's
+// registers, so a tile runs beside each decode workgroup and the HBM-bound
+// stream overlaps the MFMA-bound tiles.  The decode blocks have the lowest
+// ids, so the dispatcher places them first: they hold one slot on every CU
+// from the start instead of waiting for tiles to drain (equal static shares
+// started late would end late), and the tiles take the other slot, then both
+// once the decode workers are done.  The two roles share one LDS allocation.
+//
+// One after the other (fused_wide_kernel): one resident workgroup per CU first
+// streams its share of the lone rows, then takes tiles that have the whole
+// register file (prefill_tile.h).  Those tiles are 1.25 to 1.5 times as fast,
+// which wins where the decode rows are a small part of the work (fused_wide).
 static_assert(kPfThreads == kGroupThreads, "decode workers and prefill tiles share the workgroup shape");
 template <int DT, int HD, int TPP, bool KV8>
 __global__ __launch_bounds__(kGroupThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void fused_kernel(const DecodeParams dp, const PrefillParams pp, const unsigned n_dec) {
   __shared__ union {
     FusedDecodeLds d;
-    PrefillLds<HD, KV8> f;
+    HalfTileLds<HD, KV8> f;
   } lds;
   if (blockIdx.x < n_dec)
-    fused_decode_body<DT, HD, TPP, shared_cu_prefetch<HD, TPP>(), KV8>(dp, lds.d);
+    fused_decode_body<DT, HD, TPP, shared_cu_prefetch<HD>(), KV8>(dp, lds.d);
   else
-    prefill_block<DT, HD, TPP, KV8, false>(pp, blockIdx.x - n_dec, lds.f);
+    half_tile_block<DT, HD, TPP, KV8>(pp, blockIdx.x - n_dec, lds.f);
+}
+
+template <int DT, int HD, int TPP, bool KV8, int RG>
+__global__ __launch_bounds__(kGroupThreads) PAL_ACC_KERNEL
+void fused_wide_kernel(const DecodeParams dp, const PrefillParams pp) {
+  __shared__ union {
+    FusedDecodeLds d;
+    PrefillLds<HD, KV8, RG> f;
+  } lds;
+  fused_decode_body<DT, HD, TPP, kPrefetch, KV8>(dp, lds.d);
+  __syncthreads();  // the workgroup's decode wavefronts are done with their lists
+  prefill_items<DT, HD, TPP, KV8, RG, false>(pp, blockIdx.x, gridDim.x, lds.f);
+}
+
+// The claim counters, zero again for the next call: the lone rows' counter and
+// the tiles' (kQueues words, kTileClaims after it).
+__device__ __forceinline__ void rearm_claims(const DecodeParams& p) {
+  if (threadIdx.x == 0) *p.claim = 0u;
+  if (p.q2seq && threadIdx.x < kQueues) p.claim[kTileClaims + threadIdx.x] = 0u;
 }
 
 // Walks the merge list, slot v for virtual worker v (first block < 0:
@@ -1086,10 +1120,10 @@ void fused_kernel(const DecodeParams dp, const PrefillParams pp, const unsigned 
 // 8 dims (16 bytes) per lane, plus each row's (max, exp-sum): two load
 // instructions per head instead of one per element.  A segment with more
 // than three contributors is finished by the general loop.  Workgroup 0
-// re-arms the claim counter.
+// re-arms the claim counters.
 template <int DT, int HD, int TPP>
 __global__ __launch_bounds__(kGroupThreads) void decode_merge_kernel(const DecodeParams p) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) *p.claim = 0u;
+  if (blockIdx.x == 0) rearm_claims(p);
   const int lane = lane_id();
   const int wv = wave_id();
   constexpr int kCh = (HD + 127) / 128;                 // 8-dim chunks of a row per lane (16 lanes per row)
@@ -1280,7 +1314,7 @@ constexpr int kSegDims = 32;
 
 template <int DT, int HD, int TPP>
 __global__ __launch_bounds__(kGroupThreads) void decode_merge_seg_kernel(const DecodeParams p) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) *p.claim = 0u;
+  if (blockIdx.x == 0) rearm_claims(p);
   constexpr int kDs = HD < kSegDims ? HD : kSegDims;
   constexpr int kSlices = (HD + kDs - 1) / kDs;
   constexpr int kDg = kDs / 8;                 // 8-dim groups per slice
@@ -1496,24 +1530,49 @@ hipError_t dispatch_hd(const DecodeParams& p, int hd, int tpp, bool kv8, hipStre
   }
 }
 
+// One after the other instead of side by side?  The lone rows of a batch are
+// at most one or a few per sequence, so with L keys per sequence the stream
+// takes about num_seqs * L * Hkv * HD * 4 bytes / 6 TB/s and the tiles rows * L *
+// Hq * HD * 4 flops / 0.8 PFLOP/s; the tiles' gain (a fifth of their time) pays
+// for a stream that nothing overlaps while the stream is below a fifth of the
+// tiles: num_seqs * 133 / group < rows / 5.  Measured on both sides: 16
+// sequences, 20,000 rows, group 4 (rows * group / num_seqs = 4,700) 0.70 ->
+// 0.61 ms; 256 decode rows and 4 chunks of 1,024, group 8 (134) 0.94 side by
+// side, 1.04 ms one after the other.
+inline bool fused_wide(const PrefillParams& p) { return p.num_rows * p.group >= 640 * p.num_seqs; }
+
 // The fused op: the fused kernel, then the merge; head dims above 128: the
-// decode rows' kernels, then the prefill tiles.
+// prefill tiles, then the decode rows' kernels.
 template <int DT, int HD, int TPP, bool KV8>
-hipError_t launch_fused_t(const DecodeParams& dp, const PrefillParams& pp, hipStream_t stream) {
+hipError_t launch_fused_t(const DecodeParams& dp, PrefillParams pp, hipStream_t stream) {
   if constexpr (shares_cu(HD)) {
-    hipError_t err;
     const int64_t n_dec = (static_cast<int64_t>(dp.num_workers) + kWorkersPerGroup - 1) / kWorkersPerGroup;
+    const dim3 threads(kGroupThreads);
     const int64_t n_pf = static_cast<int64_t>(pp.num_units) * pp.num_kv_heads * pp.head_chunks;
     if (n_dec + n_pf > 0x7FFFFFFFll) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((fused_kernel<DT, HD, TPP, KV8>), dim3(static_cast<unsigned>(n_dec + n_pf)),
-                       dim3(kGroupThreads), 0, stream, dp, pp, static_cast<unsigned>(n_dec));
-    err = hipGetLastError();
+    const bool wide = fused_wide(pp);
+    if (wide) {
+      const hipError_t err = prefill_choose_tiles(pp, HD);
+      if (err != hipSuccess) return err;
+    }
+    if (!wide) {
+      hipLaunchKernelGGL((fused_kernel<DT, HD, TPP, KV8>), dim3(static_cast<unsigned>(n_dec + n_pf)), threads, 0, stream,
+                         dp, pp, static_cast<unsigned>(n_dec));
+    } else if (pp.row_groups == 1) {
+      hipLaunchKernelGGL((fused_wide_kernel<DT, HD, TPP, KV8, 1>), dim3(static_cast<unsigned>(n_dec)), threads, 0, stream,
+                         dp, pp);
+    } else {
+      hipLaunchKernelGGL((fused_wide_kernel<DT, HD, TPP, KV8, 2>), dim3(static_cast<unsigned>(n_dec)), threads, 0, stream,
+                         dp, pp);
+    }
+    const hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
     return launch_merge<DT, HD, TPP>(dp, stream);
   } else {
-    const hipError_t err = launch_decode_t<DT, HD, TPP, KV8>(dp, stream);
+    // (tiles first: the decode's merge re-arms the tiles' claim counters)
+    const hipError_t err = launch_prefill(pp, DT, HD, TPP, stream);
     if (err != hipSuccess) return err;
-    return launch_prefill(pp, DT, HD, TPP, stream);
+    return launch_decode_t<DT, HD, TPP, KV8>(dp, stream);
   }
 }
 

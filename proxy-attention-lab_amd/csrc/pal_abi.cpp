@@ -63,9 +63,10 @@ size_t align256(size_t n) { return (n + 255) & ~static_cast<size_t>(255); }
 
 constexpr int kMaxPageSize = 1024;  // prefill's run-time page sizes (multiples of 8)
 
-// Decode workspace layout (all offsets 256-aligned).  The claim counter at
-// byte 64 must be zero when a call starts; every call leaves it zero.  Every
-// other byte is scratch that each call writes before it reads.
+// Decode workspace layout (all offsets 256-aligned).  The claim counters at
+// bytes 64 (lone rows) and 128 .. 159 (the fused op's tiles) must be zero when
+// a call starts; every call leaves them zero.  Every other byte is scratch that
+// each call writes before it reads.
 struct DecodeLayout {
   size_t hdr, claim, cum, list, part_ml, part_o, total;
   int64_t list_cap;
@@ -334,9 +335,10 @@ int prefill_call(const void* q_prompt, const void* k_prompt, const void* v_promp
     return fail(PAL_ERR_INVALID_ARGUMENT, "[%s] inputs must be 16-byte aligned, out 8-byte aligned", op);
   const int group = num_q_heads / num_kv_heads;
   const int hg_max = group < 16 ? group : 16;
+  const int chunks = (group + 15) / 16;
   const int qt = pal::prefill_tokens_per_tile(group);
   const int64_t tiles = num_seqs * ((prompt_len + qt - 1) / qt);
-  if (tiles * num_kv_heads * ((group + 15) / 16) > 0x7fffffffLL || num_query_rows > 0x7fffffffLL)
+  if (tiles * num_kv_heads * chunks > 0x7fffffffLL || num_query_rows > 0x7fffffffLL)
     return fail(PAL_ERR_INVALID_ARGUMENT, "[%s] problem too large for one call", op);
   pal::PrefillParams p;
   p.q = static_cast<const uint16_t*>(q_prompt);
@@ -351,6 +353,7 @@ int prefill_call(const void* q_prompt, const void* k_prompt, const void* v_promp
   p.seq_lens = context_lens;
   p.q_offset = nullptr;
   p.q2seq = nullptr;
+  p.claims = nullptr;
   p.num_rows = num_query_rows;
   p.num_seqs = num_seqs;
   p.num_pages = num_pages;
@@ -363,8 +366,9 @@ int prefill_call(const void* q_prompt, const void* k_prompt, const void* v_promp
   p.group = group;
   p.head_chunks = (group + 15) / 16;
   p.hg_max = hg_max;
+  p.row_groups = 1;
+  p.hg_magic = (65536u + hg_max - 1) / hg_max;
   p.scale_log2 = scale_log2_for(head_dim);
-  p.scale_inv_log2 = 1.f / p.scale_log2;
   PAL_LOG("%s rows=%lld seqs=%lld P=%d Hq=%d Hkv=%d HD=%d TPP=%d dtype=%d fp8=%d tiles=%d stream=%p", op,
           static_cast<long long>(num_query_rows), static_cast<long long>(num_seqs), p.prompt_len, num_q_heads,
           num_kv_heads, head_dim, tokens_per_page, dtype, k_scales ? 1 : 0, p.num_units, static_cast<void*>(stream));
@@ -457,12 +461,14 @@ int fused_call(const void* queries, const void* k_pool, const void* v_pool, cons
   pp.group = group;
   pp.head_chunks = chunks;
   pp.hg_max = hg_max;
+  pp.row_groups = 1;
+  pp.hg_magic = (65536u + hg_max - 1) / hg_max;
   pp.scale_log2 = scale_log2_for(head_dim);
-  pp.scale_inv_log2 = 1.f / pp.scale_log2;
   // 2. rows alone in their run: split-K decode
   pal::DecodeParams dp = decode_params(queries, k_pool, v_pool, page_table, sequence_lengths, out,
                                        static_cast<char*>(workspace), lay, num_query_rows, num_pages,
                                        page_table_width, num_q_heads, num_kv_heads, head_dim, resident, 0);
+  pp.claims = dp.claim + pal::kTileClaims;
   dp.k_scales = k_scales;
   dp.v_scales = v_scales;
   dp.q2seq = query_to_seq_map;

@@ -9,12 +9,15 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "pal_hip_internal.h"
 
 namespace pal {
 
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef u32x4 u32x4_align8 __attribute__((aligned(8)));  // a 16-byte access at an 8-byte aligned address
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
@@ -99,11 +102,7 @@ struct Dt<kBF16> {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
                                                    __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
   }
-  // acc + lo + hi of a packed pair (one v_dot2c_f32_bf16 against (1, 1))
-  static __device__ __forceinline__ float sum2(uint32_t packed, float acc) {
-    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, packed), __builtin_bit_cast(bf16x2, 0x3F803F80u),
-                                           acc, false);
-  }
+  static constexpr uint32_t kOnes = 0x3F803F80u;  // a packed pair of ones
   // two fp8 e4m3 values (bytes 0-1, or 2-3 when hi) of w as a packed pair;
   // exact (every e4m3 value is a bf16 value): one v_cvt_scalef32_pk_bf16_fp8
   // with scale 1
@@ -138,10 +137,7 @@ struct Dt<kF16> {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a),
                                                   __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
   }
-  // acc + lo + hi of a packed pair (one v_dot2c_f32_f16 against (1, 1))
-  static __device__ __forceinline__ float sum2(uint32_t packed, float acc) {
-    return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, packed), __builtin_bit_cast(f16x2, 0x3C003C00u), acc, false);
-  }
+  static constexpr uint32_t kOnes = 0x3C003C00u;
   // two fp8 e4m3 values as a packed pair; exact (e4m3's range and 3-bit
   // mantissa fit fp16, subnormals included): one v_cvt_scalef32_pk_f16_fp8
   // with scale 1
@@ -291,6 +287,97 @@ __device__ __forceinline__ uint32_t lds_addr(const void* p) {
 __device__ __forceinline__ void copy_to_lds16(const void* base, uint32_t off, uint32_t lds) {
   asm volatile("s_nop 4\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "{m0}"(lds) : "memory");
 }
+// The same from per-lane addresses base + row * stride (row differs by lane or
+// not; no scalar base).  The multiply-add stands between the M0 write and the
+// copy, which is the wait state the copy needs.
+__device__ __forceinline__ void copy_row_to_lds16(uint64_t base, uint32_t row, uint32_t stride, uint32_t lds) {
+  uint64_t addr;
+  asm volatile("v_mad_u64_u32 %0, vcc, %1, %2, %3\n\tglobal_load_lds_dwordx4 %0, off"
+               : "=&v"(addr)
+               : "s"(stride), "v"(row), "v"(base), "{m0}"(lds)
+               : "memory", "vcc");
+}
+
+// Accumulators of the prefill tiles: eight 32 x 32 accumulators (16 registers
+// each) held for a whole tile in registers named in inline assembly, v192 ..
+// v255 (accumulators 0 .. 3) and a192 .. a255 (4 .. 7).  They are read only when
+// a row is rescaled and at the end of a tile; left to the compiler they would
+// be moved between registers at the branches around a step.  A kernel that
+// uses them is declared with PAL_ACC_KERNEL, which limits the compiler to the
+// 192 VGPRs and 192 AGPRs below them (amdgpu_num_vgpr counts half of a
+// wavefront's unified file), so nothing else touches them.  The wait states
+// between an MFMA and other instructions on its accumulator, which the
+// compiler would insert, are in acc_settle.
+constexpr int kAccReg = 192;
+#define PAL_ACC_KERNEL __attribute__((amdgpu_waves_per_eu(1, 1), amdgpu_num_vgpr(192)))
+// makes the kernel allocate the accumulators' registers
+__device__ __forceinline__ void acc_reserve() { asm volatile("" ::: "v255", "a255"); }
+
+#define PAL_ACC_MMA(type, file, acls)                                                                     \
+  asm volatile("v_mfma_f32_32x32x16_" type " " file "[%2:%3], %0, %1, " file "[%2:%3]" ::acls(a), "v"(b), \
+               "n"(kAccReg + 16 * (I & 3)), "n"(kAccReg + 16 * (I & 3) + 15))
+#define PAL_ACC_MMA_OF(type, acls)                    \
+  do {                                                \
+    if constexpr (I < 4) PAL_ACC_MMA(type, "v", acls); \
+    else PAL_ACC_MMA(type, "a", acls);                \
+  } while (0)
+// accumulator I += A * B (32x32x16); kAgprA: A comes from AGPRs (an LDS read
+// can land there directly)
+template <int DT, bool kAgprA, int I>
+__device__ __forceinline__ void acc_mma(u32x4 a, u32x4 b) {
+  if constexpr (DT == kBF16) {
+    if constexpr (kAgprA) PAL_ACC_MMA_OF("bf16", "a");
+    else PAL_ACC_MMA_OF("bf16", "v");
+  } else {
+    if constexpr (kAgprA) PAL_ACC_MMA_OF("f16", "a");
+    else PAL_ACC_MMA_OF("f16", "v");
+  }
+}
+#undef PAL_ACC_MMA_OF
+#undef PAL_ACC_MMA
+// the same with the accumulator's number a constant after unrolling
+template <int DT, bool kAgprA>
+__device__ __forceinline__ void acc_mma_at(int i, u32x4 a, u32x4 b) {
+  switch (i) {
+    case 0: acc_mma<DT, kAgprA, 0>(a, b); break;
+    case 1: acc_mma<DT, kAgprA, 1>(a, b); break;
+    case 2: acc_mma<DT, kAgprA, 2>(a, b); break;
+    case 3: acc_mma<DT, kAgprA, 3>(a, b); break;
+    case 4: acc_mma<DT, kAgprA, 4>(a, b); break;
+    case 5: acc_mma<DT, kAgprA, 5>(a, b); break;
+    case 6: acc_mma<DT, kAgprA, 6>(a, b); break;
+    default: acc_mma<DT, kAgprA, 7>(a, b); break;
+  }
+}
+// Waits until the accumulators may be read or written by other instructions
+// (an 8-pass MFMA needs 18 wait states at most), or, after such a write, by an
+// MFMA.
+__device__ __forceinline__ void acc_settle() { asm volatile("s_nop 15\n\ts_nop 7" ::: "memory"); }
+// element X (0 .. 127) of the accumulators
+template <int X>
+__device__ __forceinline__ float acc_get() {
+  float v;
+  if constexpr (X < 64)
+    asm volatile("v_mov_b32 %0, v[%1]" : "=v"(v) : "n"(kAccReg + X));
+  else
+    asm volatile("v_accvgpr_read_b32 %0, a[%1]" : "=v"(v) : "n"(kAccReg + X - 64));
+  return v;
+}
+template <int X>
+__device__ __forceinline__ void acc_put(float v) {
+  if constexpr (X < 64)
+    asm volatile("v_mov_b32 v[%1], %0" ::"v"(v), "n"(kAccReg + X));
+  else
+    asm volatile("v_accvgpr_write_b32 a[%1], %0" ::"v"(v), "n"(kAccReg + X - 64));
+}
+// f(integral_constant<int, I>) for I in [0, N)
+template <int N, int I = 0, typename F>
+__device__ __forceinline__ void static_for(const F& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    static_for<N, I + 1>(f);
+  }
+}
 
 // Transposing LDS read (ds_read_b64_tr_b16).  In each group of 16 lanes,
 // lane 4r + c points at 4 consecutive 16-bit elements, columns 4c .. 4c+3 of
@@ -301,6 +388,31 @@ __device__ __forceinline__ u32x2 lds_read_tr16(const uint16_t* p) {
   typedef __attribute__((address_space(3))) s16x4* lds_s16x4;
   const s16x4 r = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(p));
   return __builtin_bit_cast(u32x2, r);
+}
+
+// Row sums of packed probabilities on the matrix cores.  The B operand of a
+// 32x32x16 product (lane l: column l % 32, k-group l / 32, 8 values) fed as the
+// B operand of a 16x16x32 one reads as columns l % 16 with k-groups l / 16:
+// groups 0 and 2 are columns 0 .. 15, groups 1 and 3 columns 16 .. 31.  Against
+// an A of ones in even rows for groups 0, 2 and in odd rows for groups 1, 3,
+// register 0 of the result holds the sum of column l % 16 and register 1 that of
+// column l % 16 + 16, in every lane group.  (Two v_add_f32 per pair would sum
+// the unrounded values; a v_dot2c of the pair holds the matrix pipe as long as
+// this whole product, which sums 8 values per lane.)
+template <int DT>
+__device__ __forceinline__ u32x4 row_sum_ones() {
+  const int l = static_cast<int>(threadIdx.x) & (kWave - 1);
+  const uint32_t w = ((l ^ (l >> 4)) & 1) == 0 ? Dt<DT>::kOnes : 0u;
+  return u32x4{w, w, w, w};
+}
+// the lane's column (l % 32) of such sums
+__device__ __forceinline__ float row_sum_of(f32x4 sums) { return (threadIdx.x & 16) ? sums[1] : sums[0]; }
+// sums times a factor per column (f: that of the lane's own column)
+__device__ __forceinline__ void row_sum_scale(f32x4& sums, float f) {
+  const float g = __shfl_xor(f, 16, kWave);
+  const bool hi = threadIdx.x & 16;
+  sums[0] *= hi ? g : f;
+  sums[1] *= hi ? f : g;
 }
 
 // Scheduling fence: the compiler's instruction scheduler moves nothing
@@ -341,6 +453,19 @@ __device__ __forceinline__ float max_xor16(float v) {
 __device__ __forceinline__ float sum_xor16(float v) {
   const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// Largest v over the wavefront's 64 lanes, in every lane (DPP rotations inside
+// 16 lanes, then two lane swaps).
+__device__ __forceinline__ int wave_max(int v) {
+  v = max(v, __builtin_amdgcn_mov_dpp(v, 0x128, 0xf, 0xf, true));  // row_ror:8
+  v = max(v, __builtin_amdgcn_mov_dpp(v, 0x124, 0xf, 0xf, true));
+  v = max(v, __builtin_amdgcn_mov_dpp(v, 0x122, 0xf, 0xf, true));
+  v = max(v, __builtin_amdgcn_mov_dpp(v, 0x121, 0xf, 0xf, true));
+  const auto a = __builtin_amdgcn_permlane16_swap(static_cast<uint32_t>(v), static_cast<uint32_t>(v), false, false);
+  v = max(static_cast<int>(a[0]), static_cast<int>(a[1]));
+  const auto b = __builtin_amdgcn_permlane32_swap(static_cast<uint32_t>(v), static_cast<uint32_t>(v), false, false);
+  return max(static_cast<int>(b[0]), static_cast<int>(b[1]));
 }
 
 // 4 x 4 transpose of 32-bit words across the four 16-lane groups: lane

@@ -69,7 +69,8 @@ struct DecodeParams {
   int64_t num_pt_rows;           // page-table rows (sequences) in row mode
   // workspace
   int64_t* hdr;                // hdr[0] = total blocks T
-  uint32_t* claim;             // dynamic-chunk counter: 0 on entry, re-armed to 0 by the merge kernel
+  uint32_t* claim;             // dynamic-chunk counter, and 16 words on the 8 counters of the fused op's tiles:
+                               // 0 on entry, re-armed to 0 by the merge kernels
   int64_t* split_list;         // [list_cap][4] per virtual worker: {first block (< 0: none), blocks,
                                // output row, segment} of the split segment its range ends in
                                // (every live slot is written by each call before the merge reads it)
@@ -102,6 +103,9 @@ hipError_t decode_resident_workers(int dtype, int head_dim, int tokens_per_page,
 int64_t decode_virtual_workers(int64_t resident, int64_t max_blocks, int partition_size);
 hipError_t launch_decode(const DecodeParams& p, int dtype, int head_dim, int tokens_per_page, hipStream_t stream);
 
+// Distance of the fused op's tile counters from DecodeParams::claim (words).
+constexpr int kTileClaims = 16;
+
 // Causal attention over query tiles (prefill rows).  Uniform-prompt mode
 // (prompt_len > 0): the reference prefill, keys past each sequence's history
 // read from dense prompt K/V.  Window mode (prompt_len == 0): the fused op's
@@ -120,6 +124,7 @@ struct PrefillParams {
   const int32_t* seq_lens;     // window mode: keys per sequence; prompt mode: history per sequence
   const int32_t* q_offset;     // window mode: [R] keys visible to each row (before the seq_lens clamp)
   const uint32_t* q2seq;       // window mode: [R] sequence of each row
+  uint32_t* claims;            // window mode: 8 item counters, zero on entry (re-armed by the merge kernel)
   int64_t num_rows;            // R
   int64_t num_seqs;            // page-table rows
   int64_t num_pages;
@@ -132,12 +137,17 @@ struct PrefillParams {
   int group;
   int head_chunks;
   int hg_max;
+  int row_groups;        // 32-row groups per wavefront of a tile (1 or 2)
+  uint32_t hg_magic;     // ceil(2^16 / hg_max): m / hg_max = m * hg_magic >> 16 for m < 4096
   float scale_log2;      // log2(e) / sqrt(HD)
-  float scale_inv_log2;  // 1 / scale_log2
 };
 
-// Query tokens per prefill tile (and window) for a GQA group size.
+// Query tokens per prefill tile (and window) of the smaller size (one row
+// group, and half tiles) for a GQA group size.
 int prefill_tokens_per_tile(int group);
+// Chooses the size of tiles that have a CU to themselves: row_groups and num_units.
+hipError_t prefill_choose_tiles(PrefillParams& p, int head_dim);
+// (p holds the smaller tiles; the launch chooses)
 hipError_t launch_prefill(const PrefillParams& p, int dtype, int head_dim, int tokens_per_page, hipStream_t stream);
 
 // The fused mixed batch: the decode rows (dp, row mode) and the prefill tiles

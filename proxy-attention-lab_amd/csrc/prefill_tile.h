@@ -10,31 +10,51 @@
 // new tokens were written to the pages first.
 //
 // Design (MI355X):
-//  * One workgroup (4 wavefronts) owns a tile of 128 "M-rows": QT consecutive
-//    query tokens of one sequence times the (up to 16) query heads sharing a
-//    kv head, so one K/V tile in LDS serves the whole GQA group.
+//  * One workgroup (4 wavefronts, one per SIMD) has a CU to itself and owns a
+//    tile of RG * 128 "M-rows": consecutive query tokens of one sequence times
+//    the (up to 16) query heads sharing a kv head, so one K/V tile in LDS
+//    serves the whole GQA group.  A wavefront holds RG groups of 32 rows and the
+//    whole register file of its SIMD, so with RG = 2 an operand read from LDS
+//    feeds two MFMAs: with one (two wavefronts of 32 rows per SIMD), the LDS
+//    reads, the copies and the per-step work cost as much as the products.
+//    RG = 1 keeps the same code for problems of few tiles, whose time is one
+//    tile's latency (the choice is in prefill_choose_tiles).
+//  * O and the running PV accumulators live in registers above the compiler's
+//    reach (PAL_ACC_KERNEL), named by the MFMA instructions directly: as
+//    ordinary values they were copied and spilled around every step.
 //  * Per 32-key step the K and V tiles reach LDS by direct-to-LDS copies
-//    (global_load_lds_dwordx4, no registers), issued three steps ahead into four
-//    LDS buffers, with counted waits and one barrier per step.  Page ids come
-//    from an LDS copy of the tile's page-table slice.  Steps of dense prompt
-//    keys are copied the same way from the prompt rows (V rows untransposed,
-//    read back with transposing LDS reads); fp8 pages in window mode as fp8
-//    bytes, converted in the operand reads.  Steps across the history /
-//    prompt boundary, with invalid page ids, or of fp8 pages in prompt mode
-//    take a synchronous register path.
+//    (global_load_lds_dwordx4, no registers), kLeadK and kLeadV steps ahead,
+//    into four LDS buffers each, with counted waits and one barrier per step.
+//    Page ids come from an LDS copy of the tile's page-table slice.  Steps of
+//    dense prompt keys are copied the same way from the prompt rows (V rows
+//    untransposed, read back with transposing LDS reads); fp8 pages in window
+//    mode as fp8 bytes, converted in the operand reads.  Steps across the
+//    history / prompt boundary, with invalid page ids, or of fp8 pages in
+//    prompt mode take a synchronous register path.
 //  * Each wavefront computes S^T = K * Q^T with v_mfma_f32_32x32x16 (A = K
 //    from LDS, B = Q^T held in registers) and O^T += V^T * P^T with the same
 //    instruction.  In the transposed products a lane owns one M-row, so the
-//    softmax max / sum need one cross-half exchange (v_permlane32_swap) and
-//    the probabilities go into the PV MFMA without leaving the lane.  K is
-//    stored in the QK operand's row order and V rows are swizzled, so every
-//    operand read is one conflict-free 16-byte LDS access.
+//    softmax max needs one cross-half exchange (v_permlane32_swap) and the
+//    probabilities go into the PV MFMA without leaving the lane.  The sum of
+//    the rounded probabilities comes from an MFMA with ones (v_dot2 holds the
+//    matrix pipe for 16 cycles each).  K is stored in the QK operand's row
+//    order and V rows are swizzled, so every operand read is one conflict-free
+//    16-byte LDS access.
 //  * Steps are software-pipelined inside a wavefront: the QK MFMAs of step
-//    st+1 are issued among the exponentials of step st.
-//  * Online softmax in log2 units with a lazy rescale: the running max is only
-//    moved when a score exceeds it by more than 2^8, so O is rescaled rarely.
+//    st+1 are issued among the exponentials of step st, the row max of step
+//    st+1 and the step's copies among the PV MFMAs.  A whole unmasked step of
+//    128 dims takes 1,470 cycles with RG = 2, 1,050 of them MFMA.
+//  * Online softmax in log2 units, scale and max folded into one fma per score,
+//    with a lazy rescale: the running max is only moved when a score exceeds
+//    it by more than 2^8, so O is rescaled rarely.
 //  * Causal skipping: the key loop stops at the tile's largest limit, and key
 //    steps below every row's limit skip the mask arithmetic.
+//  * The output leaves through LDS as whole rows of 16-byte stores.
+//  * Measured (bf16, 32 query heads on 8 kv heads, head dim 128), against 32
+//    rows per wavefront and two workgroups per CU: 16 sequences of 1,280 rows
+//    on 1,024 cached 0.76 -> 0.62 ms (0.90 PFLOP/s over the keys seen); one
+//    prompt of 768 rows 32.4 -> 19.5 us (RG 1).  Under this load
+//    the card's clock falls to about 1.9 GHz.
 //  * Two ways to name the work, both without a planning pass: the reference
 //    prefill's uniform prompt (S sequences x P prompt rows; tiles are pure
 //    arithmetic; keys [0, hist[s]) come from pages and keys hist[s] + i from
@@ -58,9 +78,11 @@ namespace {
 
 constexpr int kPfWaves = 4;
 constexpr int kPfThreads = kPfWaves * kWave;
-constexpr int kMRows = kPfWaves * 32;  // M-rows (token, head) per workgroup
+// M-rows (token, head) of a workgroup whose wavefronts hold rg groups of 32 each
+constexpr int m_rows(int rg) { return kPfWaves * 32 * rg; }
 constexpr int kKeys = 32;              // keys per step
-constexpr int kNBuf = 4;               // LDS step buffers (read by stragglers, computed, two in flight)
+constexpr int kNBuf = 4;               // LDS step buffers, of K and of V
+constexpr int kLeadK = 5, kLeadV = 3;  // iteration st copies K of step st + kLeadK and V of step st + kLeadV
 constexpr int kPidChunk = 512;         // page ids staged per chunk; two chunks live in LDS
 static_assert(kPidChunk % kPfThreads == 0, "a page-id chunk is a whole number of loads per thread");
 constexpr float kLazyRescale = 8.f;    // log2 headroom before the running max moves
@@ -139,14 +161,30 @@ struct ItemMap {
   static constexpr int kVRowTile = TPP == 16 ? 64 : 128;
 };
 
+// Next-item claims of the window mode.  Items 8 apart (workgroups of one XCD:
+// the same few kv heads) form a queue with a counter of its own, zero when
+// the kernel starts; a workgroup claims from the queue of its XCD and, when
+// that is empty, from the others in turn.
+constexpr int kQueues = 8;
+struct Claim {
+  uint32_t queue;   // queue asked
+  uint32_t got;     // thread 0: the counter's value (in flight until read)
+  bool asked;
+  __device__ __forceinline__ void ask(const PrefillParams& p) {
+    if (threadIdx.x == 0) got = atomicAdd(p.claims + queue, 1u);
+    asked = true;
+  }
+};
+
 // One query tile: rows [row0, row0 + nrows) of sequence s (nrows <= tokens
 // per tile), query heads h0 .. h0+15 of kv head kvh.  PROMPT: the
 // uniform-prompt mode (keys below the history length from pages, the rest
 // from the dense prompt rows of sequence s); otherwise every key from pages.
-template <int DT, int HD, int TPP, bool PROMPT, bool KV8>
+template <int DT, int HD, int TPP, bool PROMPT, bool KV8, int RG>
 __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, int nrows, int64_t s, int kvh, int h0,
                                              uint16_t* k_lds_base, uint16_t* v_lds_base, uint16_t* junk_lds,
-                                             uint32_t* pid_lds, int* lim_lds, float* scl_lds) {
+                                             uint32_t* pid_lds, int* lim_lds, float* scl_lds, const int32_t* off_lds,
+                                             Claim* claim) {
   // TPP 0: the page size is p.tokens_per_page, known at run time (a
   // multiple of 8; the reference prefill takes any, paged_attention_prefill.h.metal:
   // 243-263).  Steps of history keys then take the register path, reading
@@ -157,11 +195,12 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
   const int tpp = TPP == 0 ? p.tokens_per_page : TPP;
   static_assert(TPP != 0 || (PROMPT && !KV8), "run-time page sizes: uniform-prompt mode, 16-bit pools");
   static_assert(HD % 32 == 0, "prefill needs head_dim % 32 == 0");
-  static_assert(2 * StepGeo<HD>::kLoads <= HD / 16, "a step's copies fit in its PV chunks");
+  constexpr int kMRows = m_rows(RG);
   constexpr int KS = HD / 16;  // QK k-steps of 16
   constexpr int DT32 = HD / 32;  // O^T row tiles of 32 dims
   constexpr int NI = StepGeo<HD>::kItems;
   constexpr int NL = StepGeo<HD>::kLoads;
+  constexpr int NCH = KS * RG;  // MFMAs (and chunks) of each product per step
   using IM = ItemMap<HD, TP>;
   // fp8 pools in window mode: steps are copied as fp8 bytes (16-byte items:
   // 16 dims of one key for K, 16 keys of one row for V; 2 HD items each, in
@@ -173,11 +212,12 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
   constexpr bool F8 = KV8 && !PROMPT && (TP == 32 || HD % 64 == 0);
   constexpr int NI8 = 2 * HD;
   constexpr int NL8 = (NI8 + kPfThreads - 1) / kPfThreads;
-  constexpr int NC = F8 ? NL8 : NL;  // copies per thread per step, K (and V)
+  constexpr int NC = F8 ? NL8 : NL;  // copies per thread per step of K, and as many of V
+  static_assert(2 * NC <= NCH, "a step's copies fit in its PV chunks");
   float* ks_lds = scl_lds;                   // fp8: K scale of page-table entry e in slot e % 1024
   float* vs_lds = scl_lds + 2 * kPidChunk;   // and V scale
-  auto k_lds = [&](int b) { return k_lds_base + b * NI * 8; };
-  auto v_lds = [&](int b) { return v_lds_base + b * NI * 8; };
+  auto k_lds = [&](int j) { return k_lds_base + (j & (kNBuf - 1)) * NI * 8; };  // step j's buffer
+  auto v_lds = [&](int j) { return v_lds_base + (j & (kNBuf - 1)) * NI * 8; };
 
   // tile coordinates are workgroup-uniform: keep them in scalar registers
   row0 = __builtin_amdgcn_readfirstlane(row0);
@@ -191,7 +231,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
   const int tid = threadIdx.x;
   const int lane = lane_id();
   const int w = wave_id();
-  const int col = lane & 31;  // this lane's M-row within the wave
+  const int col = lane & 31;  // this lane's M-row within a row group
   const int half = lane >> 5;
 
   const int64_t max_tokens = p.page_table_width * tpp;
@@ -213,29 +253,11 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
   // the first kPidChunk page-table entries of the row (staged into LDS once
   // the limits say how many the tile reads; entries past the sequence's
   // pages are never used).
-  const int m_row = w * 32 + col;  // this lane's M-row
-  const int my_t = m_row / p.hg_max;
-  const int my_h = m_row % p.hg_max;
-  const bool row_ok = my_t < nrows && my_t < qt && my_h < hg;
-  // Q^T operand: lane holds Q[M-row col][16kk + 8 half .. +7] for all k-steps.
-  u32x4 qv[KS];
-  {
-    const int64_t qrow = static_cast<int64_t>(row0 + (row_ok ? my_t : 0)) * p.num_q_heads + kvh * p.group + h0 +
-                         (row_ok ? my_h : 0);
-    const uint32_t qmask = row_ok ? 0xFFFFFFFFu : 0u;
-    if constexpr (F8) {
-      // fp8 steps read 16 dims of stripe 2j + half per K item: k-step 2j + e
-      // of this lane half takes dims 16 (2j + half) + 8e .. +7
-      const uint16_t* qp = p.q + qrow * HD + 16 * half;
-#pragma unroll
-      for (int kk = 0; kk < KS; ++kk)
-        qv[kk] = *reinterpret_cast<const u32x4*>(qp + 32 * (kk / 2) + 8 * (kk % 2)) & qmask;
-    } else {
-      const uint16_t* qp = p.q + qrow * HD + 8 * half;
-#pragma unroll
-      for (int kk = 0; kk < KS; ++kk) qv[kk] = *reinterpret_cast<const u32x4*>(qp + 16 * kk) & qmask;
-    }
-  }
+  constexpr int kLim = kMRows;  // lim_lds: per token; then 4 maxima and 4 minima, and the invalid-page flag
+  constexpr int kBad = kLim + 2 * kPfWaves;  // word set when a staged page id is out of range
+  const bool live_tok = tid < nrows && tid < qt;
+  int64_t tok_off = 0;
+  if (live_tok) tok_off = prompt_mode ? hist + (row0 + tid - s * p.prompt_len) + 1 : off_lds[tid];
   const uint32_t* pt = p.page_table + s * p.page_table_width;
   constexpr int kPidPre = kPidChunk / kPfThreads;  // entries of chunk 0 per thread
   uint32_t pid_pre[kPidPre];
@@ -244,28 +266,51 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
     const int e = tid + j * kPfThreads;
     pid_pre[j] = e < p.page_table_width ? pt[e] : 0u;
   }
-
-  // Row limits: M-row m = token * hg_max + head.  The previous tile's last
-  // reads of the min / max words passed a barrier since.
-  if (tid == 0) {
-    lim_lds[kMRows] = 0;
-    lim_lds[kMRows + 1] = 1 << 30;
+  int m_row[RG], my_t[RG], my_h[RG];
+  bool row_ok[RG];
+  // Q^T operand: lane holds Q[M-row col of the group][16kk + 8 half .. +7] for all k-steps.
+  // (An M-row past the tile takes row 0's query; its result is not written.)
+  u32x4 qv[RG][KS];
+#pragma unroll
+  for (int r = 0; r < RG; ++r) {
+    m_row[r] = (w * RG + r) * 32 + col;
+    my_t[r] = static_cast<int>((static_cast<uint32_t>(m_row[r]) * p.hg_magic) >> 16);
+    my_h[r] = m_row[r] - my_t[r] * p.hg_max;
+    row_ok[r] = my_t[r] < nrows && my_t[r] < qt && my_h[r] < hg;
+    const int64_t qrow = static_cast<int64_t>(row0 + (row_ok[r] ? my_t[r] : 0)) * p.num_q_heads + kvh * p.group + h0 +
+                         (row_ok[r] ? my_h[r] : 0);
+    if constexpr (F8) {
+      // fp8 steps read 16 dims of stripe 2j + half per K item: k-step 2j + e
+      // of this lane half takes dims 16 (2j + half) + 8e .. +7
+      const uint16_t* qp = p.q + qrow * HD + 16 * half;
+#pragma unroll
+      for (int kk = 0; kk < KS; ++kk)
+        qv[r][kk] = *reinterpret_cast<const u32x4*>(qp + 32 * (kk / 2) + 8 * (kk % 2));
+    } else {
+      const uint16_t* qp = p.q + qrow * HD + 8 * half;
+#pragma unroll
+      for (int kk = 0; kk < KS; ++kk) qv[r][kk] = *reinterpret_cast<const u32x4*>(qp + 16 * kk);
+    }
   }
+
+  // Key limits of the tile's tokens, and their largest and smallest per
+  // wavefront (reduced across lanes by DPP: LDS atomics on one word serialise
+  // over the lanes)
   __syncthreads();  // the previous tile is done with every LDS array
-  if (tid < kMRows) {
-    const int t = tid / p.hg_max;
-    const int hh = tid % p.hg_max;
+  {
     int lim = 0;
-    if (t < nrows && t < qt && hh < hg) {
-      int64_t off = prompt_mode ? hist + (row0 + t - s * p.prompt_len) + 1 : p.q_offset[row0 + t];
-      off = off < 0 ? 0 : off;
+    if (live_tok) {
+      const int64_t off = tok_off < 0 ? 0 : tok_off;
       lim = static_cast<int>(off < slen ? off : slen);
     }
-    lim_lds[tid] = lim;
-    if (t < nrows && t < qt && hh < hg) {
-      atomicMax(&lim_lds[kMRows], lim);
-      atomicMin(&lim_lds[kMRows + 1], lim);
+    if (tid < kMRows) lim_lds[tid] = lim;
+    const int mx = wave_max(lim);
+    const int mn = -wave_max(live_tok ? -lim : -(1 << 30));
+    if (lane == 0) {
+      lim_lds[kLim + w] = mx;
+      lim_lds[kLim + kPfWaves + w] = mn;
     }
+    if (tid == 0) lim_lds[kBad] = 0;
   }
   // fp8: the scales of those page-table entries, behind the page ids
   float ks_pre[kPidPre], vs_pre[kPidPre];
@@ -283,11 +328,17 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
     }
   }
   __syncthreads();
-  // largest and smallest limit over the tile's rows (LDS atomics, two
-  // words after the per-row limits, reset before the first barrier above)
-  const int max_lim = __builtin_amdgcn_readfirstlane(lim_lds[kMRows]);
-  const int min_lim = __builtin_amdgcn_readfirstlane(lim_lds[kMRows + 1]);
-  const int my_lim = lim_lds[m_row];
+  int max_lim = 0, min_lim = 1 << 30;
+#pragma unroll
+  for (int i = 0; i < kPfWaves; ++i) {
+    max_lim = max(max_lim, lim_lds[kLim + i]);
+    min_lim = min(min_lim, lim_lds[kLim + kPfWaves + i]);
+  }
+  max_lim = __builtin_amdgcn_readfirstlane(max_lim);
+  min_lim = __builtin_amdgcn_readfirstlane(min_lim);
+  int my_lim[RG];
+#pragma unroll
+  for (int r = 0; r < RG; ++r) my_lim[r] = row_ok[r] ? lim_lds[my_t[r]] : 0;
 
   const int64_t head_block = static_cast<int64_t>(HD) * tpp;
   const int64_t page_stride = head_block * p.num_kv_heads;
@@ -319,6 +370,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
     for (int e = chunk * kPidChunk + tid; e < min((chunk + 1) * kPidChunk, n_pid); e += kPfThreads) {
       const uint32_t pg = pt[e];
       pid_lds[e % (2 * kPidChunk)] = pg;
+      if (pg >= p.num_pages) lim_lds[kBad] = 1;
       stage_scales(e, pg);
     }
   };
@@ -327,36 +379,16 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
   // may end past it), in valid pages (and, in prompt mode, all 32 keys below
   // the history, or all of them prompt keys): one direct-to-LDS copy per
   // item, no registers, nothing to wait for here.  Every wavefront issues exactly
-  // 2*NL copies (items past the step go to a junk slot), so the wait counts
-  // are the same on every wavefront.
+  // NC copies of K and NC of V (items past the step go to a junk slot), so the
+  // wait counts are the same on every wavefront.
   // Slow step (invalid pages, history / prompt boundary, fp8 in prompt mode): register loads,
-  // masked, then LDS stores -- synchronous, so it also drains the copies in
+  // masked, then LDS stores -- synchronous, and it drains the copies in
   // flight, which keeps the counted waits safe.
   // pg0 / pg1: the pages of the step's first and (TP 16) second 16 keys.
-  constexpr bool kAllItems = NI % kPfThreads == 0;  // no wavefront has a padding copy
+  constexpr bool kAllItems = (F8 ? NI8 : NI) % kPfThreads == 0;  // no wavefront has a padding copy
   __builtin_assume(w >= 0 && w < kPfWaves);
   // page ids >= 2^32 - 1 cannot occur with fewer pages; such an id takes the slow path
   const uint32_t np32 = p.num_pages > 0xFFFFFFFFll ? 0xFFFFFFFFu : static_cast<uint32_t>(p.num_pages);
-  // Copy q of a fast step into buffer buf: the K items (q < NL) or the V
-  // items (q >= NL) of this thread's load q % NL, off0 / off1 the (page,
-  // kv head) blocks of the step's two pages.
-  auto copy_one = [&](int q, int buf, int64_t off0, int64_t off1) {
-    const int jj = q % NL;
-    const int i = tid + jj * kPfThreads;
-    const int ib = w * kWave + jj * kPfThreads;  // first item of this wavefront's load
-    const bool ok = kAllItems || ib < NI;
-    if (q < NL) {
-      const uint16_t* page = p.k_pool + (IM::k_page_half(ok ? ib : 0) ? off1 : off0);
-      const uint32_t src = 2u * static_cast<uint32_t>(ok ? IM::k_offset(i) : 0);
-      copy_to_lds16(page, src, lds_addr(ok ? k_lds(buf) + ib * 8 : junk_lds));
-    } else {
-      const uint16_t* page = p.v_pool + (IM::k_page_half(ok ? ib : 0) ? off1 : off0);
-      int d = 0, key = 0;
-      if (ok) IM::v_item(i, d, key);
-      const uint32_t src = 2u * static_cast<uint32_t>(d * TP + key % TP);
-      copy_to_lds16(page, src, lds_addr(ok ? v_lds(buf) + ib * 8 : junk_lds));
-    }
-  };
   // fp8 items.  K item i: page half ph (TP 16), stripe c (dims 16c ..
   // 16c+15), key of the step; V item i: page half ph (TP 16) or 16-key half
   // of the page row (TP 32), row d.  Item i is LDS slot i.
@@ -378,62 +410,56 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
   };
   const uint8_t* k8_pool = reinterpret_cast<const uint8_t*>(p.k_pool) + kv_head_off8;
   const uint8_t* v8_pool = reinterpret_cast<const uint8_t*>(p.v_pool) + kv_head_off8;
-  // Copy q of an fp8 fast step: K items (q < NL8) or V items of load q % NL8;
-  // boff0 / boff1: byte offsets of the step's two pages' blocks.
-  auto copy8 = [&](int q, int buf, int64_t boff0, int64_t boff1) {
-    const int jj = q % NL8;
-    const int i = tid + jj * kPfThreads;
-    const int ib = w * kWave + jj * kPfThreads;  // first item of this wavefront's load
-    const bool ok = ib < NI8;
-    int ph = 0, a = 0, b = 0;
-    uint32_t src = 0;
-    if (q < NL8) {
-      if (ok) k8_item(i, ph, a, b);
-      src = static_cast<uint32_t>((a * TP + b % TP) * 16);
+  // This lane's source address of copy q in page 0 of the pool: a copy of
+  // page pg reads page_bytes * pg further (one v_mad_u64_u32).
+  const uint32_t page_bytes = static_cast<uint32_t>(page_stride * (KV8 ? 1 : 2));
+  auto item_of = [&](int q) { return tid + q * kPfThreads; };
+  auto wave_item = [&](int q) { return w * kWave + q * kPfThreads; };  // first item of this wavefront's load
+  auto live_copy = [&](int q) { return kAllItems || wave_item(q) < (F8 ? NI8 : NI); };
+  auto k_src = [&](int q) {
+    const int i = live_copy(q) ? item_of(q) : lane;
+    if constexpr (F8) {
+      int ph, c, key;
+      k8_item(i, ph, c, key);
+      return reinterpret_cast<uint64_t>(k8_pool) + static_cast<uint32_t>((c * TP + key % TP) * 16);
     } else {
-      if (ok) v8_item(i, ph, a, b);
-      src = static_cast<uint32_t>(a * TP + b % TP);
+      return reinterpret_cast<uint64_t>(p.k_pool + kv_head_off) + 2u * static_cast<uint32_t>(IM::k_offset(i));
     }
-    const int phw = (TP == 16 && ok) ? ib / HD : 0;  // the load's page half (one page per instruction)
-    const uint8_t* page = (q < NL8 ? k8_pool : v8_pool) + (phw ? boff1 : boff0);
-    copy_to_lds16(page, ok ? src : 0u, lds_addr(ok ? (q < NL8 ? k_lds(buf) : v_lds(buf)) + ib * 8 : junk_lds));
   };
-  // An fp8 step on the register path (a page id out of range): the same
-  // items, zero for invalid pages, V keys past max_lim cleared.
-  auto slow8 = [&](int j, uint32_t pg0, uint32_t pg1) {
-    const int buf = j % kNBuf;
-    const int k0 = j * kKeys;
+  auto v_src = [&](int q) {
+    const int i = live_copy(q) ? item_of(q) : lane;
+    if constexpr (F8) {
+      int ph, d, kb;
+      v8_item(i, ph, d, kb);
+      return reinterpret_cast<uint64_t>(v8_pool) + static_cast<uint32_t>(d * TP + kb % TP);
+    } else {
+      int d, key;
+      IM::v_item(i, d, key);
+      return reinterpret_cast<uint64_t>(p.v_pool + kv_head_off) + 2u * static_cast<uint32_t>(d * TP + key % TP);
+    }
+  };
+  uint64_t ksrc[TPP == 0 ? 1 : NC], vsrc[TPP == 0 ? 1 : NC];
+  if constexpr (TPP != 0) {
 #pragma unroll
-    for (int jj = 0; jj < NL8; ++jj) {
-      const int i = tid + jj * kPfThreads;
-      if (i >= NI8) continue;
-      {
-        int ph, c, key;
-        k8_item(i, ph, c, key);
-        const uint32_t pg = ph ? pg1 : pg0;
-        PAL_DEBUG_FLAG(pg >= p.num_pages && k0 + key < max_lim, kDebugPageId);
-        u32x4 val = {0u, 0u, 0u, 0u};
-        if (pg < p.num_pages && k0 + key < max_lim)
-          val = *reinterpret_cast<const u32x4*>(k8_pool + static_cast<int64_t>(pg) * page_stride8 +
-                                                (c * TP + key % TP) * 16);
-        *reinterpret_cast<u32x4*>(k_lds(buf) + i * 8) = val;
-      }
-      {
-        int ph, d, kb;
-        v8_item(i, ph, d, kb);
-        const uint32_t pg = ph ? pg1 : pg0;
-        u32x4 val = {0u, 0u, 0u, 0u};
-        const int valid = max_lim - (k0 + kb);
-        if (pg < p.num_pages && valid > 0) {
-          val = *reinterpret_cast<const u32x4*>(v8_pool + static_cast<int64_t>(pg) * page_stride8 + d * TP + kb % TP);
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-#pragma unroll
-            for (int bb = 0; bb < 4; ++bb)
-              if (4 * e + bb >= valid) val[e] &= ~(0xFFu << (8 * bb));
-        }
-        *reinterpret_cast<u32x4*>(v_lds(buf) + i * 8) = val;
-      }
+    for (int q = 0; q < NC; ++q) {
+      ksrc[q] = k_src(q);
+      vsrc[q] = v_src(q);
+    }
+  }
+  // the page half (TP 16) a wavefront's load q reads: one page per instruction
+  auto copy_half = [&](int q) { return F8 ? (TP == 16 ? wave_item(q) / HD : 0) : IM::k_page_half(wave_item(q)); };
+  auto copy_k = [&](int q, int j, uint32_t pg0, uint32_t pg1) {
+    if constexpr (TPP != 0) {
+      const bool ok = live_copy(q);
+      const uint32_t pg = ok && copy_half(q) ? pg1 : pg0;
+      copy_row_to_lds16(ksrc[q], pg, page_bytes, lds_addr(ok ? k_lds(j) + wave_item(q) * 8 : junk_lds));
+    }
+  };
+  auto copy_v = [&](int q, int j, uint32_t pg0, uint32_t pg1) {
+    if constexpr (TPP != 0) {
+      const bool ok = live_copy(q);
+      const uint32_t pg = ok && copy_half(q) ? pg1 : pg0;
+      copy_row_to_lds16(vsrc[q], pg, page_bytes, lds_addr(ok ? v_lds(j) + wave_item(q) * 8 : junk_lds));
     }
   };
   // step j takes the fast path (fp8 pools only in window mode, as fp8 items;
@@ -463,131 +489,64 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
     const int r = key & 3;
     return HD % 128 == 0 ? 4 * r + 2 * (r >> 1) : (HD == 64 ? 2 * r : (HD == 32 ? 2 * (r >> 1) : 0));
   };
-  auto copy_dense = [&](int q, int buf, int j) {
-    const int jj = q % NL;
-    const int i = tid + jj * kPfThreads;
-    const int ib = w * kWave + jj * kPfThreads;
-    const bool ok = kAllItems || ib < NI;
-    const int64_t row0 = (dense_row0 + j * kKeys) * dense_stride + kvh * HD;  // key 0 of the step, this kv head
-    const int last = max_lim - 1 - j * kKeys;  // keys past it (tile's last step) read this key's row instead
-    if (q < NL) {  // K in its operand layout, as from pages
-      int c = 0, key = 0;
-      if (ok) IM::k_item(i, c, key);
-      const uint32_t src = 2u * static_cast<uint32_t>(min(key, last) * dense_stride + c * 8);
-      copy_to_lds16(p.k_dense + row0, src, lds_addr(ok ? k_lds(buf) + ib * 8 : junk_lds));
-    } else {
-      // raw rows: slot i = (key, 8-dim chunk c ^ vd_swz(key))
-      const int key = ok ? i / (HD / 8) : 0, c = ok ? (i % (HD / 8)) ^ vd_swz(key) : 0;
-      const uint32_t src = 2u * static_cast<uint32_t>(min(key, last) * dense_stride + c * 8);
-      copy_to_lds16(p.v_dense + row0, src, lds_addr(ok ? v_lds(buf) + ib * 8 : junk_lds));
-    }
+  // the dense row of the step's key `key` (keys past max_lim repeat the last one's row)
+  auto dense_row = [&](int j, int key) {
+    return static_cast<uint32_t>(static_cast<int>(dense_row0) + min(j * kKeys + key, max_lim - 1));
   };
-  auto issue = [&](int j, uint32_t pg0, uint32_t pg1) {
-    const int buf = j % kNBuf;
+  const uint32_t dense_bytes = static_cast<uint32_t>(dense_stride * 2);
+  auto copy_dense_k = [&](int q, int j) {  // K in its operand layout, as from pages
+    const bool ok = live_copy(q);
+    int c = 0, key = 0;
+    if (ok) IM::k_item(item_of(q), c, key);
+    const uint64_t src = reinterpret_cast<uint64_t>(p.k_dense + kvh * HD + c * 8);
+    copy_row_to_lds16(src, dense_row(j, key), dense_bytes, lds_addr(ok ? k_lds(j) + wave_item(q) * 8 : junk_lds));
+  };
+  auto copy_dense_v = [&](int q, int j) {  // raw rows: slot i = (key, 8-dim chunk c ^ vd_swz(key))
+    const bool ok = live_copy(q);
+    const int i = item_of(q);
+    const int key = ok ? i / (HD / 8) : 0, c = ok ? (i % (HD / 8)) ^ vd_swz(key) : 0;
+    const uint64_t src = reinterpret_cast<uint64_t>(p.v_dense + kvh * HD + c * 8);
+    copy_row_to_lds16(src, dense_row(j, key), dense_bytes, lds_addr(ok ? v_lds(j) + wave_item(q) * 8 : junk_lds));
+  };
+
+  // The K (V) part of a step on the register path.
+  auto slow_k = [&](int j, uint32_t pg0, uint32_t pg1) {
     const int k0 = j * kKeys;
-    if (is_dense(j)) {
+    uint16_t* kb = k_lds(j);
+    if constexpr (F8) {  // a page id out of range: the same items, zero for invalid pages
 #pragma unroll
-      for (int q = 0; q < 2 * NL; ++q) copy_dense(q, buf, j);
-      return;
-    }
-    if (TP != 16) pg1 = pg0;
-    const bool fast = is_fast(j, pg0, pg1);
-    if constexpr (F8) {
-      if (fast) {
-#pragma unroll
-        for (int q = 0; q < 2 * NL8; ++q)
-          copy8(q, buf, static_cast<int64_t>(pg0) * page_stride8, static_cast<int64_t>(pg1) * page_stride8);
-      } else {
-        slow8(j, pg0, pg1);
+      for (int jj = 0; jj < NL8; ++jj) {
+        const int i = item_of(jj);
+        if (i >= NI8) continue;
+        int ph, c, key;
+        k8_item(i, ph, c, key);
+        const uint32_t pg = ph ? pg1 : pg0;
+        PAL_DEBUG_FLAG(pg >= p.num_pages && k0 + key < max_lim, kDebugPageId);
+        u32x4 val = {0u, 0u, 0u, 0u};
+        if (pg < p.num_pages && k0 + key < max_lim)
+          val = *reinterpret_cast<const u32x4*>(k8_pool + static_cast<int64_t>(pg) * page_stride8 +
+                                                (c * TP + key % TP) * 16);
+        *reinterpret_cast<u32x4*>(kb + i * 8) = val;
       }
-      return;
-    }
-    if (fast) {
-      const int64_t off0 = static_cast<int64_t>(pg0) * page_stride + kv_head_off;
-      const int64_t off1 = static_cast<int64_t>(pg1) * page_stride + kv_head_off;
-#pragma unroll
-      for (int q = 0; q < 2 * NL; ++q) copy_one(q, buf, off0, off1);
-      return;
-    }
-    if constexpr (TPP == 0) {
-      // run-time page size: each key's page from the page table (8 keys
-      // of a V group share a page: the size is a multiple of 8)
+    } else {
 #pragma unroll
       for (int jj = 0; jj < NL; ++jj) {
-        const int i = tid + jj * kPfThreads;
+        const int i = item_of(jj);
         if (i >= NI) continue;
-        {
-          int kj, c;
-          IM::k_item(i, c, kj);
-          const int tok = k0 + kj;
-          u32x4 val = {0u, 0u, 0u, 0u};
-          if (tok < max_lim) {
-            if (tok < hist) {
-              const uint32_t pg = pt[tok / tpp];
-              PAL_DEBUG_FLAG(pg >= p.num_pages, kDebugPageId);
-              if (pg < p.num_pages)
-                val = *reinterpret_cast<const u32x4*>(p.k_pool + static_cast<int64_t>(pg) * page_stride + kv_head_off +
-                                                      (static_cast<int64_t>(c) * tpp + tok % tpp) * 8);
-            } else {
-              val = *reinterpret_cast<const u32x4*>(p.k_dense + (dense_row0 + tok) * dense_stride + kvh * HD + c * 8);
-            }
-          }
-          *reinterpret_cast<u32x4*>(k_lds(buf) + i * 8) = val;
-        }
-        {
-          int d, key;
-          IM::v_item(i, d, key);
-          const int tok = k0 + key;
-          u32x4 val = {0u, 0u, 0u, 0u};
-          if (tok < max_lim) {
-            const uint32_t pg = tok < hist ? pt[tok / tpp] : 0u;
-            const bool pg_ok = pg < p.num_pages;
-            const uint16_t* vrow = p.v_pool + static_cast<int64_t>(pg) * page_stride + kv_head_off +
-                                   static_cast<int64_t>(d) * tpp + tok % tpp;
-            if (tok + 8 <= hist) {
-              if (pg_ok) val = *reinterpret_cast<const u32x4*>(vrow);
-            } else {
-              uint32_t e16[8];
-#pragma unroll
-              for (int e = 0; e < 8; ++e) {
-                const int t2 = tok + e;
-                uint16_t x = 0;
-                if (t2 < max_lim) {
-                  if (t2 >= hist)
-                    x = p.v_dense[(dense_row0 + t2) * dense_stride + kvh * HD + d];
-                  else if (pg_ok)
-                    x = vrow[e];
-                }
-                e16[e] = x;
-              }
-              val = {e16[0] | (e16[1] << 16), e16[2] | (e16[3] << 16), e16[4] | (e16[5] << 16),
-                     e16[6] | (e16[7] << 16)};
-            }
-            const int valid = max_lim - tok;  // keys past the largest limit may hold anything
-            if (valid < 8) {
-#pragma unroll
-              for (int e = 0; e < 4; ++e)
-                val[e] &= (2 * e < valid ? 0x0000FFFFu : 0u) | (2 * e + 1 < valid ? 0xFFFF0000u : 0u);
-            }
-          }
-          *reinterpret_cast<u32x4*>(v_lds(buf) + i * 8) = val;
-        }
-      }
-      return;
-    }
-#pragma unroll
-    for (int jj = 0; jj < NL; ++jj) {
-      const int i = tid + jj * kPfThreads;
-      if (i >= NI) continue;
-      const uint32_t pg = IM::k_page_half(i) ? pg1 : pg0;
-      const bool pg_ok = pg < p.num_pages;
-      PAL_DEBUG_FLAG(!pg_ok && k0 + (IM::k_page_half(i) ? 16 : 0) < (prompt_mode ? min(max_lim, static_cast<int>(hist)) : max_lim),
-                     kDebugPageId);
-      // K: stripe c, key kj of the step
-      {
         int kj, c;
         IM::k_item(i, c, kj);
         const int tok = k0 + kj;
+        // run-time page size: each key's page from the page table
+        const uint32_t pg = TPP == 0 ? (tok < max_lim && tok < hist ? pt[tok / tpp] : 0u)
+                                     : (IM::k_page_half(i) ? pg1 : pg0);
+        const bool pg_ok = pg < p.num_pages;
+        if constexpr (TPP == 0) {
+          PAL_DEBUG_FLAG(!pg_ok, kDebugPageId);
+        } else {
+          PAL_DEBUG_FLAG(!pg_ok && k0 + (IM::k_page_half(i) ? 16 : 0) <
+                                       (prompt_mode ? min(max_lim, static_cast<int>(hist)) : max_lim),
+                         kDebugPageId);
+        }
         u32x4 val = {0u, 0u, 0u, 0u};
         if (!prompt_mode || tok < hist) {
           if (pg_ok && tok < max_lim) {
@@ -597,32 +556,66 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
               val = fp8x8_scaled<DT>(*reinterpret_cast<const u32x2*>(kp8),
                                      p.k_scales[static_cast<int64_t>(pg) * p.num_kv_heads + kvh]);
             } else {
-              val = *reinterpret_cast<const u32x4*>(p.k_pool + static_cast<int64_t>(pg) * page_stride + kv_head_off +
-                                                    IM::k_offset(i));
+              const int64_t off = TPP == 0 ? (static_cast<int64_t>(c) * tpp + tok % tpp) * 8 : IM::k_offset(i);
+              val = *reinterpret_cast<const u32x4*>(p.k_pool + static_cast<int64_t>(pg) * page_stride + kv_head_off + off);
             }
           }
         } else if (tok < max_lim) {
           val = *reinterpret_cast<const u32x4*>(p.k_dense + (dense_row0 + tok) * dense_stride + kvh * HD + c * 8);
         }
-        *reinterpret_cast<u32x4*>(k_lds(buf) + i * 8) = val;
+        *reinterpret_cast<u32x4*>(kb + i * 8) = val;
       }
-      // V: row d, keys key .. key+7 of the step
-      {
+    }
+    __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
+  };
+  auto slow_v = [&](int j, uint32_t pg0, uint32_t pg1) {
+    const int k0 = j * kKeys;
+    uint16_t* vb = v_lds(j);
+    if constexpr (F8) {  // zero for invalid pages, keys past max_lim cleared
+#pragma unroll
+      for (int jj = 0; jj < NL8; ++jj) {
+        const int i = item_of(jj);
+        if (i >= NI8) continue;
+        int ph, d, kb;
+        v8_item(i, ph, d, kb);
+        const uint32_t pg = ph ? pg1 : pg0;
+        u32x4 val = {0u, 0u, 0u, 0u};
+        const int valid = max_lim - (k0 + kb);
+        if (pg < p.num_pages && valid > 0) {
+          val = *reinterpret_cast<const u32x4*>(v8_pool + static_cast<int64_t>(pg) * page_stride8 + d * TP + kb % TP);
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int bb = 0; bb < 4; ++bb)
+              if (4 * e + bb >= valid) val[e] &= ~(0xFFu << (8 * bb));
+        }
+        *reinterpret_cast<u32x4*>(vb + i * 8) = val;
+      }
+    } else {
+#pragma unroll
+      for (int jj = 0; jj < NL; ++jj) {
+        const int i = item_of(jj);
+        if (i >= NI) continue;
+        // row d, keys key .. key+7 of the step (they share a page: page sizes are multiples of 8)
         int d, key;
         IM::v_item(i, d, key);
         const int tok = k0 + key;
-        const uint16_t* vpage = p.v_pool + static_cast<int64_t>(pg) * page_stride + kv_head_off + d * TP;
-        const uint8_t* vpage8 = reinterpret_cast<const uint8_t*>(p.v_pool) + static_cast<int64_t>(pg) * page_stride8 +
-                                kv_head_off8 + d * TP;
+        const uint32_t pg = TPP == 0 ? (tok < max_lim && tok < hist ? pt[tok / tpp] : 0u)
+                                     : (IM::k_page_half(i) ? pg1 : pg0);
+        const bool pg_ok = pg < p.num_pages;
+        const int slot = TPP == 0 ? tok % tpp : key % TP;
+        const uint16_t* vrow = p.v_pool + static_cast<int64_t>(pg) * page_stride + kv_head_off +
+                               static_cast<int64_t>(d) * tpp + slot;
+        const uint8_t* vrow8 = reinterpret_cast<const uint8_t*>(p.v_pool) + static_cast<int64_t>(pg) * page_stride8 +
+                               kv_head_off8 + d * TP + slot;
         const float vsc = KV8 && pg_ok ? p.v_scales[static_cast<int64_t>(pg) * p.num_kv_heads + kvh] : 1.f;
         u32x4 val = {0u, 0u, 0u, 0u};
         if (!prompt_mode || tok + 8 <= hist) {
           if (pg_ok && tok < max_lim) {
-            if constexpr (KV8) {
-              val = fp8x8_scaled<DT>(*reinterpret_cast<const u32x2*>(vpage8 + key % TP), vsc);
-            } else {
-              val = *reinterpret_cast<const u32x4*>(vpage + key % TP);
-            }
+            if constexpr (KV8)
+              val = fp8x8_scaled<DT>(*reinterpret_cast<const u32x2*>(vrow8), vsc);
+            else
+              val = *reinterpret_cast<const u32x4*>(vrow);
           }
         } else if (tok < max_lim) {
           // some of the 8 keys are prompt tokens (dense, strided by row)
@@ -636,10 +629,9 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
               if (!pgd) {
                 x = p.v_dense[(dense_row0 + t2) * dense_stride + kvh * HD + d];
               } else if constexpr (KV8) {
-                const uint32_t code = vpage8[(key + e) % TP];
-                x = static_cast<uint16_t>(fp8x8_scaled<DT>(u32x2{code, 0u}, vsc)[0] & 0xFFFFu);
+                x = static_cast<uint16_t>(fp8x8_scaled<DT>(u32x2{vrow8[e], 0u}, vsc)[0] & 0xFFFFu);
               } else {
-                x = vpage[(key + e) % TP];
+                x = vrow[e];
               }
             }
             e16[e] = x;
@@ -655,24 +647,49 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
             val[e] &= keep;
           }
         }
-        *reinterpret_cast<u32x4*>(v_lds(buf) + i * 8) = val;
+        *reinterpret_cast<u32x4*>(vb + i * 8) = val;
       }
+    }
+    __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
+  };
+  auto issue_k = [&](int j, uint32_t pg0, uint32_t pg1) {
+    if (is_dense(j)) {
+#pragma unroll
+      for (int q = 0; q < NC; ++q) copy_dense_k(q, j);
+    } else if (is_fast(j, pg0, pg1)) {
+#pragma unroll
+      for (int q = 0; q < NC; ++q) copy_k(q, j, pg0, pg1);
+    } else {
+      slow_k(j, pg0, pg1);
+    }
+  };
+  auto issue_v = [&](int j, uint32_t pg0, uint32_t pg1) {
+    if (is_dense(j)) {
+#pragma unroll
+      for (int q = 0; q < NC; ++q) copy_dense_v(q, j);
+    } else if (is_fast(j, pg0, pg1)) {
+#pragma unroll
+      for (int q = 0; q < NC; ++q) copy_v(q, j, pg0, pg1);
+    } else {
+      slow_v(j, pg0, pg1);
     }
   };
   // The tile's last step j, when it ends past max_lim and was copied: the
   // keys no row sees hold whatever the pages (or, in prompt mode, the row of
   // the last key) held, and a masked probability of 0 times a NaN there
   // would still be NaN, so their V entries are cleared.  Each thread clears
-  // its own items, after the barrier that saw the copies land and before the
+  // the items it copied itself, once its copies have landed and before the
   // barrier preceding the step's V reads (a slow step's entries are zero
   // already).
   auto fix_tail = [&](int j) {
+    __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
+    compiler_fence();
     const int valid0 = max_lim - j * kKeys;  // valid keys of the step, 1 .. 31
-    uint16_t* vb = v_lds(j % kNBuf);
+    uint16_t* vb = v_lds(j);
     if constexpr (F8) {  // fp8 items: 16 key bytes of one row
 #pragma unroll
       for (int jj = 0; jj < NL8; ++jj) {
-        const int i = tid + jj * kPfThreads;
+        const int i = item_of(jj);
         if (i >= NI8) continue;
         int ph, d, kb;
         v8_item(i, ph, d, kb);
@@ -693,7 +710,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
     const bool dense = is_dense(j);
 #pragma unroll
     for (int jj = 0; jj < NL; ++jj) {
-      const int i = tid + jj * kPfThreads;
+      const int i = item_of(jj);
       if (i >= NI) continue;
       u32x4* slot = reinterpret_cast<u32x4*>(vb + i * 8);
       if (dense) {  // raw rows: slot i holds 8 dims of key i / (HD / 8)
@@ -713,28 +730,19 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
     }
   };
   const bool tail_partial = max_lim % kKeys != 0;  // the last step ends past max_lim
-  // the page ids of step j (an LDS broadcast read; TP 32: one page)
   // fp8: the scales of step j's first and (TP 16) second page (LDS
   // broadcast); 0 for a page past the tile's last staged entry (the tail
   // step's keys past max_lim: their V bytes are cleared, and 0 x a stale
   // scale could be NaN)
   auto read_scales = [&](const float* arr, int j, float& s0, float& s1) {
-    const int e = j * kKeys / TP;
-    s0 = e < n_pid ? arr[e % (2 * kPidChunk)] : 0.f;
-    s1 = TP == 16 ? (e + 1 < n_pid ? arr[(e + 1) % (2 * kPidChunk)] : 0.f) : s0;
+    const int e = j * (kKeys / TP);  // (even with TP 16)
+    const float a0 = arr[e & (2 * kPidChunk - 1)], a1 = arr[(e + (TP == 16)) & (2 * kPidChunk - 1)];
+    s0 = e < n_pid ? a0 : 0.f;
+    s1 = TP == 16 ? (e + 1 < n_pid ? a1 : 0.f) : s0;
   };
-  // fp8: step j's scores times the K scale of each key's page (register r
-  // holds key 16 (r / 8) + ..., so r < 8: the first page)
-  auto scale_scores = [&](f32x16& sacc, int j) {
-    if constexpr (F8) {
-      float s0, s1;
-      read_scales(ks_lds, j, s0, s1);
-#pragma unroll
-      for (int r = 0; r < 16; ++r) sacc[r] *= half ? s1 : s0;  // the lane's keys are 16 half .. +15
-    }
-  };
+  // the page ids of step j (an LDS broadcast read; TP 32: one page)
   auto read_pids = [&](int j) {
-    const int e = (j * kKeys / TP) % (2 * kPidChunk);
+    const int e = (j * (kKeys / TP)) & (2 * kPidChunk - 1);
     u32x2 v;
     if (TP == 16) {
       v = *reinterpret_cast<const u32x2*>(pid_lds + e);  // e is even: 8-byte aligned
@@ -745,91 +753,86 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
     return v;
   };
 
-  float m_run = -INFINITY;  // running max of this lane's M-row (raw score units)
-  float l_run = 0.f;        // this lane's share of the exp-sum
-  f32x16 o[DT32];
+  float mb[RG];     // minus the running max of this lane's M-row (log2 units; 0 before its first key)
+  // exp-sum: of the probabilities as rounded for the PV product, by MFMA
+  // (fp8: this lane's share of the sum, before the V scale)
+  f32x4 l_sum[F8 ? 1 : RG];
+  float l_run[RG];
+  const u32x4 ones = row_sum_ones<DT>();
+  // O^T of row group r, row tile n (dims 32 n ..): accumulator r * DT32 + n
+  static_assert(RG * DT32 <= 8, "eight accumulators");
+  acc_reserve();
+  auto acc_zero = [&] { static_for<RG * DT32 * 16>([](auto x) { acc_put<decltype(x)::value>(0.f); }); };
 #pragma unroll
-  for (int n = 0; n < DT32; ++n)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) o[n][r] = 0.f;
+  for (int r = 0; r < RG; ++r) {
+    mb[r] = 0.f;
+    l_run[r] = 0.f;
+    if constexpr (!F8) l_sum[r] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
 
   // Key order inside a 32-key step.  The QK product's A operand takes key
   // kperm(m) as its row m (bits 2 and 3 of m swapped); then the 8 scores a
   // lane feeds into each PV k-step are 8 consecutive keys, and the V^T operand
   // is one 16-byte LDS read per lane.  LDS already holds K in this row order.
 
-  // S^T[key][M-row] = sum_d K[key][d] Q[M-row][d] for step st (raw scores).
-  auto read_k = [&](int st, u32x4 (&ka)[KS]) {
-    const int buf = st % kNBuf;
-    if constexpr (F8) {  // lane: key kperm_f8(col), all 16 dims of stripe 2j + half: k-steps 2j and 2j + 1
-      const int key = kperm_f8(col);
-      const uint8_t* kb = reinterpret_cast<const uint8_t*>(k_lds(buf));
-#pragma unroll
-      for (int j = 0; j < KS / 2; ++j) {
-        const int c = 2 * j + half;
-        const int slot = TP == 16 ? (key / 16) * HD + c * 16 + ((key % 16) ^ (key >= 16 ? 12 : 0)) : c * 32 + col;
-        const u32x4 v = *reinterpret_cast<const u32x4*>(kb + slot * 16);
-        // exact in 16 bits; the K scale goes on the scores
-        ka[2 * j] = fp8x8_exact<DT>(u32x2{v.x, v.y});
-        ka[2 * j + 1] = fp8x8_exact<DT>(u32x2{v.z, v.w});
-      }
-      return;
-    }
-#pragma unroll
-    for (int kk = 0; kk < KS; ++kk) {
-      const int c = 2 * kk + half;  // stripe of dims 16kk + 8 half .. +7
-      ka[kk] = *reinterpret_cast<const u32x4*>(k_lds(buf) + IM::k_slot(col, c) * 8);
-    }
+  // S^T[key][M-row] = sum_d K[key][d] Q[M-row][d]: k-step kk's K operand.
+  // fp8: lane: key kperm_f8(col), all 16 dims of stripe 2j + half: k-steps 2j
+  // and 2j + 1 (read raw into k16, converted by the k-step's chunk).
+  auto read_k = [&](int j, int kk) {
+    const int c = 2 * kk + half;  // stripe of dims 16kk + 8 half .. +7
+    return *reinterpret_cast<const u32x4*>(k_lds(j) + IM::k_slot(col, c) * 8);
+  };
+  auto read_k8 = [&](int j, int kj) {
+    const int key = kperm_f8(col);
+    const int c = 2 * kj + half;
+    const int slot = TP == 16 ? (key / 16) * HD + c * 16 + ((key % 16) ^ (key >= 16 ? 12 : 0)) : c * 32 + col;
+    return *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint8_t*>(k_lds(j)) + slot * 16);
   };
   // V^T operand bases: k-step kk takes keys 16kk + 8 half .. +7; row tile n
   // (dims 32n + col) sits kVRowTile slots further
   const int v_base[2] = {IM::v_slot(col, 8 * half), IM::v_slot(col, 16 + 8 * half)};
-  // register r holds key k0 + 16 (r/8) + 8 half + 4 ((r/4)%2) + r%4 of
-  // M-row col (fp8 steps: key k0 + 16 half + r).  Scores stay raw (the scale is positive, so maxima commute
-  // with it); the exponent is one fma: s * scale_log2 - m * scale_log2.  The
-  // rounding of m * scale_log2 is common to a step's keys and cancels in the
-  // normalisation while that product stays below ~2^14 (log2 units; trained
-  // models' logits are far below); it grows with the product and overflows
-  // exp2 past ~2^31.  An exact (s - m) * scale_log2 costs 16 more VALU
-  // instructions per step (a rarely taken branch to it: 3 % on config 4).
-  auto mask_score = [&](f32x16& sacc, int r, int st) {
-    const int key = F8 ? st * kKeys + 16 * half + r
-                       : st * kKeys + 16 * (r >> 3) + 8 * half + 4 * ((r >> 2) & 1) + (r & 3);
-    if (key >= my_lim) sacc[r] = -INFINITY;
-  };
-  // Given this lane's max bm of a step's scores: moves the running max to the
-  // row max if it grew by more than the headroom (rescaling this row's O and
-  // exp-sum), and returns the exponent offset of the step.
-  auto update_max = [&](float bm) {
-    bm = max_xor32(bm);
-    if (__ballot(bm > m_run + kLazyRescale * p.scale_inv_log2)) {
-      const bool grow = bm > m_run + kLazyRescale * p.scale_inv_log2;
-      const float m_new = fmaxf(m_run, bm);
-      const float alpha = (m_run == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f((m_run - m_new) * p.scale_log2);
-      // rows whose max did not grow by more than the headroom keep their scale
-      const float a = grow ? alpha : 1.f;
-      if (grow) m_run = m_new;
-      l_run *= a;
-#pragma unroll
-      for (int n = 0; n < DT32; ++n) o[n] *= a;
+  // Score register x of a step holds key k0 + 16 (x/8) + 8 half + 4 ((x/4)%2) +
+  // x%4 of M-row col (fp8 steps: key k0 + 16 half + x).  The exponent is one
+  // fma: s * scale_log2 - m * scale_log2.  The rounding of m * scale_log2 is
+  // common to a step's keys and cancels in the normalisation while that
+  // product stays below ~2^14 (log2 units; trained models' logits are far
+  // below); it grows with the product and overflows exp2 past ~2^31.  An exact
+  // (s - m) * scale_log2 costs one more VALU instruction per score.
+  // keys of step j's half-step that M-row r sees: register x is visible while
+  // its key's place in the lane's order is below
+  auto seen = [&](int r, int j) { return my_lim[r] - j * kKeys - (F8 ? 16 : 8) * half; };
+  auto place = [](int x) { return F8 ? x : 16 * (x >> 3) + 4 * ((x >> 2) & 1) + (x & 3); };
+  // fp8: the K scale of each key's page rides on the score scale (the lane's
+  // keys are one page half)
+  auto score_scale = [&](int j) {
+    if constexpr (F8) {
+      float s0, s1;
+      read_scales(ks_lds, j, s0, s1);
+      return p.scale_log2 * (half ? s1 : s0);
+    } else {
+      return p.scale_log2;
     }
-    return (m_run == -INFINITY) ? 0.f : -m_run * p.scale_log2;
   };
 
-  // Pipeline.  Memory: three steps ahead.  Iteration st waits for step st+1
-  // (step st+2 may still be in flight), passes the barrier, and then issues
-  // the copies of step st+3 into the buffer of step st-1, which every
-  // wavefront finished reading before the barrier; hence four buffers.
-  // Compute, inside a wavefront: all operand reads of the iteration go out
-  // first; the QK MFMAs of step st+1 run beside the exponentials of step st,
-  // and the PV MFMAs of step st beside the exp-sum of step st and the row max
-  // of step st+1, which gives the next iteration its exponent offset.
+  // Pipeline (iteration st; step st's exponents e are in registers, and the K
+  // operands of step st+1).
+  //  Memory: iteration st issues the copies of K step st+5 and V step st+3, in
+  //  that order.  At its top it waits for those issued three iterations ago or
+  //  earlier (K step st+2, V step st) and passes the barrier.  K step st+2 is
+  //  read in this iteration's second half, so buffers hold K steps st+2 ..
+  //  st+5 and V steps st .. st+3; the copies overwrite K step st+1 and V step
+  //  st-1, which every wavefront finished reading before the barrier.
+  //  Compute, first half: the QK MFMAs of step st+1 beside the exponentials
+  //  of step st and the V operand reads; second half: the PV MFMAs of step st
+  //  beside the exp-sum of step st, the exponents and row max of step st+1 and
+  //  the K operand reads of step st+2.
   if (nsteps > 0) {
 #pragma unroll
     for (int j = 0; j < kPidPre; ++j) {  // chunk 0, loaded above
       const int e = tid + j * kPfThreads;
       if (e < n_pid) {
         pid_lds[e] = pid_pre[j];
+        if (pid_pre[j] >= p.num_pages) lim_lds[kBad] = 1;
         if constexpr (F8) {
           ks_lds[e] = ks_pre[j];
           vs_lds[e] = vs_pre[j];
@@ -838,293 +841,617 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
     }
     if (n_pid > kPidChunk) stage_pids(1);
   }
+  // The query loads are waited for here, on every path: the compiler would
+  // otherwise wait for them (and so for the copies, which it does not see)
+  // inside the step loops.
+#pragma unroll
+  for (int r = 0; r < RG; ++r)
+#pragma unroll
+    for (int kk = 0; kk < KS; ++kk) asm volatile("" : "+v"(qv[r][kk]));
   __syncthreads();
-  auto wait_barrier = [&](int pending_steps) {  // all but the pending_steps youngest steps' copies landed
-    compiler_fence();
-    if (pending_steps >= 2)
-      __builtin_amdgcn_s_waitcnt(vmcnt_only(4 * NC));
-    else if (pending_steps == 1)
-      __builtin_amdgcn_s_waitcnt(vmcnt_only(2 * NC));
-    else
-      __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
+  auto barrier = [&] {
     __builtin_amdgcn_s_waitcnt(kLgkmZero);
     __builtin_amdgcn_s_barrier();
     compiler_fence();
   };
-  f32x16 s_cur;
+  // all copies but those of the last two iterations landed (fewer were
+  // issued near the tile's end: the V copies only, or none)
+  auto wait_top = [&](int st) {
+    compiler_fence();
+    if (st + kLeadK - 1 < nsteps)
+      __builtin_amdgcn_s_waitcnt(vmcnt_only(4 * NC));
+    else if (st + kLeadV - 1 < nsteps)
+      __builtin_amdgcn_s_waitcnt(vmcnt_only(2 * NC));
+    else
+      __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
+    barrier();
+  };
+  f32x16 e_cur[RG];
+  u32x4 ka[F8 ? KS / 2 : KS];  // K operands of the next QK product (fp8: raw items of two k-steps)
+  auto k_operand = [&](int kk) {
+    if constexpr (F8) {  // exact in 16 bits; the K scale goes on the scores
+      const u32x4 v = ka[kk / 2];
+      return fp8x8_exact<DT>(kk % 2 ? u32x2{v.z, v.w} : u32x2{v.x, v.y});
+    } else {
+      return ka[kk];
+    }
+  };
+  auto read_k_all = [&](int j) {
 #pragma unroll
-  for (int r = 0; r < 16; ++r) s_cur[r] = 0.f;
-  float mb = 0.f;
+    for (int kk = 0; kk < (F8 ? KS / 2 : KS); ++kk) ka[kk] = F8 ? read_k8(j, kk) : read_k(j, kk);
+  };
+  const int paged_full = (TPP != 0 && (!KV8 || F8)) ? paged_keys / kKeys : 0;  // whole steps in pages
   if (nsteps > 0) {
-    for (int j = 0; j < 3 && j < nsteps; ++j) {
-      const u32x2 pg = read_pids(j);
-      issue(j, __builtin_amdgcn_readfirstlane(pg.x), __builtin_amdgcn_readfirstlane(pg.y));
+    auto pids = [&](int j, uint32_t& a, uint32_t& b) {
+      const u32x2 v = read_pids(j);
+      a = __builtin_amdgcn_readfirstlane(v.x);
+      b = TP == 16 ? __builtin_amdgcn_readfirstlane(v.y) : a;
+    };
+    // K 0, K 1, V 0, K 2, V 1, K 3, V 2
+    if (paged_full >= 4 && __builtin_amdgcn_readfirstlane(lim_lds[kBad]) == 0) {
+      u32x2 pg[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) pg[j] = read_pids(j);
+#pragma unroll
+      for (int t = 0; t < 7; ++t) {
+        const bool is_k = t == 0 || (t & 1);
+        const int j = is_k ? (t + 1) / 2 : t / 2 - 1;
+#pragma unroll
+        for (int q = 0; q < NC; ++q) {
+          if (is_k)
+            copy_k(q, j, pg[j].x, pg[j].y);
+          else
+            copy_v(q, j, pg[j].x, pg[j].y);
+        }
+      }
+    } else {
+#pragma unroll 1
+      for (int t = 0; t < 7; ++t) {
+        const bool is_k = t == 0 || (t & 1);
+        const int j = is_k ? (t + 1) / 2 : t / 2 - 1;
+        if (j >= nsteps) continue;
+        uint32_t pa, pb;
+        pids(j, pa, pb);
+        if (is_k)
+          issue_k(j, pa, pb);
+        else
+          issue_v(j, pa, pb);
+      }
     }
-    wait_barrier(min(nsteps - 1, 2));  // step 0 has landed
+    acc_zero();
+    compiler_fence();
+    if (nsteps >= 4)
+      __builtin_amdgcn_s_waitcnt(vmcnt_only(5 * NC));  // K steps 0 and 1
+    else
+      __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
     if (nsteps == 1 && tail_partial) fix_tail(0);
-    u32x4 ka[KS];
-    read_k(0, ka);
+    barrier();
+    read_k_all(0);
+    f32x16 s0[RG];
 #pragma unroll
-    for (int kk = 0; kk < KS; ++kk) s_cur = Dt<DT>::mma32x32x16(ka[kk], qv[kk], s_cur);
-    scale_scores(s_cur, 0);
-    float bm = -INFINITY;
+    for (int r = 0; r < RG; ++r)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      if (min_lim < kKeys) mask_score(s_cur, r, 0);
-      bm = fmaxf(bm, s_cur[r]);
-    }
-    mb = update_max(bm);
-  }
-  // Steps whose next step needs no mask (every row sees all its keys) run
-  // the unmasked body.  The last step is always in the masked part, whose
-  // mask also discards the scores of the stale buffer it reads as "next".
-  const int n_main = max(0, min(nsteps, min_lim / kKeys - 1));
-  // dense_v: step st's V rows were copied untransposed (a dense prompt step);
-  // each combination is its own loop body, so the operand reads carry no
-  // per-chunk branch.
-  auto step = [&](auto masked, auto dense_v, int st) {
-    constexpr bool kMask = decltype(masked)::value;
-    constexpr bool vdense = decltype(dense_v)::value;
-    wait_barrier(st + 2 < nsteps ? 1 : 0);  // step st+1 has landed
-    const int j = st + 3;
-    const u32x2 pgv = read_pids(j);  // used after the MFMAs (in bounds whether or not step j exists)
-    u32x4 ka[KS];
-    read_k(st + 1, ka);
-    if (kMask && st + 2 == nsteps && tail_partial) fix_tail(st + 1);
-    float pe[16];
-#pragma unroll
-    for (int r = 0; r < 16; ++r) pe[r] = fmaf(s_cur[r], p.scale_log2, mb);
-    // The rest is written in issue order, chunk by chunk, with scheduling
-    // fences between chunks (the compiler would otherwise keep two operand
-    // reads in flight, wait before every MFMA and bunch the vector work):
-    // each QK MFMA of step st+1 (K operands all read above) goes out with one
-    // V operand read of step st and a share of step st's exponentials and
-    // conversions; each PV MFMA of step st with a share of the exp-sum and of
-    // the row max of step st+1.
-    sched_fence();
-    // Raised wave priority through the MFMA chunks: the other wavefront on
-    // the SIMD is then more often in its vector/LDS phase while this one
-    // issues MFMAs (measured +1 % on config 4, -1 to -3 % time on config 5).
-    __builtin_amdgcn_s_setprio(1);
-    const int vbuf = st % kNBuf;
-    float vs0 = 1.f, vs1 = 1.f;  // fp8: V scales of step st's pages
-    if constexpr (F8) read_scales(vs_lds, st, vs0, vs1);
-    f32x16 s_next;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) s_next[r] = 0.f;
-    u32x4 va[KS];  // PV operand m: k-step m / DT32, row tile m % DT32 (KS == 2 * DT32)
-    u32x4 v16[F8 ? DT32 : 1];  // fp8: row tile t's item (16 keys of one row), both PV k-steps
-    uint32_t pp[8];  // packed probabilities of the lane's scores 2q, 2q+1
+      for (int x = 0; x < 16; ++x) s0[r][x] = 0.f;
 #pragma unroll
     for (int kk = 0; kk < KS; ++kk) {
-      s_next = Dt<DT>::mma32x32x16(ka[kk], qv[kk], s_next);
-      if constexpr (vdense) {
-        // raw rows: V[key][d] in chunk (d / 8) ^ vd_swz(key) of row key.  Lane
-        // 4r + c of a 16-lane group points at keys kg + 4t + r, dims d0 + 4c ..
-        // +3 (d0 = 32 (kk % DT32) + (col & 16)); the transposing read hands
-        // lane j dim d0 + j = col + 32 (kk % DT32) of those 4 keys.
-        const int l16 = lane & 15;
-        const int key = 16 * (kk / DT32) + 8 * half + (l16 >> 2);
-        const int d = 32 * (kk % DT32) + (col & 16) + 4 * (l16 & 3);
-        const uint16_t* vr = v_lds(vbuf) + key * HD + (((d >> 3) ^ vd_swz(key)) << 3) + (d & 7);
-        const u32x2 lo = lds_read_tr16(vr);           // keys kg .. kg+3
-        const u32x2 hi = lds_read_tr16(vr + 4 * HD);  // keys kg+4 .. kg+7 (vd_swz(key + 4) = vd_swz(key))
-        va[kk] = u32x4{lo[0], lo[1], hi[0], hi[1]};
-      } else if constexpr (F8) {
-        // chunk t < DT32 reads row tile t's item (half, d = col + 32 t): keys
-        // 16 half .. +7 for k-step 0 (operand t), +8 .. +15 for k-step 1
-        // (operand t + DT32).  Exact in 16 bits; the V scale is on P.  Each
-        // half is converted in a later chunk than its read (the LDS read has
-        // landed) and consumed there, so the conversions are not sunk to the
-        // PV MFMAs.
-        if (kk < DT32)
-          v16[kk] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint8_t*>(v_lds(vbuf)) +
-                                                    (half * HD + col + 32 * kk) * 16);
-        if (kk >= 1 && kk <= DT32) {
-          va[kk - 1] = fp8x8_exact<DT>(u32x2{v16[kk - 1].x, v16[kk - 1].y});
-          asm volatile("" ::"v"(va[kk - 1]));
-        }
-        if (kk >= DT32) {
-          va[kk] = fp8x8_exact<DT>(u32x2{v16[kk - DT32].z, v16[kk - DT32].w});
-          asm volatile("" ::"v"(va[kk]));
-        }
-      } else {
-        va[kk] = *reinterpret_cast<const u32x4*>(v_lds(vbuf) + (v_base[kk / DT32] + (kk % DT32) * IM::kVRowTile) * 8);
-      }
+      const u32x4 kop = k_operand(kk);
 #pragma unroll
-      for (int r = kk * 16 / KS; r < (kk + 1) * 16 / KS; ++r) pe[r] = __builtin_amdgcn_exp2f(pe[r]);
-#pragma unroll
-      for (int q = kk * 8 / KS; q < (kk + 1) * 8 / KS; ++q) {
-        if constexpr (F8) {  // the exp-sum of the probabilities, then P times its key's page V scale
-          const float sv = half ? vs1 : vs0;  // the lane's keys 16 half .. +15: page half (TP 32: vs1 == vs0)
-          l_run += pe[2 * q] + pe[2 * q + 1];
-          pp[q] = Dt<DT>::pack2(pe[2 * q] * sv, pe[2 * q + 1] * sv);
-        } else {
-          pp[q] = Dt<DT>::pack2(pe[2 * q], pe[2 * q + 1]);
-        }
-        // consumed here, so the exponentials and the conversion stay in this
-        // chunk beside its QK MFMA (the fences only bind the scheduler: code
-        // motion would otherwise sink them to the PV MFMAs that use them,
-        // past the copy branches)
-        asm volatile("" ::"v"(pp[q]));
-      }
-      sched_fence();
+      for (int r = 0; r < RG; ++r) s0[r] = Dt<DT>::mma32x32x16(kop, qv[r][kk], s0[r]);
     }
-    const u32x4 pb[2] = {u32x4{pp[0], pp[1], pp[2], pp[3]}, u32x4{pp[4], pp[5], pp[6], pp[7]}};
-    scale_scores(s_next, st + 1);
-    // O^T[d][M-row] += sum_key V[key][d] P[M-row][key]; k-step kk takes
-    // registers 8kk .. 8kk+7 = keys 16kk + 8 half .. +7.
-    float bm = -INFINITY;
-    // A fast step j issues its copies one per PV chunk (the first 2 NL
-    // chunks), so the wavefront's MFMAs run while an issue waits for the
-    // memory pipeline (measured 3 % on config 4 against issuing them all
-    // after the chunks); other steps take the synchronous path below.
-    const uint32_t jp0 = __builtin_amdgcn_readfirstlane(pgv.x);
-    const uint32_t jp1 = TP == 16 ? __builtin_amdgcn_readfirstlane(pgv.y) : jp0;
-    const bool jdense = j < nsteps && (vdense || is_dense(j));  // steps after a dense one are dense
-    const bool jfast = j < nsteps && (jdense || is_fast(j, jp0, jp1));
-    const int64_t joff0 = static_cast<int64_t>(jp0) * page_stride + kv_head_off;
-    const int64_t joff1 = static_cast<int64_t>(jp1) * page_stride + kv_head_off;
-#pragma unroll
-    for (int m = 0; m < KS; ++m) {
-      if (jfast && m < 2 * NC) {
-        if constexpr (F8)
-          copy8(m, j % kNBuf, static_cast<int64_t>(jp0) * page_stride8, static_cast<int64_t>(jp1) * page_stride8);
-        else if (jdense)
-          copy_dense(m, j % kNBuf, j);
-        else
-          copy_one(m, j % kNBuf, joff0, joff1);
-      }
-      o[m % DT32] = Dt<DT>::mma32x32x16(va[m], pb[m / DT32], o[m % DT32]);
-      // the exp-sum adds the probabilities as rounded for the PV product
-#pragma unroll
-      for (int q = m * 8 / KS; q < (m + 1) * 8 / KS; ++q)
-        if constexpr (!F8) l_run = Dt<DT>::sum2(pp[q], l_run);
-#pragma unroll
-      for (int r = m * 16 / KS; r < (m + 1) * 16 / KS; ++r) {
-        if (kMask) mask_score(s_next, r, st + 1);
-        bm = fmaxf(bm, s_next[r]);
-      }
-      sched_fence();
+    read_k_all(1);
+    barrier();  // every wavefront has read K step 0: its buffer takes step 4
+    if (nsteps > 4) {
+      uint32_t pa, pb;
+      pids(4, pa, pb);
+      issue_k(4, pa, pb);
     }
-    __builtin_amdgcn_s_setprio(0);
-    mb = update_max(bm);
-    if (j < nsteps) {
-      // entering page-id chunk q (q >= 1): stage chunk q + 1 over chunk q - 1,
-      // whose last reader finished before this iteration's barrier; the next
-      // barriers publish it long before its first reader
-      const int e0 = j * kKeys / TP;
-      if (e0 % kPidChunk == 0 && e0 > 0 && e0 + kPidChunk < n_pid) stage_pids(e0 / kPidChunk + 1);
-      if (!jfast) issue(j, jp0, jp1);
-    }
-    s_cur = s_next;
-  };
-  // prompt mode: steps from ceil(hist / 32) on are dense (the one across the
-  // boundary, if any, is not)
-  const int fd = PROMPT ? min(nsteps, static_cast<int>((hist + kKeys - 1) / kKeys)) : nsteps;
-  int st = 0;
-  for (; st < min(n_main, fd); ++st) step(std::false_type{}, std::false_type{}, st);
-  if constexpr (PROMPT)
-    for (; st < n_main; ++st) step(std::false_type{}, std::true_type{}, st);
-  for (; st < fd; ++st) step(std::true_type{}, std::false_type{}, st);
-  if constexpr (PROMPT)
-    for (; st < nsteps; ++st) step(std::true_type{}, std::true_type{}, st);
-
-  // ---- normalise and write: lane holds O[M-row col][32n + 8(r/4) + 4 half + r%4]
-  float l = sum_xor32(l_run);
-  if (row_ok) {
-    const float inv = l > 0.f ? 1.f / l : 0.f;
-    const int64_t orow = static_cast<int64_t>(row0 + my_t) * p.num_q_heads + kvh * p.group + h0 + my_h;
-    uint16_t* op = p.out + orow * HD;
+    const float sc = score_scale(0);
 #pragma unroll
-    for (int n = 0; n < DT32; ++n) {
+    for (int r = 0; r < RG; ++r) {
+      float bm = -INFINITY;
 #pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4) {
-        const int d = 32 * n + 8 * q4 + 4 * half;
-        const u32x2 pk = {Dt<DT>::pack2(o[n][4 * q4 + 0] * inv, o[n][4 * q4 + 1] * inv),
-                          Dt<DT>::pack2(o[n][4 * q4 + 2] * inv, o[n][4 * q4 + 3] * inv)};
-        *reinterpret_cast<u32x2*>(op + d) = pk;
+      for (int x = 0; x < 16; ++x) {
+        e_cur[r][x] = s0[r][x] * sc;
+        if (min_lim < kKeys && place(x) >= seen(r, 0)) e_cur[r][x] = -INFINITY;
+        bm = fmaxf(bm, e_cur[r][x]);
       }
+      bm = max_xor32(bm);
+      mb[r] = bm == -INFINITY ? 0.f : -bm;
+#pragma unroll
+      for (int x = 0; x < 16; ++x) e_cur[r][x] += mb[r];
     }
   }
-}
+  // One iteration.  kFast: step st+1 needs no mask and the iteration's copies
+  // are plain (pages known to be valid, or whole dense steps): no test of a
+  // page id and no branch in the body.  Otherwise scores are masked and each
+  // copy's route is looked up.  kLast: the tile's last step (nothing follows).
+  // vdense: step st's V rows were copied untransposed (a dense prompt step);
+  // each combination is its own loop body, so the operand reads carry no
+  // per-chunk branch.
+  enum { kFast, kAny, kLast };
+  auto step = [&](auto mode_c, auto dense_v, int st) {
+    constexpr int kMode = decltype(mode_c)::value;
+    constexpr bool vdense = decltype(dense_v)::value;
+    if constexpr (kMode == kFast) {
+      compiler_fence();
+      __builtin_amdgcn_s_waitcnt(vmcnt_only(4 * NC));
+      barrier();
+    } else {
+      wait_top(st);
+    }
+    const int jk = st + kLeadK, jv = st + kLeadV;
+    const u32x2 pgk = read_pids(jk), pgv = read_pids(jv);  // used in the second half (in bounds whether or not the steps exist)
+    if (kMode == kAny && st + 2 == nsteps && tail_partial) fix_tail(st + 1);
+    // The rest is written in issue order, chunk by chunk, with scheduling
+    // fences between chunks (the compiler would otherwise keep two operand
+    // reads in flight, wait before every MFMA and bunch the vector work).
+    sched_fence();
+    float vs0 = 1.f, vs1 = 1.f;  // fp8: V scales of step st's pages
+    if constexpr (F8) read_scales(vs_lds, st, vs0, vs1);
+    const float svs = half ? vs1 : vs0;  // the lane's keys 16 half .. +15: page half (TP 32: vs1 == vs0)
+    f32x16 s_next[RG];
+#pragma unroll
+    for (int r = 0; r < RG; ++r)
+#pragma unroll
+      for (int x = 0; x < 16; ++x) s_next[r][x] = 0.f;
+    u32x4 va[KS];  // PV operand m: k-step m / DT32, row tile m % DT32 (KS == 2 * DT32)
+    u32x4 v16[F8 ? DT32 : 1];  // fp8: row tile t's item (16 keys of one row), both PV k-steps
+    u32x4 pp[RG][2];  // packed probabilities of the lane's scores, 8 per PV k-step
+    // probability pair q (row group q / 8): exponentials, and one chunk later
+    // (past their latency) the conversion
+    auto pair_exp = [&](int q) {
+      const int r = q / 8, i = q % 8;
+      e_cur[r][2 * i] = __builtin_amdgcn_exp2f(e_cur[r][2 * i]);
+      e_cur[r][2 * i + 1] = __builtin_amdgcn_exp2f(e_cur[r][2 * i + 1]);
+    };
+    auto pair_pack = [&](int q) {
+      const int r = q / 8, i = q % 8;
+      const float p0 = e_cur[r][2 * i], p1 = e_cur[r][2 * i + 1];
+      if constexpr (F8)  // P times its key's page V scale (the exp-sum stays unscaled)
+        pp[r][i / 4][i % 4] = Dt<DT>::pack2(p0 * svs, p1 * svs);
+      else
+        pp[r][i / 4][i % 4] = Dt<DT>::pack2(p0, p1);
+      // Held here: code motion would otherwise sink the conversion to the PV
+      // MFMA that reads it, which (as inline assembly) must stand two
+      // instructions or more behind it.
+      if (i % 4 == 3) asm volatile("" : "+v"(pp[r][i / 4]));
+    };
+    auto pair_sum = [&](int q) {
+      if constexpr (!F8) return;
+      const int r = q / 8, i = q % 8;
+      l_run[r] += e_cur[r][2 * i];
+      l_run[r] += e_cur[r][2 * i + 1];
+    };
+    constexpr int kPairs = 8 * RG;
+    // row group 0's share of the exp-sum goes beside the QK MFMAs, row group
+    // 1's beside the first PV MFMAs (its exponents are replaced last)
+    constexpr int kSumA = RG == 2 ? 8 : kPairs;
+    u32x4 kop;
+#pragma unroll
+    for (int c = 0; c < NCH; ++c) {
+      const int kk = c / RG;
+      if constexpr (kMode != kLast) {
+        if (c % RG == 0) kop = k_operand(kk);
+        s_next[c % RG] = Dt<DT>::mma32x32x16(kop, qv[c % RG][kk], s_next[c % RG]);
+      }
+      if (c % RG == 0) {
+        if constexpr (vdense) {
+          // raw rows: V[key][d] in chunk (d / 8) ^ vd_swz(key) of row key.  Lane
+          // 4r + c of a 16-lane group points at keys kg + 4t + r, dims d0 + 4c ..
+          // +3 (d0 = 32 (kk % DT32) + (col & 16)); the transposing read hands
+          // lane j dim d0 + j = col + 32 (kk % DT32) of those 4 keys.
+          const int l16 = lane & 15;
+          const int key = 16 * (kk / DT32) + 8 * half + (l16 >> 2);
+          const int d = 32 * (kk % DT32) + (col & 16) + 4 * (l16 & 3);
+          const uint16_t* vr = v_lds(st) + key * HD + (((d >> 3) ^ vd_swz(key)) << 3) + (d & 7);
+          const u32x2 lo = lds_read_tr16(vr);           // keys kg .. kg+3
+          const u32x2 hi = lds_read_tr16(vr + 4 * HD);  // keys kg+4 .. kg+7 (vd_swz(key + 4) = vd_swz(key))
+          va[kk] = u32x4{lo[0], lo[1], hi[0], hi[1]};
+        } else if constexpr (F8) {
+          // chunk t < DT32 reads row tile t's item (half, d = col + 32 t): keys
+          // 16 half .. +7 for k-step 0 (operand t), +8 .. +15 for k-step 1
+          // (operand t + DT32).  Exact in 16 bits; the V scale is on P.
+          if (kk < DT32)
+            v16[kk] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint8_t*>(v_lds(st)) +
+                                                      (half * HD + col + 32 * kk) * 16);
+          // each half is converted in a later chunk than its read (the LDS
+          // read has landed) and consumed there, so the conversions are not
+          // sunk to the PV MFMAs
+          if (kk >= 1 && kk <= DT32) {
+            va[kk - 1] = fp8x8_exact<DT>(u32x2{v16[kk - 1].x, v16[kk - 1].y});
+            asm volatile("" ::"v"(va[kk - 1]));
+          }
+          if (kk >= DT32) {
+            va[kk] = fp8x8_exact<DT>(u32x2{v16[kk - DT32].z, v16[kk - DT32].w});
+            asm volatile("" ::"v"(va[kk]));
+          }
+        } else {
+          va[kk] = *reinterpret_cast<const u32x4*>(v_lds(st) + (v_base[kk / DT32] + (kk % DT32) * IM::kVRowTile) * 8);
+        }
+      }
+#pragma unroll
+      for (int q = c * kPairs / NCH; q < (c + 1) * kPairs / NCH; ++q) pair_exp(q);
+      if (c > 0) {
+#pragma unroll
+        for (int q = (c - 1) * kPairs / NCH; q < c * kPairs / NCH; ++q) {
+          pair_pack(q);
+          if (q < kSumA) pair_sum(q);
+        }
+      }
+      sched_fence();
+    }
+    // O^T[d][M-row] += sum_key V[key][d] P[M-row][key]; k-step kk takes
+    // registers 8kk .. 8kk+7 = keys 16kk + 8 half .. +7.
+    float bm[RG];
+#pragma unroll
+    for (int r = 0; r < RG; ++r) bm[r] = -INFINITY;
+    // The iteration's copies go out one per PV chunk, K then V, so the
+    // wavefront's MFMAs run while an issue waits for the memory pipeline
+    // (steps that cannot be copied take the synchronous path below).
+    bool kdn = false, vdn = false, kfast = false, vfast = false;
+    uint32_t kp0 = 0, kp1 = 0, vp0 = 0, vp1 = 0;
+    if (kMode == kAny && jv < nsteps) {
+      kp0 = __builtin_amdgcn_readfirstlane(pgk.x);
+      kp1 = TP == 16 ? __builtin_amdgcn_readfirstlane(pgk.y) : kp0;
+      vp0 = __builtin_amdgcn_readfirstlane(pgv.x);
+      vp1 = TP == 16 ? __builtin_amdgcn_readfirstlane(pgv.y) : vp0;
+      kdn = jk < nsteps && (vdense || is_dense(jk));  // steps after a dense one are dense
+      vdn = jv < nsteps && (vdense || is_dense(jv));
+      kfast = jk < nsteps && (kdn || is_fast(jk, kp0, kp1));
+      vfast = jv < nsteps && (vdn || is_fast(jv, vp0, vp1));
+    }
+    int vis[RG];
+#pragma unroll
+    for (int r = 0; r < RG; ++r) vis[r] = seen(r, st + 1);
+    const float sc = kMode == kLast ? 0.f : score_scale(st + 1);
+    constexpr int kFirst = NCH >= 8 ? 2 : 1;  // the chunks before it cover the last QK MFMAs
+#pragma unroll
+    for (int c = 0; c < NCH; ++c) {
+      const int m = c / RG, r = c % RG;
+      if constexpr (kMode == kFast) {
+        if (c < NC) {
+          if constexpr (vdense) copy_dense_k(c, jk); else copy_k(c, jk, pgk.x, pgk.y);
+        } else if (c < 2 * NC) {
+          if constexpr (vdense) copy_dense_v(c - NC, jv); else copy_v(c - NC, jv, pgv.x, pgv.y);
+        }
+      } else if constexpr (kMode == kAny) {
+        if (c < NC) {
+          if (kfast) {
+            if (kdn) copy_dense_k(c, jk); else copy_k(c, jk, kp0, kp1);
+          }
+        } else if (c < 2 * NC) {
+          if (vfast) {
+            if (vdn) copy_dense_v(c - NC, jv); else copy_v(c - NC, jv, vp0, vp1);
+          }
+        }
+      }
+      acc_mma_at<DT, !F8>(r * DT32 + m % DT32, va[m], pp[r][m / DT32]);
+      if (c == 0) {
+#pragma unroll
+        for (int q = (NCH - 1) * kPairs / NCH; q < kPairs; ++q) {
+          pair_pack(q);
+          if (q < kSumA) pair_sum(q);
+        }
+      }
+      if constexpr (!F8) {  // the exp-sum's MFMAs, one per row group and PV k-step
+        constexpr int kAt = NCH >= 8 ? 2 : 0;  // (every probability is packed by the end of chunk 0)
+        if (c >= kAt && c < kAt + 2 * RG) {
+          const int x = c - kAt;
+          l_sum[x % RG] = Dt<DT>::mma16x16x32(ones, pp[x % RG][x / RG], l_sum[x % RG]);
+        }
+      }
+      if constexpr (RG == 2) {  // before chunk kFirst + (NCH - kFirst) / 2
+#pragma unroll
+        for (int q = c * 8 / (NCH / 2); q < (c + 1) * 8 / (NCH / 2); ++q)
+          if (q < 8) pair_sum(8 + q);
+      }
+      if constexpr (kMode != kLast) {
+        // (all in the first chunks, so they have landed by the next barrier)
+        if (c < (F8 ? KS / 2 : KS)) ka[c] = F8 ? read_k8(st + 2, c) : read_k(st + 2, c);
+        if (c >= kFirst) {
+          constexpr int kTot = 16 * RG, kN = NCH - kFirst;
+#pragma unroll
+          for (int x = (c - kFirst) * kTot / kN; x < (c - kFirst + 1) * kTot / kN; ++x) {
+            const int rr = x / 16, xx = x % 16;
+            float v = fmaf(s_next[rr][xx], sc, mb[rr]);
+            if (kMode == kAny) v = place(xx) < vis[rr] ? v : -INFINITY;
+            e_cur[rr][xx] = v;
+            bm[rr] = fmaxf(bm[rr], v);
+          }
+        }
+      }
+      sched_fence();
+    }
+    if constexpr (kMode == kLast) {
+      acc_settle();
+    } else {
+      // the running max of a row moves only when a score passes it by more
+      // than the headroom (rescaling the row's O and exp-sum)
+      float big = bm[0];
+#pragma unroll
+      for (int r = 1; r < RG; ++r) big = fmaxf(big, bm[r]);
+      if (__ballot(big > kLazyRescale)) {
+        acc_settle();
+        float scale[RG];
+#pragma unroll
+        for (int r = 0; r < RG; ++r) {
+          const float row_max = max_xor32(bm[r]);
+          const float m_new = row_max > kLazyRescale ? mb[r] - row_max : mb[r];
+          const float d = m_new - mb[r];
+          scale[r] = __builtin_amdgcn_exp2f(d);
+          mb[r] = m_new;
+          if constexpr (F8) l_run[r] *= scale[r];
+          else row_sum_scale(l_sum[r], scale[r]);
+#pragma unroll
+          for (int x = 0; x < 16; ++x) e_cur[r][x] += d;
+        }
+        static_for<RG * DT32 * 16>([&](auto x) {
+          constexpr int X = decltype(x)::value;
+          acc_put<X>(acc_get<X>() * scale[X / (DT32 * 16)]);
+        });
+        acc_settle();
+      }
+      if constexpr (kMode == kAny) {
+        // entering page-id chunk q (q >= 1): stage chunk q + 1 over chunk q - 1,
+        // whose last reader (V step jv - 1) finished before this iteration's
+        // barrier; the next barriers publish it long before its first reader
+        if (jv < nsteps) {
+        const int e0 = jv * kKeys / TP;
+        if (e0 % kPidChunk == 0 && e0 > 0 && e0 + kPidChunk < n_pid) stage_pids(e0 / kPidChunk + 1);
+        if (jk < nsteps && !kfast) slow_k(jk, kp0, kp1);
+        if (!vfast) slow_v(jv, vp0, vp1);
+        }
+      }
+    }
+  };
+  using Fast = std::integral_constant<int, kFast>;
+  using Any = std::integral_constant<int, kAny>;
+  using Last = std::integral_constant<int, kLast>;
+  constexpr std::true_type yes{};
+  constexpr std::false_type no{};
+  // Iterations [0, n_main) need no mask in their next step (every row sees all
+  // its keys).  In prompt mode steps from fd = ceil(hist / 32) on are dense
+  // (the one across the boundary, if any, is not).  The fast body runs where
+  // the K and V steps it copies are whole steps of one kind: pages, up to the
+  // next page-id chunk (an Any iteration stages the following one there), or
+  // dense rows.
+  const int n_main = min(nsteps - 1, min_lim / kKeys - 1);
+  const int fd = PROMPT ? min(nsteps, static_cast<int>((hist + kKeys - 1) / kKeys)) : nsteps;
+  constexpr int kChunkSteps = kPidChunk * TP / kKeys;                         // steps of a page-id chunk
+  int st = 0;
+  int staged_at = -2;  // the iteration that staged page ids last (its flag is read two iterations later)
+  while (st < min(nsteps - 1, fd)) {
+    // the next iteration whose V step enters a page-id chunk
+    const int chunk_st = (st + kLeadV + kChunkSteps - 1) / kChunkSteps * kChunkSteps - kLeadV;
+    const int fast_end = min(min(n_main, paged_full - kLeadK), chunk_st);
+    if (st < fast_end && st >= staged_at + 2 && __builtin_amdgcn_readfirstlane(lim_lds[kBad]) == 0) {
+      for (; st < fast_end; ++st) step(Fast{}, no, st);
+    } else {
+      if (st == chunk_st) staged_at = st;
+      step(Any{}, no, st);
+      ++st;
+    }
+  }
+  if constexpr (PROMPT) {
+    const int fast_end = min(n_main, max_lim / kKeys - kLeadK);
+    for (; st < fast_end; ++st) step(Fast{}, yes, st);
+    for (; st < nsteps - 1; ++st) step(Any{}, yes, st);
+  }
+  if (nsteps > 0) {
+    if (PROMPT && st >= fd)
+      step(Last{}, yes, st);
+    else
+      step(Last{}, no, st);
+  }
 
-// Rows [0, R) of the query batch alternate runs of one sequence.  Is row r
-// alone in its run (a decode row, served by the decode kernels)?
-__device__ __forceinline__ bool single_row(const uint32_t* q2seq, int64_t r, int64_t n) {
-  const uint32_t sq = q2seq[r];
-  return (r == 0 || q2seq[r - 1] != sq) && (r + 1 == n || q2seq[r + 1] != sq);
+  if (claim) claim->ask(p);  // the workgroup's next item, on its way while this tile is written
+  // ---- normalise and write: lane holds O[M-row col][32n + 8(x/4) + 4 half + x%4].
+  // A store straight from the accumulators would write 16 bytes of each of 32
+  // rows per instruction; the rows go through the step buffers instead (a
+  // region per row group, 16-byte chunk c of row i at chunk c ^ i, so that both
+  // sides spread over the banks) and out as whole rows, 16 bytes per lane,
+  // non-temporally (nothing here reads them again).
+  if (nsteps == 0) {
+    acc_zero();
+    acc_settle();
+  }
+  __syncthreads();  // every wavefront has read the last step
+  constexpr int kCh = HD / 8;  // 16-byte chunks of a row
+  auto place_chunk = [](int row, int c) { return (kCh & (kCh - 1)) == 0 ? c ^ (row & (kCh - 1)) : (c + row) % kCh; };
+  static_for<RG>([&](auto rc) {
+    constexpr int r = decltype(rc)::value;
+    uint16_t* region = k_lds_base + (w * RG + r) * 32 * HD;  // K buffers, then V buffers: 8 regions of 32 rows
+    float l;
+    if constexpr (F8) l = sum_xor32(l_run[r]);
+    else l = row_sum_of(l_sum[r]);
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+    static_for<DT32 * 4>([&](auto qc) {
+      constexpr int c = decltype(qc)::value, n = c / 4, q4 = c % 4;
+      constexpr int x = (r * DT32 + n) * 16 + 4 * q4;
+      const u32x2 pk = {Dt<DT>::pack2(acc_get<x>() * inv, acc_get<x + 1>() * inv),
+                        Dt<DT>::pack2(acc_get<x + 2>() * inv, acc_get<x + 3>() * inv)};
+      *reinterpret_cast<u32x2*>(region + col * HD + place_chunk(col, c) * 8 + 4 * half) = pk;
+    });
+  });
+  uint16_t* out_tile = p.out + (static_cast<int64_t>(row0) * p.num_q_heads + kvh * p.group + h0) * HD;
+  compiler_fence();
+  __builtin_amdgcn_s_waitcnt(kLgkmZero);  // a wavefront reads only what it wrote
+  compiler_fence();
+#pragma unroll
+  for (int r = 0; r < RG; ++r) {
+    const uint16_t* region = k_lds_base + (w * RG + r) * 32 * HD;
+#pragma unroll
+    for (int it = 0; it < kCh / 2; ++it) {
+      const int i = it * kWave + lane;
+      const int row = i / kCh, c = i % kCh;
+      const int m = (w * RG + r) * 32 + row;
+      const int t = static_cast<int>((static_cast<uint32_t>(m) * p.hg_magic) >> 16);
+      const int h = m - t * p.hg_max;
+      const u32x4 val = *reinterpret_cast<const u32x4*>(region + row * HD + place_chunk(row, c) * 8);
+      // (offsets inside a tile's rows fit 32 bits)
+      if (t < nrows && t < qt && h < hg)
+        __builtin_nontemporal_store(
+            val, reinterpret_cast<u32x4_align8*>(out_tile + static_cast<uint32_t>((t * p.num_q_heads + h) * HD + c * 8)));
+    }
+  }
 }
 
 // LDS of a prefill workgroup: four K and four V step buffers, the target of
-// padding copies, two chunks of page ids, the rows' key limits (with their
-// max and min) and the run starts of a window.
-template <int HD, bool KV8>
+// padding copies, two chunks of page ids, the tokens' key limits (with their
+// largest and smallest per wavefront) and the runs of a window.
+template <int HD, bool KV8, int RG>
 struct PrefillLds {
   __attribute__((aligned(16))) uint16_t k[kNBuf * StepGeo<HD>::kItems * 8];
   __attribute__((aligned(16))) uint16_t v[kNBuf * StepGeo<HD>::kItems * 8];
   __attribute__((aligned(16))) uint16_t junk[kWave * 8];
   uint32_t pid[2 * kPidChunk];
   float scl[KV8 ? 4 * kPidChunk : 1];  // fp8 pools: K then V scale of each staged page id
-  int lim[kMRows + 2];
-  int run_start[kMRows];
+  int lim[m_rows(RG) + 2 * kPfWaves + 1];
+  uint32_t seq[m_rows(RG)];               // window: the rows' sequences and key limits
+  int32_t off[m_rows(RG)];
+  uint64_t start[m_rows(RG) / kWave];     // window: rows that start a run, rows alone in their run
+  uint64_t lone[m_rows(RG) / kWave];
+  uint32_t next[2];                       // the claimed item (or none left), the queue it came from
 };
 
-// The work of prefill block b (a 1-D grid, XCD-aware): head group
-// g = b % G (G = kv heads x head chunks) and work unit b / G, so consecutive
-// blocks -- which the dispatcher spreads over the 8 XCDs -- take different kv
-// heads, and each kv head's K/V stay in few L2s.
+// Window mode: one row of an item's window per thread (its sequence, those of
+// the rows beside it, its key limit).
+struct RowMap {
+  uint32_t cur, prev, next;
+  int32_t off;
+};
+template <int RG>
+__device__ __forceinline__ RowMap load_row_map(const PrefillParams& p, unsigned item) {
+  RowMap m{0u, 0u, 0u, 0};
+  const unsigned G = static_cast<unsigned>(p.num_kv_heads) * p.head_chunks;
+  const int unit = static_cast<int>(item / G);
+  const int qt = m_rows(RG) / p.hg_max;
+  const int64_t r = static_cast<int64_t>(p.num_units - 1 - unit) * qt + threadIdx.x;
+  if (unit < p.num_units && static_cast<int>(threadIdx.x) < qt && r < p.num_rows) {
+    m.cur = p.q2seq[r];
+    m.prev = r > 0 ? p.q2seq[r - 1] : 0u;
+    m.next = r + 1 < p.num_rows ? p.q2seq[r + 1] : 0u;
+    m.off = p.q_offset[r];
+  }
+  return m;
+}
+
+// Work item `item` of the prefill: head group g = item % G (G = kv heads x
+// head chunks) and work unit item / G, so that items 8 apart -- workgroups of
+// one XCD -- take the same few kv heads and a kv head's K/V stay in few L2s.
 //  * prompt mode: unit = (sequence, tile), the last tile of a sequence first
 //    (it has the most keys);
 //  * window mode (fused op): unit = window of `tokens per tile` rows, the
 //    last window first (rows of a sequence usually come in position order,
 //    so its later windows see more keys); every run of rows of one sequence
-//    inside the window that is not a lone decode row is computed as a tile.
-// kPromptMode false: the caller never runs the uniform-prompt mode (the
-// fused kernel), which is then not compiled in.
-template <int DT, int HD, int TPP, bool KV8, bool kPromptMode = true>
-__device__ __forceinline__ void prefill_block(const PrefillParams& p, unsigned block, PrefillLds<HD, KV8>& L) {
-  uint16_t* k_lds = L.k;
-  uint16_t* v_lds = L.v;
-  uint16_t* junk_lds = L.junk;
-  uint32_t* pid_lds = L.pid;
-  float* scl_lds = L.scl;
-  int* lim_lds = L.lim;
-  int* run_start = L.run_start;
+//    inside the window that is not a lone decode row (served by the decode
+//    workers) is computed as a tile.
+template <int DT, int HD, int TPP, bool KV8, int RG, bool kPromptMode>
+__device__ __forceinline__ void prefill_item(const PrefillParams& p, unsigned item, Claim& claim,
+                                             PrefillLds<HD, KV8, RG>& L) {
   const int G = p.num_kv_heads * p.head_chunks;
-  const int g = static_cast<int>(block % static_cast<unsigned>(G));
-  const int unit = static_cast<int>(block / static_cast<unsigned>(G));
+  const int g = static_cast<int>(item % static_cast<unsigned>(G));
+  const int unit = static_cast<int>(item / static_cast<unsigned>(G));
   const int kvh = g / p.head_chunks;
   const int h0 = (g % p.head_chunks) * 16;
-  const int qt = kMRows / p.hg_max;
+  const int qt = m_rows(RG) / p.hg_max;
   if constexpr (kPromptMode) {
-    if (p.prompt_len > 0) {
-      const int tps = (p.prompt_len + qt - 1) / qt;
-      const int s = unit / tps;
-      const int j = tps - 1 - (unit - s * tps);
-      const int row0 = s * p.prompt_len + j * qt;
-      prefill_tile<DT, HD, TPP, true, KV8>(p, row0, min(qt, p.prompt_len - j * qt), s, kvh, h0, k_lds, v_lds,
-                                           junk_lds, pid_lds, lim_lds, scl_lds);
-      return;
+    const int tps = (p.prompt_len + qt - 1) / qt;
+    const int s = unit / tps;
+    const int j = tps - 1 - (unit - s * tps);
+    const int row0 = s * p.prompt_len + j * qt;
+    prefill_tile<DT, HD, TPP, true, KV8, RG>(p, row0, min(qt, p.prompt_len - j * qt), s, kvh, h0, L.k, L.v, L.junk, L.pid,
+                                             L.lim, L.scl, nullptr, nullptr);
+  } else {
+    const int w0 = (p.num_units - 1 - unit) * qt;
+    const int n = static_cast<int>(min(static_cast<int64_t>(qt), p.num_rows - w0));
+    constexpr int kMasks = m_rows(RG) / kWave;
+    const RowMap rm = load_row_map<RG>(p, item);
+    __syncthreads();  // the previous item is done with the run masks
+    if (wave_id() < kMasks) {  // a wavefront per 64 rows of the window
+      const int i = wave_id() * kWave + lane_id();
+      const bool in = i < n;
+      const bool head = in && (w0 + i == 0 || rm.prev != rm.cur);  // starts a run of its sequence's rows
+      const bool tail = in && (w0 + i + 1 == p.num_rows || rm.next != rm.cur);
+      L.seq[i] = rm.cur;
+      L.off[i] = rm.off;
+      const uint64_t st = __ballot(in && (i == 0 || head));
+      const uint64_t lo = __ballot(head && tail);
+      if (lane_id() == 0) {
+        L.start[wave_id()] = st;
+        L.lone[wave_id()] = lo;
+      }
+    }
+    __syncthreads();
+    auto uniform64 = [](uint64_t v) {
+      return (static_cast<uint64_t>(__builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v >> 32))) << 32) |
+             static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v)));
+    };
+    int cur = 0;
+    while (cur < n) {
+      // the next run's start, from the masks' bits past cur
+      int end = n;
+      const int from = cur + 1;
+      for (int i = from / kWave; i < kMasks; ++i) {
+        uint64_t m = uniform64(L.start[i]);
+        if (i == from / kWave) m &= ~0ull << (from % kWave);
+        if (m) {
+          end = min(n, i * kWave + __builtin_ctzll(m));
+          break;
+        }
+      }
+      const bool lone = (uniform64(L.lone[cur / kWave]) >> (cur % kWave)) & 1;
+      if (!lone)
+        prefill_tile<DT, HD, TPP, false, KV8, RG>(p, w0 + cur, end - cur, L.seq[cur], kvh, h0, L.k, L.v, L.junk, L.pid,
+                                                  L.lim, L.scl, L.off + cur, end == n ? &claim : nullptr);
+      cur = end;
     }
   }
-  if constexpr (TPP != 0) {  // run-time page sizes: uniform-prompt mode only
-    // windows in reverse row order: a sequence's later rows see more keys, so
-    // its longest tiles start first and the grid ends on short ones
-    const int w0 = (p.num_units - 1 - unit) * qt;
-    const int w1 = static_cast<int>(min(static_cast<int64_t>(w0 + qt), p.num_rows));
-    const int tid = threadIdx.x;
-    if (tid < w1 - w0) run_start[tid] = (tid == 0 || p.q2seq[w0 + tid] != p.q2seq[w0 + tid - 1]) ? 1 : 0;
-    __syncthreads();
-    int cur = w0;
-    while (cur < w1) {
-      int end = cur + 1;
-      while (end < w1 && !run_start[end - w0]) ++end;
-      end = __builtin_amdgcn_readfirstlane(end);
-      if (end - cur > 1 || !single_row(p.q2seq, cur, p.num_rows))
-        prefill_tile<DT, HD, TPP, false, KV8>(p, cur, end - cur, p.q2seq[cur], kvh, h0, k_lds, v_lds, junk_lds, pid_lds,
-                                         lim_lds, scl_lds);
-      cur = end;
+}
+
+// The prefill's items on a resident grid, one workgroup per CU: a workgroup
+// that starts on a CU pays several us before its first load (measured: 6.5 us
+// between a workgroup's end and its successor's first instruction on the same
+// CU, tiles of 30-60 us).
+//  * Window mode: items are claimed, the first by place (workgroup b starts on
+//    item b).  Lengths differ by item, and a static share left CUs idle for up
+//    to a fifth of the time (16 sequences of 512 to 2,048 rows on 0 to 2,048
+//    cached keys).
+//  * Prompt mode (no workspace to hold counters): workgroup b of nb takes items
+//    b, nb + b', 2 nb + b, ... (b' = the mirrored place among the workgroups of
+//    b's XCD, so that a pass over ever shorter items evens out the previous one).
+template <int DT, int HD, int TPP, bool KV8, int RG, bool kPromptMode>
+__device__ __forceinline__ void prefill_items(const PrefillParams& p, unsigned b, unsigned nb,
+                                              PrefillLds<HD, KV8, RG>& L) {
+  const unsigned items = static_cast<unsigned>(p.num_units) * p.num_kv_heads * p.head_chunks;
+  Claim claim{b % kQueues, 0u, false};
+  if constexpr (kPromptMode) {
+    const unsigned mirrored = nb % 8 == 0 ? nb - 8 - (b & ~7u) + (b & 7u) : b;
+    for (unsigned pass = 0; pass * nb < items; ++pass) {
+      const unsigned item = pass * nb + ((pass & 1) ? mirrored : b);
+      if (item < items) prefill_item<DT, HD, TPP, KV8, RG, true>(p, item, claim, L);
+    }
+  } else {
+    // queue q: items q, q + 8, ...; its first ceil((nb - q) / 8) are taken by place
+    auto item_of = [&](uint32_t q, uint32_t n) { return q + kQueues * (n + (nb + kQueues - 1 - q) / kQueues); };
+    unsigned item = b;
+    while (item < items) {
+      claim.asked = false;
+      prefill_item<DT, HD, TPP, KV8, RG, false>(p, item, claim, L);
+      if (!claim.asked) claim.ask(p);
+      if (threadIdx.x == 0) {
+        uint32_t q = claim.queue;
+        unsigned next = item_of(q, claim.got);
+        for (int k = 1; k < kQueues && next >= items; ++k) {  // that queue is empty: the next one with an item
+          q = (q + 1) % kQueues;
+          next = item_of(q, atomicAdd(p.claims + q, 1u));
+        }
+        L.next[0] = next;
+        L.next[1] = q;
+      }
+      __syncthreads();
+      item = __builtin_amdgcn_readfirstlane(L.next[0]);
+      claim.queue = __builtin_amdgcn_readfirstlane(L.next[1]);
     }
   }
 }

@@ -394,6 +394,32 @@ def test_fused_fp8_pages(dtype, hd, tpp):
     assert_close(host_f32(out), ref, dtype, f"fp8 fused {dtype} hd{hd} tpp{tpp}")
 
 
+@pytest.mark.parametrize("hd,tpp", [(64, 16), (64, 32), (128, 16), (128, 32), (256, 16)])
+@pytest.mark.parametrize("rows", [161, 300, 401])
+def test_fused_fp8_tile_sizes(rows, hd, tpp):
+    """Prefill tiles with a CU to themselves over fp8 pages: of one row group
+    (161 rows: 168 tiles on 8 kv heads of 16 query heads), of two (300: 152
+    tiles of 16 rows; head dims above 128: one), and beyond one round (401
+    rows on twice the kv heads)."""
+    from pal_cases import make_fused_case
+
+    rng = np.random.default_rng(hd + tpp + rows)
+    hkv = 16 if rows > 400 else 8
+    fc = make_fused_case(hd + tpp + rows, [70], [(45, rows)], 16 * hkv, hkv, hd, tpp, "bf16", block=rows)
+    c = fc.case
+    kc, vc, ks, vs = fp8_case(c, rng)
+    announce(f"fused fp8 tile sizes rows={rows} hd={hd} tpp={tpp}")
+    args = (dev_bits(fc.queries, "bf16"), dev_codes(kc), dev_codes(vc), dev_index(c.page_table, torch.uint32),
+            dev_index(c.seq_lens), dev_index(fc.q2seq, torch.uint32), dev_index(fc.q_offset))
+    scales = {"k_scales": torch.from_numpy(ks).to(DEV), "v_scales": torch.from_numpy(vs).to(DEV)}
+    out = host_f32(pal.paged_attention(*args, **scales))
+    again = host_f32(pal.paged_attention(*args, **scales))
+    ref = orc.paged_attention(fc.queries, kc, vc, c.page_table, c.seq_lens, fc.q2seq, fc.q_offset, "bf16",
+                              kv_scales=(ks, vs))
+    assert_close(out, ref, "bf16", f"fp8 tile sizes rows={rows} hd{hd} tpp{tpp}")
+    assert np.array_equal(out, again)
+
+
 @pytest.mark.parametrize("dtype", ["bf16", "f16"])
 def test_fused_fp8_query_magnitudes(dtype):
     """fp8 pages under the fused op with query heads across the dtype's range

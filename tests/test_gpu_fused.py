@@ -186,3 +186,37 @@ def test_fused_query_magnitudes(dtype):
     fc.queries = extreme_query_bits(np.random.default_rng(74), fc.queries.shape, dtype, tiles=True)
     out = _check_fused(fc, f"query magnitudes {dtype}")
     assert np.isfinite(out).all()
+
+
+# (query heads, kv heads, decode lengths, chunks, block): few decode rows per
+# prefill row, so tiles have a CU to themselves from 640 (row, head of a group)
+# per sequence on: one side of that line and the other, tiles of one row group,
+# of two, and more tiles than CUs of either (claimed), windows that start
+# and end inside a run
+TILE_CASES = {
+    "beside-decode": (32, 8, [300], [(100, 318)], 400),            # 319 rows * 4 < 640 * 2
+    "one-group": (32, 8, [300], [(100, 319)], 400),                # 320 rows * 4 = 640 * 2; 80 tiles
+    "one-group-claimed": (32, 32, [], [(0, 1400)], 1400),          # 352 tiles of 128 rows
+    "two-groups": (128, 8, [], [(37, 300), (500, 1)], 300),        # 304 tiles of 8 rows, 152 of 16
+    "two-groups-claimed": (256, 16, [70], [(65, 401)], 401),       # 816 tiles of 8 rows, 416 of 16
+    "lone-rows": (64, 4, [900] * 20 + [0], [(20, 900), (3, 40)], 33),  # interleaved with blocks of runs
+}
+
+
+@pytest.mark.parametrize("hd,tpp,dtype", [(32, 16, "f16"), (64, 32, "bf16"), (128, 16, "bf16"), (256, 16, "bf16")])
+@pytest.mark.parametrize("name", TILE_CASES)
+def test_fused_tile_sizes(name, hd, tpp, dtype):
+    """Twice each: a call leaves the counters its tiles are claimed from as it
+    found them, and the claim order does not show in the result."""
+    hq, hkv, dec, chunks, block = TILE_CASES[name]
+    fc = make_fused_case(hd + 77, dec, chunks, hq, hkv, hd, tpp, dtype, block=block)
+    first = _check_fused(fc, name)
+    again = host_f32(_fused_gpu(fc.case, fc.queries, fc.q2seq, fc.q_offset))
+    assert np.array_equal(first, again)
+
+
+def test_fused_tile_claims_across_head_dims():
+    """Head dims above and up to 128 claim tiles in kernels of different launch
+    sequences, from the counters of one workspace."""
+    for i, hd in enumerate([256, 64, 256, 32]):
+        _check_fused(make_fused_case(90 + i, [40], [(10, 700)], 64, 32, hd, 16, "bf16", block=700), f"claims hd{hd}")

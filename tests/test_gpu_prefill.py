@@ -165,3 +165,14 @@ def test_prefill_query_magnitudes(dtype):
     assert np.isfinite(out).all()
     ref = orc.paged_attention_prefill(q, k, v, case.k_pool, case.v_pool, case.page_table, case.seq_lens, dtype)
     assert_close(out, ref, dtype, f"prefill query magnitudes {dtype}")
+
+
+@pytest.mark.parametrize("hd,tpp,dtype", [(32, 16, "bf16"), (64, 16, "f16"), (96, 8, "bf16"), (128, 16, "bf16"),
+                                          (128, 32, "f16"), (256, 32, "bf16")])
+@pytest.mark.parametrize("plen", [190, 259, 520])
+def test_prefill_tile_rounds(plen, hd, tpp, dtype):
+    """More tiles than CUs: with 64 query heads on 16 kv heads 190 rows make
+    288 tiles of one row group (32 rows) or 144 of two, 259 rows 432 / 240 with
+    three rows in the last one, 520 rows 816 / 432, two rounds of the larger
+    tiles (head dims above 128 have the smaller ones only)."""
+    _check(hd + plen, [0, 33, 150], plen, 64, 16, hd, tpp, dtype, "tile rounds")
