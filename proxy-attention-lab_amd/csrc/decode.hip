@@ -1530,16 +1530,15 @@ hipError_t dispatch_hd(const DecodeParams& p, int hd, int tpp, bool kv8, hipStre
   }
 }
 
-// One after the other instead of side by side?  The lone rows of a batch are
-// at most one or a few per sequence, so with L keys per sequence the stream
-// takes about num_seqs * L * Hkv * HD * 4 bytes / 6 TB/s and the tiles rows * L *
-// Hq * HD * 4 flops / 0.8 PFLOP/s; the tiles' gain (a fifth of their time) pays
-// for a stream that nothing overlaps while the stream is below a fifth of the
-// tiles: num_seqs * 133 / group < rows / 5.  Measured on both sides: 16
-// sequences, 20,000 rows, group 4 (rows * group / num_seqs = 4,700) 0.70 ->
-// 0.61 ms; 256 decode rows and 4 chunks of 1,024, group 8 (134) 0.94 side by
-// side, 1.04 ms one after the other.
-inline bool fused_wide(const PrefillParams& p) { return p.num_rows * p.group >= 640 * p.num_seqs; }
+// One after the other instead of side by side?  The stream of the lone rows
+// then overlaps nothing, which the faster tiles pay for only if the batch is
+// mostly prefill: many (row, head) products per sequence whose keys may be
+// streamed.  Measured side by side -> one after the other, by rows * group /
+// num_seqs (head dim 128, 8 kv heads): 5,000 (16 sequences, 20,000 rows) 0.70 ->
+// 0.61 ms; 1,370 (8 decode rows, 4 chunks of 1,024) 238 -> 210 us; 1,030 (7 decode
+// rows of 30,000 keys, one chunk of 2,048) 221 -> 228 us; 820 (4 decode rows, one
+// chunk of 1,024) 69 -> 88 us; 134 (256 decode rows, 4 chunks) 0.94 -> 1.04 ms.
+inline bool fused_wide(const PrefillParams& p) { return p.num_rows * p.group >= 1200 * p.num_seqs; }
 
 // The fused op: the fused kernel, then the merge; head dims above 128: the
 // prefill tiles, then the decode rows' kernels.

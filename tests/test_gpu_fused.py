@@ -189,17 +189,17 @@ def test_fused_query_magnitudes(dtype):
 
 
 # (query heads, kv heads, decode lengths, chunks, block): few decode rows per
-# prefill row, so tiles have a CU to themselves from 640 (row, head of a group)
+# prefill row, so tiles have a CU to themselves from 1,200 (row, head of a group)
 # per sequence on: one side of that line and the other, tiles of one row group,
 # of two, and more tiles than CUs of either (claimed), windows that start
 # and end inside a run
 TILE_CASES = {
-    "beside-decode": (32, 8, [300], [(100, 318)], 400),            # 319 rows * 4 < 640 * 2
-    "one-group": (32, 8, [300], [(100, 319)], 400),                # 320 rows * 4 = 640 * 2; 80 tiles
+    "beside-decode": (32, 8, [300], [(100, 598)], 600),            # 599 rows * 4 < 1200 * 2
+    "one-group": (32, 8, [300], [(100, 599)], 600),                # 600 rows * 4 = 1200 * 2; 152 tiles
     "one-group-claimed": (32, 32, [], [(0, 1400)], 1400),          # 352 tiles of 128 rows
     "two-groups": (128, 8, [], [(37, 300), (500, 1)], 300),        # 304 tiles of 8 rows, 152 of 16
     "two-groups-claimed": (256, 16, [70], [(65, 401)], 401),       # 816 tiles of 8 rows, 416 of 16
-    "lone-rows": (64, 4, [900] * 20 + [0], [(20, 900), (3, 40)], 33),  # interleaved with blocks of runs
+    "lone-rows": (64, 4, [900] * 20 + [0], [(20, 1700), (3, 40)], 33),  # interleaved with blocks of runs
 }
 
 
@@ -219,4 +219,4 @@ def test_fused_tile_claims_across_head_dims():
     """Head dims above and up to 128 claim tiles in kernels of different launch
     sequences, from the counters of one workspace."""
     for i, hd in enumerate([256, 64, 256, 32]):
-        _check_fused(make_fused_case(90 + i, [40], [(10, 700)], 64, 32, hd, 16, "bf16", block=700), f"claims hd{hd}")
+        _check_fused(make_fused_case(90 + i, [], [(10, 700)], 64, 32, hd, 16, "bf16", block=700), f"claims hd{hd}")
