@@ -168,14 +168,14 @@ __device__ __forceinline__ void half_tile(const PrefillParams& p, int row0, int 
     if constexpr (F8) {
       const bool ok = pg < p.num_pages;
       const int64_t si = static_cast<int64_t>(ok ? pg : 0) * p.num_kv_heads + kvh;
-      ks_lds[e % (2 * kPidChunk)] = ok ? p.k_scales[si] : 0.f;
-      vs_lds[e % (2 * kPidChunk)] = ok ? p.v_scales[si] : 0.f;
+      ks_lds[pid_slot(e)] = ok ? p.k_scales[si] : 0.f;
+      vs_lds[pid_slot(e)] = ok ? p.v_scales[si] : 0.f;
     }
   };
   auto stage_pids = [&](int chunk) {  // synchronous; callers hold a barrier after it
     for (int e = chunk * kPidChunk + tid; e < min((chunk + 1) * kPidChunk, n_pid); e += kPfThreads) {
       const uint32_t pg = pt[e];
-      pid_lds[e % (2 * kPidChunk)] = pg;
+      pid_lds[pid_slot(e)] = pg;
       stage_scales(e, pg);
     }
   };
@@ -414,8 +414,8 @@ __device__ __forceinline__ void half_tile(const PrefillParams& p, int row0, int 
   // scale could be NaN)
   auto read_scales = [&](const float* arr, int j, float& s0, float& s1) {
     const int e = j * kKeys / TPP;
-    s0 = e < n_pid ? arr[e % (2 * kPidChunk)] : 0.f;
-    s1 = TPP == 16 ? (e + 1 < n_pid ? arr[(e + 1) % (2 * kPidChunk)] : 0.f) : s0;
+    s0 = e < n_pid ? arr[pid_slot(e)] : 0.f;
+    s1 = TPP == 16 ? (e + 1 < n_pid ? arr[pid_slot(e + 1)] : 0.f) : s0;
   };
   // fp8: step j's scores times the K scale of each key's page (register r
   // holds key 16 (r / 8) + ..., so r < 8: the first page)
@@ -428,7 +428,7 @@ __device__ __forceinline__ void half_tile(const PrefillParams& p, int row0, int 
     }
   };
   auto read_pids = [&](int j) {
-    const int e = (j * kKeys / TPP) % (2 * kPidChunk);
+    const int e = pid_slot(j * kKeys / TPP);
     u32x2 v;
     if (TPP == 16) {
       v = *reinterpret_cast<const u32x2*>(pid_lds + e);  // e is even: 8-byte aligned
@@ -580,7 +580,7 @@ __device__ __forceinline__ void half_tile(const PrefillParams& p, int row0, int 
   auto step = [&](auto masked, int st) {
     constexpr bool kMask = decltype(masked)::value;
     wait_barrier(st + 2 < nsteps ? 1 : 0);  // step st+1 has landed
-    const int j = st + 3;
+    const int j = st + kLeadHalf;
     const u32x2 pgv = read_pids(j);  // used after the MFMAs (in bounds whether or not step j exists)
     u32x4 ka[KS];
     read_k(st + 1, ka);
@@ -686,14 +686,8 @@ __device__ __forceinline__ void half_tile(const PrefillParams& p, int row0, int 
     }
     __builtin_amdgcn_s_setprio(0);
     mb = update_max(bm);
-    if (j < nsteps) {
-      // entering page-id chunk q (q >= 1): stage chunk q + 1 over chunk q - 1,
-      // whose last reader finished before this iteration's barrier; the next
-      // barriers publish it long before its first reader
-      const int e0 = j * kKeys / TPP;
-      if (e0 % kPidChunk == 0 && e0 > 0 && e0 + kPidChunk < n_pid) stage_pids(e0 / kPidChunk + 1);
-      if (!jfast) issue(j, jp0, jp1);
-    }
+    if (const int chunk = pid_chunk_to_stage(st, TPP, n_pid)) stage_pids(chunk);
+    if (j < nsteps && !jfast) issue(j, jp0, jp1);
     s_cur = s_next;
   };
   int st = 0;

@@ -71,6 +71,7 @@
 #include <type_traits>
 
 #include "pal_device.h"
+#include "pid_window.h"
 
 namespace pal {
 namespace {
@@ -80,10 +81,6 @@ constexpr int kPfWaves = 4;
 constexpr int kPfThreads = kPfWaves * kWave;
 // M-rows (token, head) of a workgroup whose wavefronts hold rg groups of 32 each
 constexpr int m_rows(int rg) { return kPfWaves * 32 * rg; }
-constexpr int kKeys = 32;              // keys per step
-constexpr int kNBuf = 4;               // LDS step buffers, of K and of V
-constexpr int kLeadK = 5, kLeadV = 3;  // iteration st copies K of step st + kLeadK and V of step st + kLeadV
-constexpr int kPidChunk = 512;         // page ids staged per chunk; two chunks live in LDS
 static_assert(kPidChunk % kPfThreads == 0, "a page-id chunk is a whole number of loads per thread");
 constexpr float kLazyRescale = 8.f;    // log2 headroom before the running max moves
 
@@ -362,14 +359,14 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
     if constexpr (F8) {
       const bool ok = pg < p.num_pages;
       const int64_t si = static_cast<int64_t>(ok ? pg : 0) * p.num_kv_heads + kvh;
-      ks_lds[e % (2 * kPidChunk)] = ok ? p.k_scales[si] : 0.f;
-      vs_lds[e % (2 * kPidChunk)] = ok ? p.v_scales[si] : 0.f;
+      ks_lds[pid_slot(e)] = ok ? p.k_scales[si] : 0.f;
+      vs_lds[pid_slot(e)] = ok ? p.v_scales[si] : 0.f;
     }
   };
   auto stage_pids = [&](int chunk) {  // synchronous; callers hold a barrier after it
     for (int e = chunk * kPidChunk + tid; e < min((chunk + 1) * kPidChunk, n_pid); e += kPfThreads) {
       const uint32_t pg = pt[e];
-      pid_lds[e % (2 * kPidChunk)] = pg;
+      pid_lds[pid_slot(e)] = pg;
       if (pg >= p.num_pages) lim_lds[kBad] = 1;
       stage_scales(e, pg);
     }
@@ -736,13 +733,13 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
   // scale could be NaN)
   auto read_scales = [&](const float* arr, int j, float& s0, float& s1) {
     const int e = j * (kKeys / TP);  // (even with TP 16)
-    const float a0 = arr[e & (2 * kPidChunk - 1)], a1 = arr[(e + (TP == 16)) & (2 * kPidChunk - 1)];
+    const float a0 = arr[pid_slot(e)], a1 = arr[pid_slot(e + (TP == 16))];
     s0 = e < n_pid ? a0 : 0.f;
     s1 = TP == 16 ? (e + 1 < n_pid ? a1 : 0.f) : s0;
   };
   // the page ids of step j (an LDS broadcast read; TP 32: one page)
   auto read_pids = [&](int j) {
-    const int e = (j * (kKeys / TP)) & (2 * kPidChunk - 1);
+    const int e = pid_slot(j * (kKeys / TP));
     u32x2 v;
     if (TP == 16) {
       v = *reinterpret_cast<const u32x2*>(pid_lds + e);  // e is even: 8-byte aligned
@@ -1192,14 +1189,10 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
         acc_settle();
       }
       if constexpr (kMode == kAny) {
-        // entering page-id chunk q (q >= 1): stage chunk q + 1 over chunk q - 1,
-        // whose last reader (V step jv - 1) finished before this iteration's
-        // barrier; the next barriers publish it long before its first reader
+        if (const int chunk = pid_chunk_to_stage(st, TP, n_pid)) stage_pids(chunk);
         if (jv < nsteps) {
-        const int e0 = jv * kKeys / TP;
-        if (e0 % kPidChunk == 0 && e0 > 0 && e0 + kPidChunk < n_pid) stage_pids(e0 / kPidChunk + 1);
-        if (jk < nsteps && !kfast) slow_k(jk, kp0, kp1);
-        if (!vfast) slow_v(jv, vp0, vp1);
+          if (jk < nsteps && !kfast) slow_k(jk, kp0, kp1);
+          if (!vfast) slow_v(jv, vp0, vp1);
         }
       }
     }
@@ -1213,16 +1206,14 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
   // its keys).  In prompt mode steps from fd = ceil(hist / 32) on are dense
   // (the one across the boundary, if any, is not).  The fast body runs where
   // the K and V steps it copies are whole steps of one kind: pages, up to the
-  // next page-id chunk (an Any iteration stages the following one there), or
-  // dense rows.
+  // next iteration that stages a page-id chunk (an Any iteration), or dense
+  // rows.
   const int n_main = min(nsteps - 1, min_lim / kKeys - 1);
   const int fd = PROMPT ? min(nsteps, static_cast<int>((hist + kKeys - 1) / kKeys)) : nsteps;
-  constexpr int kChunkSteps = kPidChunk * TP / kKeys;                         // steps of a page-id chunk
   int st = 0;
   int staged_at = -2;  // the iteration that staged page ids last (its flag is read two iterations later)
   while (st < min(nsteps - 1, fd)) {
-    // the next iteration whose V step enters a page-id chunk
-    const int chunk_st = (st + kLeadV + kChunkSteps - 1) / kChunkSteps * kChunkSteps - kLeadV;
+    const int chunk_st = pid_next_staging(st, TP);
     const int fast_end = min(min(n_main, paged_full - kLeadK), chunk_st);
     if (st < fast_end && st >= staged_at + 2 && __builtin_amdgcn_readfirstlane(lim_lds[kBad]) == 0) {
       for (; st < fast_end; ++st) step(Fast{}, no, st);

@@ -420,6 +420,34 @@ def test_fused_fp8_tile_sizes(rows, hd, tpp):
     assert np.array_equal(out, again)
 
 
+@pytest.mark.parametrize("decode", [[], [50]], ids=["wide", "beside-decode"])
+@pytest.mark.parametrize("hd,tpp,keys", [(128, 16, 26000), (64, 32, 50000), (256, 16, 26000)])
+def test_fused_fp8_long_history_scales(hd, tpp, keys, decode):
+    """Prefill rows over more page-table entries than the tiles' LDS holds (two
+    chunks of 512), in both forms of the fused op.  The pages before each change
+    of chunk carry 4 times the scales of the others, so their keys dominate the
+    softmax: a scale of another page there is far outside the tolerance."""
+    from pal_cases import make_fused_case
+
+    rng = np.random.default_rng(hd + tpp)
+    fc = make_fused_case(hd + tpp + 5, decode, [(keys, 80)], 16, 1, hd, tpp, "bf16", block=80)
+    c = fc.case
+    kc, vc, ks, vs = fp8_case(c, rng)
+    entries = np.concatenate([np.arange(512 * q - 12, 512 * q) for q in (1, 2)])
+    pages = c.page_table[len(decode), entries]
+    ks[pages] *= 4
+    vs[pages] *= 4
+    announce(f"fused fp8 long history hd={hd} tpp={tpp} keys={keys} decode rows={len(decode)}")
+    out = pal.paged_attention(dev_bits(fc.queries, "bf16"), dev_codes(kc), dev_codes(vc),
+                              dev_index(c.page_table, torch.uint32), dev_index(c.seq_lens),
+                              dev_index(fc.q2seq, torch.uint32), dev_index(fc.q_offset),
+                              k_scales=torch.from_numpy(ks).to(DEV), v_scales=torch.from_numpy(vs).to(DEV))
+    torch.cuda.synchronize()
+    ref = orc.paged_attention(fc.queries, kc, vc, c.page_table, c.seq_lens, fc.q2seq, fc.q_offset, "bf16",
+                              kv_scales=(ks, vs))
+    assert_close(host_f32(out), ref, "bf16", f"fp8 long history hd{hd} tpp{tpp}")
+
+
 @pytest.mark.parametrize("dtype", ["bf16", "f16"])
 def test_fused_fp8_query_magnitudes(dtype):
     """fp8 pages under the fused op with query heads across the dtype's range
