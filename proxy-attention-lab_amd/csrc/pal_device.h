@@ -74,6 +74,7 @@ constexpr uint32_t kDebugFillDest = 4u;   // a fill token with no valid destinat
 //   mma16x16x32: A[16 x 32] * B[32 x 16] (8 elements per lane per operand)
 //   mma16x16x16: A[16 x 16] * B[16 x 16] (4 elements per lane per operand)
 //   mma32x32x16: A[32 x 16] * B[16 x 32] (8 elements per lane per operand)
+//   mma4x4x4: 16 blocks of A[4 x 4] * B[4 x 4] (4 elements per lane per operand)
 // ---------------------------------------------------------------------------
 template <int DT>
 struct Dt;
@@ -101,6 +102,9 @@ struct Dt<kBF16> {
   static __device__ __forceinline__ f32x16 mma32x32x16(u32x4 a, u32x4 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
                                                    __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ f32x4 mma4x4x4(u32x2 a, u32x2 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(__builtin_bit_cast(s16x4, a), __builtin_bit_cast(s16x4, b), c, 0, 0, 0);
   }
   static constexpr uint32_t kOnes = 0x3F803F80u;  // a packed pair of ones
   // two fp8 e4m3 values (bytes 0-1, or 2-3 when hi) of w as a packed pair;
@@ -136,6 +140,9 @@ struct Dt<kF16> {
   static __device__ __forceinline__ f32x16 mma32x32x16(u32x4 a, u32x4 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a),
                                                   __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ f32x4 mma4x4x4(u32x2 a, u32x2 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_4x4x4f16(__builtin_bit_cast(f16x4, a), __builtin_bit_cast(f16x4, b), c, 0, 0, 0);
   }
   static constexpr uint32_t kOnes = 0x3C003C00u;
   // two fp8 e4m3 values as a packed pair; exact (e4m3's range and 3-bit
@@ -390,29 +397,16 @@ __device__ __forceinline__ u32x2 lds_read_tr16(const uint16_t* p) {
   return __builtin_bit_cast(u32x2, r);
 }
 
-// Row sums of packed probabilities on the matrix cores.  The B operand of a
-// 32x32x16 product (lane l: column l % 32, k-group l / 32, 8 values) fed as the
-// B operand of a 16x16x32 one reads as columns l % 16 with k-groups l / 16:
-// groups 0 and 2 are columns 0 .. 15, groups 1 and 3 columns 16 .. 31.  Against
-// an A of ones in even rows for groups 0, 2 and in odd rows for groups 1, 3,
-// register 0 of the result holds the sum of column l % 16 and register 1 that of
-// column l % 16 + 16, in every lane group.  (Two v_add_f32 per pair would sum
-// the unrounded values; a v_dot2c of the pair holds the matrix pipe as long as
-// this whole product, which sums 8 values per lane.)
+// acc + the lane's own 8 packed values p, in every register of acc: two 4x4x4
+// products of 16 blocks, against an A of ones (block l / 4, column l % 4 is
+// lane l's, so a NaN or infinity in one lane reaches no other lane's sum).  They
+// hold the matrix pipe for 16 cycles together; as many v_dot2c of one pair each
+// would take 64, and adds of the unrounded values 8 vector instructions.
 template <int DT>
-__device__ __forceinline__ u32x4 row_sum_ones() {
-  const int l = static_cast<int>(threadIdx.x) & (kWave - 1);
-  const uint32_t w = ((l ^ (l >> 4)) & 1) == 0 ? Dt<DT>::kOnes : 0u;
-  return u32x4{w, w, w, w};
-}
-// the lane's column (l % 32) of such sums
-__device__ __forceinline__ float row_sum_of(f32x4 sums) { return (threadIdx.x & 16) ? sums[1] : sums[0]; }
-// sums times a factor per column (f: that of the lane's own column)
-__device__ __forceinline__ void row_sum_scale(f32x4& sums, float f) {
-  const float g = __shfl_xor(f, 16, kWave);
-  const bool hi = threadIdx.x & 16;
-  sums[0] *= hi ? g : f;
-  sums[1] *= hi ? f : g;
+__device__ __forceinline__ f32x4 lane_sum8(u32x4 p, f32x4 acc) {
+  constexpr u32x2 ones = {Dt<DT>::kOnes, Dt<DT>::kOnes};
+  acc = Dt<DT>::mma4x4x4(ones, u32x2{p.x, p.y}, acc);
+  return Dt<DT>::mma4x4x4(ones, u32x2{p.z, p.w}, acc);
 }
 
 // Scheduling fence: the compiler's instruction scheduler moves nothing

@@ -442,8 +442,7 @@ __device__ __forceinline__ void half_tile(const PrefillParams& p, int row0, int 
   const float scale_inv_log2 = 1.f / p.scale_log2;
   float m_run = -INFINITY;  // running max of this lane's M-row (raw score units)
   float l_run = 0.f;        // fp8: this lane's share of the exp-sum
-  f32x4 l_sum = {0.f, 0.f, 0.f, 0.f};  // else: sums of the probabilities as rounded for the PV product
-  const u32x4 ones = row_sum_ones<DT>();
+  f32x4 l_sum = {0.f, 0.f, 0.f, 0.f};  // else: of the probabilities as rounded for the PV product (register 0)
   f32x16 o[DT32];
 #pragma unroll
   for (int n = 0; n < DT32; ++n)
@@ -507,7 +506,7 @@ __device__ __forceinline__ void half_tile(const PrefillParams& p, int row0, int 
       const float a = grow ? alpha : 1.f;
       if (grow) m_run = m_new;
       if constexpr (F8) l_run *= a;
-      else row_sum_scale(l_sum, a);
+      else l_sum[0] *= a;
 #pragma unroll
       for (int n = 0; n < DT32; ++n) o[n] *= a;
     }
@@ -676,7 +675,7 @@ __device__ __forceinline__ void half_tile(const PrefillParams& p, int row0, int 
       }
       o[m % DT32] = Dt<DT>::mma32x32x16(va[m], pb[m / DT32], o[m % DT32]);
       if constexpr (!F8)
-        if (m % DT32 == 0) l_sum = Dt<DT>::mma16x16x32(ones, pb[m / DT32], l_sum);
+        if (m % DT32 == 0) l_sum = lane_sum8<DT>(pb[m / DT32], l_sum);
 #pragma unroll
       for (int r = m * 16 / KS; r < (m + 1) * 16 / KS; ++r) {
         if (kMask) mask_score(s_next, r, st + 1);
@@ -697,7 +696,7 @@ __device__ __forceinline__ void half_tile(const PrefillParams& p, int row0, int 
   // ---- normalise and write: lane holds O[M-row col][32n + 8(r/4) + 4 half + r%4]
   float l;
   if constexpr (F8) l = sum_xor32(l_run);
-  else l = row_sum_of(l_sum);
+  else l = sum_xor32(l_sum[0]);
   if (row_ok) {
     const float inv = l > 0.f ? 1.f / l : 0.f;
     const int64_t orow = static_cast<int64_t>(row0 + my_t) * p.num_q_heads + kvh * p.group + h0 + my_h;

@@ -36,8 +36,8 @@
 //    instruction.  In the transposed products a lane owns one M-row, so the
 //    softmax max needs one cross-half exchange (v_permlane32_swap) and the
 //    probabilities go into the PV MFMA without leaving the lane.  The sum of
-//    the rounded probabilities comes from an MFMA with ones (v_dot2 holds the
-//    matrix pipe for 16 cycles each).  K is stored in the QK operand's row
+//    the rounded probabilities comes from MFMAs with ones, each lane's own
+//    (v_dot2 holds the matrix pipe for 16 cycles each).  K is stored in the QK operand's row
 //    order and V rows are swizzled, so every operand read is one conflict-free
 //    16-byte LDS access.
 //  * Steps are software-pipelined inside a wavefront: the QK MFMAs of step
@@ -751,11 +751,10 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
   };
 
   float mb[RG];     // minus the running max of this lane's M-row (log2 units; 0 before its first key)
-  // exp-sum: of the probabilities as rounded for the PV product, by MFMA
-  // (fp8: this lane's share of the sum, before the V scale)
+  // this lane's share of the exp-sum: of the probabilities as rounded for the
+  // PV product, by MFMA (register 0; fp8: of the probabilities before the V scale)
   f32x4 l_sum[F8 ? 1 : RG];
   float l_run[RG];
-  const u32x4 ones = row_sum_ones<DT>();
   // O^T of row group r, row tile n (dims 32 n ..): accumulator r * DT32 + n
   static_assert(RG * DT32 <= 8, "eight accumulators");
   acc_reserve();
@@ -1130,11 +1129,11 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
           if (q < kSumA) pair_sum(q);
         }
       }
-      if constexpr (!F8) {  // the exp-sum's MFMAs, one per row group and PV k-step
+      if constexpr (!F8) {  // the exp-sum's MFMAs, a pair per row group and PV k-step
         constexpr int kAt = NCH >= 8 ? 2 : 0;  // (every probability is packed by the end of chunk 0)
         if (c >= kAt && c < kAt + 2 * RG) {
           const int x = c - kAt;
-          l_sum[x % RG] = Dt<DT>::mma16x16x32(ones, pp[x % RG][x / RG], l_sum[x % RG]);
+          l_sum[x % RG] = lane_sum8<DT>(pp[x % RG][x / RG], l_sum[x % RG]);
         }
       }
       if constexpr (RG == 2) {  // before chunk kFirst + (NCH - kFirst) / 2
@@ -1178,7 +1177,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
           scale[r] = __builtin_amdgcn_exp2f(d);
           mb[r] = m_new;
           if constexpr (F8) l_run[r] *= scale[r];
-          else row_sum_scale(l_sum[r], scale[r]);
+          else l_sum[r][0] *= scale[r];
 #pragma unroll
           for (int x = 0; x < 16; ++x) e_cur[r][x] += d;
         }
@@ -1254,7 +1253,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
     uint16_t* region = k_lds_base + (w * RG + r) * 32 * HD;  // K buffers, then V buffers: 8 regions of 32 rows
     float l;
     if constexpr (F8) l = sum_xor32(l_run[r]);
-    else l = row_sum_of(l_sum[r]);
+    else l = sum_xor32(l_sum[r][0]);
     const float inv = l > 0.f ? 1.f / l : 0.f;
     static_for<DT32 * 4>([&](auto qc) {
       constexpr int c = decltype(qc)::value, n = c / 4, q4 = c % 4;

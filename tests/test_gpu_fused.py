@@ -220,3 +220,36 @@ def test_fused_tile_claims_across_head_dims():
     sequences, from the counters of one workspace."""
     for i, hd in enumerate([256, 64, 256, 32]):
         _check_fused(make_fused_case(90 + i, [], [(10, 700)], 64, 32, hd, 16, "bf16", block=700), f"claims hd{hd}")
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("hd,tpp", [(32, 16), (64, 32), (128, 16), (256, 16)])
+@pytest.mark.parametrize("decode,rows,heads", [([], 90, (16, 1)), ([], 2300, (8, 8)), ([300], 60, (8, 2))],
+                         ids=["wide", "wide-more-rows", "beside-decode"])
+def test_fused_nan_stays_in_its_rows(decode, rows, heads, hd, tpp, dtype):
+    """A NaN in one query head of one row, or in a key that only the last row
+    sees, leaves every other row's bits as they are without it."""
+    fc = make_fused_case(hd + rows, decode, [(30, rows)], *heads, hd, tpp, dtype, block=rows)
+    c = fc.case
+    announce(f"NaN rows: fused R={len(fc.q2seq)} heads={heads} HD={hd} TPP={tpp} {dtype}")
+    nan = 0x7FC0 if dtype == "bf16" else 0x7E00
+    clean = host_bits(_fused_gpu(c, fc.queries, fc.q2seq, fc.q_offset))
+    chunk = np.flatnonzero(fc.q2seq == len(decode))  # in position order
+
+    q = fc.queries.copy()
+    hit = chunk[[3, 40, len(chunk) - 1]]
+    q[hit, 1, 5] = nan
+    out = _fused_gpu(c, q, fc.q2seq, fc.q_offset)
+    keep = np.ones(clean.shape[:2], bool)
+    keep[hit, 1] = False
+    assert np.isnan(host_f32(out)[hit, 1]).all()
+    assert np.array_equal(host_bits(out)[keep], clean[keep])
+
+    last = int(c.seq_lens[len(decode)]) - 1
+    page = int(c.page_table[len(decode), last // tpp])
+    c.k_pool[page, :, 0, last % tpp, 2] = nan
+    out = _fused_gpu(c, fc.queries, fc.q2seq, fc.q_offset)
+    keep = np.ones(len(clean), bool)
+    keep[chunk[-1]] = False
+    assert np.isnan(host_f32(out)[chunk[-1]]).all()
+    assert np.array_equal(host_bits(out)[keep], clean[keep])

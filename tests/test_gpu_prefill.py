@@ -176,3 +176,35 @@ def test_prefill_tile_rounds(plen, hd, tpp, dtype):
     three rows in the last one, 520 rows 816 / 432, two rounds of the larger
     tiles (head dims above 128 have the smaller ones only)."""
     _check(hd + plen, [0, 33, 150], plen, 64, 16, hd, tpp, dtype, "tile rounds")
+
+
+@pytest.mark.parametrize("hd,tpp,dtype", [(32, 16, "bf16"), (64, 32, "f16"), (96, 8, "bf16"), (128, 16, "f16"),
+                                          (256, 16, "bf16")])
+@pytest.mark.parametrize("plen,heads", [(40, (8, 2)), (700, (32, 16))])
+def test_prefill_nan_stays_in_its_rows(plen, heads, hd, tpp, dtype):
+    """A NaN in one query head of one prompt row, or in the last prompt key,
+    leaves every other row's bits as they are without it."""
+    case, q, k, v = make_prefill_case(hd + plen, [0, 45], plen, *heads, hd, tpp, dtype)
+    announce(f"NaN rows: prefill P={plen} heads={heads} HD={hd} TPP={tpp} {dtype}")
+    nan = 0x7FC0 if dtype == "bf16" else 0x7E00
+    pools = (case.k_pool, case.v_pool, case.page_table, case.seq_lens, dtype)
+    rows = 2 * plen
+
+    def run(qq, kk):
+        out = _prefill_gpu(qq, kk, v, *pools)
+        return host_bits(out).reshape(rows, heads[0], hd), host_f32(out).reshape(rows, heads[0], hd)
+
+    clean, _ = run(q, k)
+    bad_q = q.copy()
+    hit = np.array([2, 25, plen - 1, plen + 7])
+    bad_q[hit, 1, 5] = nan
+    bits, vals = run(bad_q, k)
+    keep = np.ones((rows, heads[0]), bool)
+    keep[hit, 1] = False
+    assert np.isnan(vals[hit, 1]).all()
+    assert np.array_equal(bits[keep], clean[keep])
+    bad_k = k.copy()
+    bad_k[rows - 1, :, 3] = nan  # the last key of the second sequence: its last row alone sees it
+    bits, vals = run(q, bad_k)
+    assert np.isnan(vals[rows - 1]).all()
+    assert np.array_equal(bits[:-1], clean[:-1])
