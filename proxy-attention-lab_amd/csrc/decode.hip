@@ -889,7 +889,7 @@ __device__ __forceinline__ void fused_claim_rows(const DecodeParams& p, FusedDec
   for (;;) {
     uint32_t k = 0;
     if (lane == 0) k = atomicAdd(p.claim, 1u);
-    const int64_t batch = static_cast<int64_t>(__builtin_amdgcn_readfirstlane(k)) * kWave;
+    const int64_t batch = static_cast<int64_t>(__builtin_amdgcn_readfirstlane(k) & (kClaimsTaken - 1)) * kWave;
     if (batch >= n_rows) break;
     const int64_t r = batch + lane;
     int32_t len = 0;
@@ -1094,13 +1094,6 @@ void fused_wide_kernel(const DecodeParams dp, const PrefillParams pp) {
   prefill_items<DT, HD, TPP, KV8, RG, false>(pp, blockIdx.x, gridDim.x, lds.f);
 }
 
-// The claim counters, zero again for the next call: the lone rows' counter and
-// the tiles' (kQueues words, kTileClaims after it).
-__device__ __forceinline__ void rearm_claims(const DecodeParams& p) {
-  if (threadIdx.x == 0) *p.claim = 0u;
-  if (p.q2seq && threadIdx.x < kQueues) p.claim[kTileClaims + threadIdx.x] = 0u;
-}
-
 // Walks the merge list, slot v for virtual worker v (first block < 0:
 // nothing to merge; every slot of the live range was written by this call's
 // workers, with the segment's first block, block count, output row and
@@ -1120,10 +1113,10 @@ __device__ __forceinline__ void rearm_claims(const DecodeParams& p) {
 // 8 dims (16 bytes) per lane, plus each row's (max, exp-sum): two load
 // instructions per head instead of one per element.  A segment with more
 // than three contributors is finished by the general loop.  Workgroup 0
-// re-arms the claim counters.
+// re-arms the claim word.
 template <int DT, int HD, int TPP>
 __global__ __launch_bounds__(kGroupThreads) void decode_merge_kernel(const DecodeParams p) {
-  if (blockIdx.x == 0) rearm_claims(p);
+  if (blockIdx.x == 0 && threadIdx.x == 0) *p.claim = 0u;
   const int lane = lane_id();
   const int wv = wave_id();
   constexpr int kCh = (HD + 127) / 128;                 // 8-dim chunks of a row per lane (16 lanes per row)
@@ -1314,7 +1307,7 @@ constexpr int kSegDims = 32;
 
 template <int DT, int HD, int TPP>
 __global__ __launch_bounds__(kGroupThreads) void decode_merge_seg_kernel(const DecodeParams p) {
-  if (blockIdx.x == 0) rearm_claims(p);
+  if (blockIdx.x == 0 && threadIdx.x == 0) *p.claim = 0u;
   constexpr int kDs = HD < kSegDims ? HD : kSegDims;
   constexpr int kSlices = (HD + kDs - 1) / kDs;
   constexpr int kDg = kDs / 8;                 // 8-dim groups per slice
@@ -1568,7 +1561,7 @@ hipError_t launch_fused_t(const DecodeParams& dp, PrefillParams pp, hipStream_t 
     if (err != hipSuccess) return err;
     return launch_merge<DT, HD, TPP>(dp, stream);
   } else {
-    // (tiles first: the decode's merge re-arms the tiles' claim counters)
+    // (tiles first: the decode's merge re-arms the claim word)
     const hipError_t err = launch_prefill(pp, DT, HD, TPP, stream);
     if (err != hipSuccess) return err;
     return launch_decode_t<DT, HD, TPP, KV8>(dp, stream);

@@ -63,10 +63,10 @@ size_t align256(size_t n) { return (n + 255) & ~static_cast<size_t>(255); }
 
 constexpr int kMaxPageSize = 1024;  // prefill's run-time page sizes (multiples of 8)
 
-// Decode workspace layout (all offsets 256-aligned).  The claim counters at
-// bytes 64 (lone rows) and 128 .. 159 (the fused op's tiles) must be zero when
-// a call starts; every call leaves them zero.  Every other byte is scratch that
-// each call writes before it reads.
+// Decode workspace layout (all offsets 256-aligned).  The 4-byte claim word at
+// byte 64 must be zero when a call starts; every call leaves it zero.  Every
+// other byte is scratch that each call writes before it reads (bytes 128 .. 159:
+// the counters the fused op's tiles are claimed from).
 struct DecodeLayout {
   size_t hdr, claim, cum, list, part_ml, part_o, total;
   int64_t list_cap;
@@ -353,7 +353,7 @@ int prefill_call(const void* q_prompt, const void* k_prompt, const void* v_promp
   p.seq_lens = context_lens;
   p.q_offset = nullptr;
   p.q2seq = nullptr;
-  p.claims = nullptr;
+  p.claim = nullptr;
   p.num_rows = num_query_rows;
   p.num_seqs = num_seqs;
   p.num_pages = num_pages;
@@ -468,7 +468,7 @@ int fused_call(const void* queries, const void* k_pool, const void* v_pool, cons
   pal::DecodeParams dp = decode_params(queries, k_pool, v_pool, page_table, sequence_lengths, out,
                                        static_cast<char*>(workspace), lay, num_query_rows, num_pages,
                                        page_table_width, num_q_heads, num_kv_heads, head_dim, resident, 0);
-  pp.claims = dp.claim + pal::kTileClaims;
+  pp.claim = dp.claim;
   dp.k_scales = k_scales;
   dp.v_scales = v_scales;
   dp.q2seq = query_to_seq_map;

@@ -69,8 +69,7 @@ struct DecodeParams {
   int64_t num_pt_rows;           // page-table rows (sequences) in row mode
   // workspace
   int64_t* hdr;                // hdr[0] = total blocks T
-  uint32_t* claim;             // dynamic-chunk counter, and 16 words on the 8 counters of the fused op's tiles:
-                               // 0 on entry, re-armed to 0 by the merge kernels
+  uint32_t* claim;             // claim word: dynamic-chunk counter and kClaims* bits; 0 on entry, re-armed to 0 by the merge kernels
   int64_t* split_list;         // [list_cap][4] per virtual worker: {first block (< 0: none), blocks,
                                // output row, segment} of the split segment its range ends in
                                // (every live slot is written by each call before the merge reads it)
@@ -103,8 +102,13 @@ hipError_t decode_resident_workers(int dtype, int head_dim, int tokens_per_page,
 int64_t decode_virtual_workers(int64_t resident, int64_t max_blocks, int partition_size);
 hipError_t launch_decode(const DecodeParams& p, int dtype, int head_dim, int tokens_per_page, hipStream_t stream);
 
-// Distance of the fused op's tile counters from DecodeParams::claim (words).
+// The fused op's tiles are claimed from 8 counters, kTileClaims words after the
+// claim word.  They hold anything when a call starts: the bits of the claim word
+// say whether the call's clearing of them has begun, and is done.  (The counter
+// below the bits counts batches of 64 rows, fewer than 2^27.)
 constexpr int kTileClaims = 16;
+constexpr uint32_t kClaimsTaken = 1u << 30;
+constexpr uint32_t kClaimsReady = 1u << 31;
 
 // Causal attention over query tiles (prefill rows).  Uniform-prompt mode
 // (prompt_len > 0): the reference prefill, keys past each sequence's history
@@ -124,7 +128,7 @@ struct PrefillParams {
   const int32_t* seq_lens;     // window mode: keys per sequence; prompt mode: history per sequence
   const int32_t* q_offset;     // window mode: [R] keys visible to each row (before the seq_lens clamp)
   const uint32_t* q2seq;       // window mode: [R] sequence of each row
-  uint32_t* claims;            // window mode: 8 item counters, zero on entry (re-armed by the merge kernel)
+  uint32_t* claim;             // window mode: the claim word (as DecodeParams::claim), the item counters behind it
   int64_t num_rows;            // R
   int64_t num_seqs;            // page-table rows
   int64_t num_pages;

@@ -159,17 +159,43 @@ struct ItemMap {
 };
 
 // Next-item claims of the window mode.  Items 8 apart (workgroups of one XCD:
-// the same few kv heads) form a queue with a counter of its own, zero when
-// the kernel starts; a workgroup claims from the queue of its XCD and, when
-// that is empty, from the others in turn.
+// the same few kv heads) form a queue with a counter of its own; a workgroup
+// claims from the queue of its XCD and, when that is empty, from the others in
+// turn.  Of the workspace only the claim word is zero when a call starts, so the
+// first workgroup of the call to claim (it sets kClaimsTaken) clears the
+// counters and then sets kClaimsReady; one that comes while it does so waits for
+// that bit.  The wait ends: the clearing thread is running and waits for
+// nothing.  The merge kernel clears the claim word.
 constexpr int kQueues = 8;
 struct Claim {
   uint32_t queue;   // queue asked
   uint32_t got;     // thread 0: the counter's value (in flight until read)
+  bool wanted;      // are there items that are not taken by place?
   bool asked;
+  bool ready;       // thread 0: the counters have been seen ready
+  __device__ __forceinline__ uint32_t take(const PrefillParams& p, uint32_t q) {
+    return atomicAdd(p.claim + kTileClaims + q, 1u);
+  }
   __device__ __forceinline__ void ask(const PrefillParams& p) {
-    if (threadIdx.x == 0) got = atomicAdd(p.claims + queue, 1u);
+    if (threadIdx.x == 0) {
+      if (!ready) make_ready(p);
+      ready = true;
+      got = take(p, queue);
+    }
     asked = true;
+  }
+  __device__ __forceinline__ void make_ready(const PrefillParams& p) {
+    uint32_t word = __hip_atomic_fetch_or(p.claim, kClaimsTaken, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
+    if (!(word & kClaimsTaken)) {
+      for (int q = 0; q < kQueues; ++q)
+        __hip_atomic_exchange(p.claim + kTileClaims + q, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_fetch_or(p.claim, kClaimsReady, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+      return;
+    }
+    while (!(word & kClaimsReady)) {
+      __builtin_amdgcn_s_sleep(1);
+      word = __hip_atomic_load(p.claim, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
+    }
   }
 };
 
@@ -1234,7 +1260,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
       step(Last{}, no, st);
   }
 
-  if (claim) claim->ask(p);  // the workgroup's next item, on its way while this tile is written
+  if (claim && claim->wanted) claim->ask(p);  // the workgroup's next item, on its way while this tile is written
   // ---- normalise and write: lane holds O[M-row col][32n + 8(x/4) + 4 half + x%4].
   // A store straight from the accumulators would write 16 bytes of each of 32
   // rows per instruction; the rows go through the step buffers instead (a
@@ -1414,7 +1440,7 @@ template <int DT, int HD, int TPP, bool KV8, int RG, bool kPromptMode>
 __device__ __forceinline__ void prefill_items(const PrefillParams& p, unsigned b, unsigned nb,
                                               PrefillLds<HD, KV8, RG>& L) {
   const unsigned items = static_cast<unsigned>(p.num_units) * p.num_kv_heads * p.head_chunks;
-  Claim claim{b % kQueues, 0u, false};
+  Claim claim{b % kQueues, 0u, items > nb, false, false};
   if constexpr (kPromptMode) {
     const unsigned mirrored = nb % 8 == 0 ? nb - 8 - (b & ~7u) + (b & 7u) : b;
     for (unsigned pass = 0; pass * nb < items; ++pass) {
@@ -1428,13 +1454,14 @@ __device__ __forceinline__ void prefill_items(const PrefillParams& p, unsigned b
     while (item < items) {
       claim.asked = false;
       prefill_item<DT, HD, TPP, KV8, RG, false>(p, item, claim, L);
+      if (!claim.wanted) return;
       if (!claim.asked) claim.ask(p);
       if (threadIdx.x == 0) {
         uint32_t q = claim.queue;
         unsigned next = item_of(q, claim.got);
         for (int k = 1; k < kQueues && next >= items; ++k) {  // that queue is empty: the next one with an item
           q = (q + 1) % kQueues;
-          next = item_of(q, atomicAdd(p.claims + q, 1u));
+          next = item_of(q, claim.take(p, q));
         }
         L.next[0] = next;
         L.next[1] = q;

@@ -13,9 +13,10 @@ import pytest
 import torch
 
 import proxy_attention_lab as pal
-from gpu_util import announce, dev_bits, dev_index, host_bits, host_f32
+from gpu_util import DEV, announce, dev_bits, dev_index, host_bits, host_f32
 from oracle import pal_oracle as orc
 from pal_cases import assert_close, extreme_query_bits, make_fused_case, make_paged_case, make_prefill_case, randn_bits
+from proxy_attention_lab import _lib
 
 pytestmark = pytest.mark.gpu
 DTYPES = ["f16", "bf16"]
@@ -253,3 +254,37 @@ def test_fused_nan_stays_in_its_rows(decode, rows, heads, hd, tpp, dtype):
     keep[chunk[-1]] = False
     assert np.isnan(host_f32(out)[chunk[-1]]).all()
     assert np.array_equal(host_bits(out)[keep], clean[keep])
+
+
+@pytest.mark.parametrize("hd", [64, 256])
+@pytest.mark.parametrize("rows,heads", [(2200, (32, 32)), (700, (64, 16)), (2300, (128, 8))],
+                         ids=["one-group", "few", "two-groups"])
+def test_fused_workspace_contract(rows, heads, hd):
+    """Of the workspace, the four bytes at 64 are all that has to be zero before
+    a call (head dim 64: 576 tiles of one row group on 256 CUs; 352 of one, 176
+    of two; 2,304 / 1,152: claimed, all taken by place, claimed), and are zero again
+    after it."""
+    hq, hkv = heads
+    fc = make_fused_case(rows + hd, [], [(10, rows)], hq, hkv, hd, 16, "bf16", block=rows)
+    c = fc.case
+    announce(f"fused workspace contract rows={rows} heads={heads} HD={hd}")
+    ref = host_bits(_fused_gpu(c, fc.queries, fc.q2seq, fc.q_offset))
+    lib = _lib.lib()
+    q, k, v = dev_bits(fc.queries, "bf16"), dev_bits(c.k_pool, "bf16"), dev_bits(c.v_pool, "bf16")
+    pt, lens = dev_index(c.page_table, torch.uint32), dev_index(c.seq_lens)
+    q2s, off = dev_index(fc.q2seq, torch.uint32), dev_index(fc.q_offset)
+    n = len(fc.q2seq)
+    size = lib.pal_paged_attention_workspace_size(_lib.DTYPE_BFLOAT16, n, hq, hkv, hd, 16)
+    ws = torch.zeros(size, dtype=torch.uint8, device=DEV)
+    ws[:256] = 0xA5
+    ws[64:68] = 0
+    for call in range(2):
+        out = torch.full_like(q, 7.0)
+        st = lib.pal_paged_attention(q.data_ptr(), k.data_ptr(), v.data_ptr(), pt.data_ptr(), lens.data_ptr(),
+                                     q2s.data_ptr(), off.data_ptr(), out.data_ptr(), _lib.DTYPE_BFLOAT16, n, c.num_seqs,
+                                     hq, hkv, hd, 16, int(c.k_pool.shape[0]), int(c.page_table.shape[1]), ws.data_ptr(),
+                                     size, torch.cuda.current_stream().cuda_stream)
+        assert st == 0, lib.pal_last_error()
+        torch.cuda.synchronize()
+        assert np.array_equal(host_bits(out), ref), f"call {call}"
+        assert not ws[64:68].any(), f"call {call}"
