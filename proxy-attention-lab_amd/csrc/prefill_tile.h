@@ -889,6 +889,23 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
     barrier();
   };
   f32x16 e_cur[RG];
+  // Step j's largest score (log2 units) of M-row r that the row sees, and its
+  // exponents with the running max as it is now.  Both come from the raw scores:
+  // an exponent is rounded once, in its fma, however far the max moves.
+  auto step_max = [&](int r, int j, bool masked, const f32x16& s, float sc) {
+    float bm = -INFINITY;
+#pragma unroll
+    for (int x = 0; x < 16; ++x)
+      if (!masked || place(x) < seen(r, j)) bm = fmaxf(bm, s[x] * sc);
+    return max_xor32(bm);
+  };
+  auto exponents = [&](int r, int j, bool masked, const f32x16& s, float sc) {
+#pragma unroll
+    for (int x = 0; x < 16; ++x) {
+      const float v = fmaf(s[x], sc, mb[r]);
+      e_cur[r][x] = !masked || place(x) < seen(r, j) ? v : -INFINITY;
+    }
+  };
   u32x4 ka[F8 ? KS / 2 : KS];  // K operands of the next QK product (fp8: raw items of two k-steps)
   auto k_operand = [&](int kk) {
     if constexpr (F8) {  // exact in 16 bits; the K scale goes on the scores
@@ -970,17 +987,9 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
     const float sc = score_scale(0);
 #pragma unroll
     for (int r = 0; r < RG; ++r) {
-      float bm = -INFINITY;
-#pragma unroll
-      for (int x = 0; x < 16; ++x) {
-        e_cur[r][x] = s0[r][x] * sc;
-        if (min_lim < kKeys && place(x) >= seen(r, 0)) e_cur[r][x] = -INFINITY;
-        bm = fmaxf(bm, e_cur[r][x]);
-      }
-      bm = max_xor32(bm);
+      const float bm = step_max(r, 0, min_lim < kKeys, s0[r], sc);
       mb[r] = bm == -INFINITY ? 0.f : -bm;
-#pragma unroll
-      for (int x = 0; x < 16; ++x) e_cur[r][x] += mb[r];
+      exponents(r, 0, min_lim < kKeys, s0[r], sc);
     }
   }
   // One iteration.  kFast: step st+1 needs no mask and the iteration's copies
@@ -1197,15 +1206,13 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
         float scale[RG];
 #pragma unroll
         for (int r = 0; r < RG; ++r) {
-          const float row_max = max_xor32(bm[r]);
-          const float m_new = row_max > kLazyRescale ? mb[r] - row_max : mb[r];
-          const float d = m_new - mb[r];
-          scale[r] = __builtin_amdgcn_exp2f(d);
+          const bool moves = max_xor32(bm[r]) > kLazyRescale;
+          const float m_new = moves ? -step_max(r, st + 1, kMode == kAny, s_next[r], sc) : mb[r];
+          scale[r] = __builtin_amdgcn_exp2f(m_new - mb[r]);
           mb[r] = m_new;
+          exponents(r, st + 1, kMode == kAny, s_next[r], sc);
           if constexpr (F8) l_run[r] *= scale[r];
           else l_sum[r][0] *= scale[r];
-#pragma unroll
-          for (int x = 0; x < 16; ++x) e_cur[r][x] += d;
         }
         static_for<RG * DT32 * 16>([&](auto x) {
           constexpr int X = decltype(x)::value;

@@ -208,3 +208,36 @@ def test_prefill_nan_stays_in_its_rows(plen, heads, hd, tpp, dtype):
     bits, vals = run(q, bad_k)
     assert np.isnan(vals[rows - 1]).all()
     assert np.array_equal(bits[:-1], clean[:-1])
+
+
+@pytest.mark.parametrize("hist", [0, 32, 320])
+def test_prefill_exponents_round_once(hist):
+    """Two keys whose scores are about 1.9e5 (log2 units) and differ by N(0, 1):
+    their probabilities depend on the difference alone, however large the scores
+    and however far the running max moves (after hist keys of score 0).
+
+    Scores are exact in fp32 here (multiples of 2^-3 below 2^21).  A rounding of
+    a key's own scaled score (2^-7 of its magnitude 2^17.5) would shift its
+    probability by up to 0.5 %; what is left is the probabilities' rounding to
+    fp16 (2^-12 each) and the output's (2^-12): 7.4e-4."""
+    hq, hkv, hd, seqs = 16, 4, 64, 32
+    rng = np.random.default_rng(17 + hist)
+    k1 = np.round(rng.standard_normal((seqs * 2, hkv)) * 64) / 64
+    k = np.zeros((seqs * 2, hkv, hd), np.float32)
+    k[..., 0] = 1024
+    k[..., 1] = k1
+    v = np.zeros_like(k)
+    v[0::2] = 1
+    v[1::2] = -1
+    q = np.zeros((seqs * 2, hq, hd), np.float32)
+    q[..., 0] = 1024
+    q[..., 1] = 8
+    case, *_ = make_prefill_case(5, [hist] * seqs, 2, hq, hkv, hd, 16, "f16")
+    case.k_pool[:] = 0
+    announce(f"prefill exponents of large scores, hist={hist}")
+    out = host_f32(_prefill_gpu(*(orc.f32_to_bits(x, "f16") for x in (q, k, v)), case.k_pool, case.v_pool,
+                                case.page_table, case.seq_lens, "f16")).reshape(seqs, 2, hq, hd)
+    d = (k1[0::2] - k1[1::2]).astype(np.float64)  # [seqs, hkv]; the last row sees both keys
+    expect = np.repeat(np.tanh(d / 2), hq // hkv, axis=1)
+    err = np.abs(out[:, 1] - expect[:, :, None]).max()
+    assert err < 1e-3, err
