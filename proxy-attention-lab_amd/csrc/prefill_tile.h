@@ -83,6 +83,7 @@ constexpr int kPfThreads = kPfWaves * kWave;
 constexpr int m_rows(int rg) { return kPfWaves * 32 * rg; }
 static_assert(kPidChunk % kPfThreads == 0, "a page-id chunk is a whole number of loads per thread");
 constexpr float kLazyRescale = 8.f;    // log2 headroom before the running max moves
+constexpr float kNoMax = 0x1p126f;     // minus the running max of a row that has seen no score above -inf
 
 // A step moves 4*HD items of 16 bytes of K and as many of V.
 template <int HD>
@@ -776,7 +777,10 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
     return v;
   };
 
-  float mb[RG];     // minus the running max of this lane's M-row (log2 units; 0 before its first key)
+  // minus the running max of this lane's M-row (log2 units).  kNoMax, until the
+  // row's first score above -inf: with it the exponent of -inf is -inf, and that
+  // of any other score so far past the headroom that the max moves to it.
+  float mb[RG];
   // this lane's share of the exp-sum: of the probabilities as rounded for the
   // PV product, by MFMA (register 0; fp8: of the probabilities before the V scale)
   f32x4 l_sum[F8 ? 1 : RG];
@@ -988,7 +992,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
 #pragma unroll
     for (int r = 0; r < RG; ++r) {
       const float bm = step_max(r, 0, min_lim < kKeys, s0[r], sc);
-      mb[r] = bm == -INFINITY ? 0.f : -bm;
+      mb[r] = bm == -INFINITY ? kNoMax : -bm;
       exponents(r, 0, min_lim < kKeys, s0[r], sc);
     }
   }
@@ -1207,6 +1211,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
 #pragma unroll
         for (int r = 0; r < RG; ++r) {
           const bool moves = max_xor32(bm[r]) > kLazyRescale;
+          // (a row that moves has a score above -inf)
           const float m_new = moves ? -step_max(r, st + 1, kMode == kAny, s_next[r], sc) : mb[r];
           scale[r] = __builtin_amdgcn_exp2f(m_new - mb[r]);
           mb[r] = m_new;

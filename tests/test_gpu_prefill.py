@@ -241,3 +241,28 @@ def test_prefill_exponents_round_once(hist):
     expect = np.repeat(np.tanh(d / 2), hq // hkv, axis=1)
     err = np.abs(out[:, 1] - expect[:, :, None]).max()
     assert err < 1e-3, err
+
+
+@pytest.mark.parametrize("hd,tpp,dtype", [(64, 16, "f16"), (128, 32, "bf16"), (256, 16, "bf16")])
+@pytest.mark.parametrize("hist,lost", [(200, 40), (200, 100), (0, 33), (20, 64)])
+def test_prefill_first_keys_at_minus_infinity(hist, lost, hd, tpp, dtype):
+    """The first `lost` keys score -inf in every row, the others about -500 (log2
+    units): the first step's maximum is no running max, and rows that see one of
+    the later keys are softmaxes over those."""
+    plen, hq, hkv = 150, 8, 2
+    case, q, k, v = make_prefill_case(hd + hist + lost, [hist, hist], plen, hq, hkv, hd, tpp, dtype, garbage_tail=False)
+    qf, kf = orc.bits_to_f32(q, dtype), orc.bits_to_f32(k, dtype)
+    qf[..., 0], qf[..., 1] = np.abs(qf[..., 0]) + 1, 64
+    inf, minus = (orc.f32_to_bits(np.float32([x]), dtype)[0] for x in (-np.inf, -64 * np.sqrt(hd) / 11.3))
+    kf[..., 0], kf[..., 1] = 0, -64 * np.sqrt(hd) / 11.3
+    q, k = orc.f32_to_bits(qf, dtype), orc.f32_to_bits(kf, dtype)
+    case.k_pool[:, :, 0, :, 0], case.k_pool[:, :, 0, :, 1] = 0, minus
+    for s in range(2):
+        for pos in range(min(lost, hist)):
+            case.k_pool[case.page_table[s, pos // tpp], :, 0, pos % tpp, 0] = inf
+        k[s * plen:s * plen + max(0, lost - hist), :, 0] = inf
+    announce(f"prefill: {lost} keys at -inf, hist={hist} HD={hd} TPP={tpp} {dtype}")
+    out = host_f32(_prefill_gpu(q, k, v, case.k_pool, case.v_pool, case.page_table, case.seq_lens, dtype))
+    ref = orc.paged_attention_prefill(q, k, v, case.k_pool, case.v_pool, case.page_table, case.seq_lens, dtype)
+    rows = np.arange(2 * plen * hq) // hq % plen + hist >= lost  # rows that see a key above -inf
+    assert_close(out.reshape(-1, hd)[rows], ref.reshape(-1, hd)[rows], dtype, "keys at -inf")
