@@ -411,8 +411,13 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
   // pg0 / pg1: the pages of the step's first and (TP 16) second 16 keys.
   constexpr bool kAllItems = (F8 ? NI8 : NI) % kPfThreads == 0;  // no wavefront has a padding copy
   __builtin_assume(w >= 0 && w < kPfWaves);
+  // The copies take a page's (a prompt row's) stride as 32 bits; longer ones go
+  // the slow path.
+  const bool long_pages = page_stride * (KV8 ? 1 : 2) > 0xFFFFFFFFll;
+  const bool long_rows = PROMPT && dense_stride * 2 > 0xFFFFFFFFll;
   // page ids >= 2^32 - 1 cannot occur with fewer pages; such an id takes the slow path
-  const uint32_t np32 = p.num_pages > 0xFFFFFFFFll ? 0xFFFFFFFFu : static_cast<uint32_t>(p.num_pages);
+  const uint32_t np32 =
+      long_pages ? 0u : (p.num_pages > 0xFFFFFFFFll ? 0xFFFFFFFFu : static_cast<uint32_t>(p.num_pages));
   // fp8 items.  K item i: page half ph (TP 16), stripe c (dims 16c ..
   // 16c+15), key of the step; V item i: page half ph (TP 16) or 16-key half
   // of the page row (TP 32), row d.  Item i is LDS slot i.
@@ -501,7 +506,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
   // of such a step transpose).
   auto is_dense = [&](int j) {
     const int k0 = j * kKeys;
-    return PROMPT && k0 >= hist && k0 < max_lim;
+    return PROMPT && !long_rows && k0 >= hist && k0 < max_lim;
   };
   // Untransposed V rows, read back with transposing reads: each 16-lane
   // group reads 32 bytes of each of 4 consecutive keys, the other group of
@@ -923,7 +928,8 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
 #pragma unroll
     for (int kk = 0; kk < (F8 ? KS / 2 : KS); ++kk) ka[kk] = F8 ? read_k8(j, kk) : read_k(j, kk);
   };
-  const int paged_full = (TPP != 0 && (!KV8 || F8)) ? paged_keys / kKeys : 0;  // whole steps in pages
+  // whole steps in pages that the copies can read
+  const int paged_full = (TPP != 0 && (!KV8 || F8)) && !long_pages ? paged_keys / kKeys : 0;
   if (nsteps > 0) {
     auto pids = [&](int j, uint32_t& a, uint32_t& b) {
       const u32x2 v = read_pids(j);
@@ -1246,7 +1252,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
   // next iteration that stages a page-id chunk (an Any iteration), or dense
   // rows.
   const int n_main = min(nsteps - 1, min_lim / kKeys - 1);
-  const int fd = PROMPT ? min(nsteps, static_cast<int>((hist + kKeys - 1) / kKeys)) : nsteps;
+  const int fd = PROMPT && !long_rows ? min(nsteps, static_cast<int>((hist + kKeys - 1) / kKeys)) : nsteps;
   int st = 0;
   int staged_at = -2;  // the iteration that staged page ids last (its flag is read two iterations later)
   while (st < min(nsteps - 1, fd)) {
@@ -1316,10 +1322,9 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
       const int t = static_cast<int>((static_cast<uint32_t>(m) * p.hg_magic) >> 16);
       const int h = m - t * p.hg_max;
       const u32x4 val = *reinterpret_cast<const u32x4*>(region + row * HD + place_chunk(row, c) * 8);
-      // (offsets inside a tile's rows fit 32 bits)
       if (t < nrows && t < qt && h < hg)
         __builtin_nontemporal_store(
-            val, reinterpret_cast<u32x4_align8*>(out_tile + static_cast<uint32_t>((t * p.num_q_heads + h) * HD + c * 8)));
+            val, reinterpret_cast<u32x4_align8*>(out_tile + (static_cast<int64_t>(t) * p.num_q_heads + h) * HD + c * 8));
     }
   }
 }

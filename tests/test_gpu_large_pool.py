@@ -212,3 +212,32 @@ def test_large_pool_rope_fill(kv):
     assert np.array_equal(host_pool(kd[base:], kv), ek), "K pool differs"
     assert np.array_equal(host_pool(vd[base:], kv), ev), "V pool differs"
     assert np.array_equal(host_bits(qo), eq), "rotated queries differ"
+
+
+def test_prefill_pages_of_4_gib():
+    """262,144 kv heads of 32-token pages at head dim 256: one page of K is 4 GiB,
+    so its stride does not fit the 32 bits of the tiles' page copies.  A few
+    heads are compared, bit for bit, with the same operators over those heads
+    alone (pages of 48 KiB)."""
+    heads, hd, tpp, keys, rows = 1 << 18, 256, 32, 64, 2
+    some = torch.tensor([0, heads // 2 + 5, heads - 1], device=DEV)
+    announce("prefill over pages of 4 GiB")
+    g = torch.Generator(device=DEV)
+    g.manual_seed(3)
+
+    def randn(*shape):
+        return torch.empty(shape, dtype=torch.bfloat16, device=DEV).normal_(generator=g)
+
+    k_pool, v_pool = randn(2, heads, hd // 8, tpp, 8), randn(2, heads, hd, tpp)
+    q, k, v = (randn(rows, heads, hd) for _ in range(3))
+    pt, lens = dev_index(np.array([[1, 0]], np.uint32), torch.uint32), dev_index(np.array([keys]))
+    q2s, off = dev_index(np.zeros(rows, np.uint32), torch.uint32), dev_index(np.array([keys - 1, keys]))
+    pools = (k_pool, v_pool)
+    few = tuple(x[:, some].contiguous() for x in pools)
+    qs, ks, vs = (x[:, some].contiguous() for x in (q, k, v))
+    out = pal.paged_attention_prefill(q, k, v, *pools, pt, lens).view(rows, heads, hd)
+    ref = pal.paged_attention_prefill(qs, ks, vs, *few, pt, lens).view(rows, len(some), hd)
+    assert np.array_equal(host_bits(out[:, some]), host_bits(ref))
+    out = pal.paged_attention(q, *pools, pt, lens, q2s, off)
+    ref = pal.paged_attention(qs, *few, pt, lens, q2s, off)
+    assert np.array_equal(host_bits(out[:, some]), host_bits(ref))
