@@ -1079,7 +1079,7 @@ void fused_kernel(const DecodeParams dp, const PrefillParams pp, const unsigned 
   if (blockIdx.x < n_dec)
     fused_decode_body<DT, HD, TPP, shared_cu_prefetch<HD>(), KV8>(dp, lds.d);
   else
-    half_tile_block<DT, HD, TPP, KV8>(pp, blockIdx.x - n_dec, lds.f);
+    half_tile_block<DT, HD, TPP, KV8, false>(pp, blockIdx.x - n_dec, lds.f);
 }
 
 template <int DT, int HD, int TPP, bool KV8, int RG>

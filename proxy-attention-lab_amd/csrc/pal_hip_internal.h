@@ -141,7 +141,7 @@ struct PrefillParams {
   int group;
   int head_chunks;
   int hg_max;
-  int row_groups;        // 32-row groups per wavefront of a tile (1 or 2)
+  int row_groups;        // 32-row groups per wavefront of a tile with a CU to itself (1 or 2); 0: half tiles
   uint32_t hg_magic;     // ceil(2^16 / hg_max): m / hg_max = m * hg_magic >> 16 for m < 4096
   float scale_log2;      // log2(e) / sqrt(HD)
 };
@@ -149,7 +149,8 @@ struct PrefillParams {
 // Query tokens per prefill tile (and window) of the smaller size (one row
 // group, and half tiles) for a GQA group size.
 int prefill_tokens_per_tile(int group);
-// Chooses the size of tiles that have a CU to themselves: row_groups and num_units.
+// Chooses the tiles of a prefill launch: row_groups and num_units (up to head
+// dim 128 in window mode: of tiles that have a CU to themselves).
 hipError_t prefill_choose_tiles(PrefillParams& p, int head_dim);
 // (p holds the smaller tiles; the launch chooses)
 hipError_t launch_prefill(const PrefillParams& p, int dtype, int head_dim, int tokens_per_page, hipStream_t stream);

@@ -1,13 +1,17 @@
-// Prefill tiles within half of a SIMD's registers: the tiles that run beside
-// the decode stream of a mixed batch (fused_kernel in decode.hip), one tile
-// workgroup and one decode workgroup per CU.  A wavefront holds 32 M-rows, so
-// an operand read from LDS feeds one MFMA where the tiles of prefill_tile.h
-// (64 rows, the whole register file, nothing beside them) feed two; their
-// layouts, item maps and step geometry are the ones described there.
-//  * Every key is read from pages (window mode).  Per 32-key step the K and V
-//    tiles reach LDS by direct-to-LDS copies issued three steps ahead into four
-//    LDS buffers, with counted waits and one barrier per step; a step with an
-//    invalid page id takes a synchronous register path.
+// Prefill tiles within half of a SIMD's registers (up to head dim 128): the
+// tiles that run beside the decode stream of a mixed batch (fused_kernel in
+// decode.hip), one tile workgroup and one decode workgroup per CU, and two to a
+// CU in the prefill kernels, for the calls that whole tiles do not serve faster
+// (prefill_choose_tiles).  A wavefront holds 32 M-rows, so an operand read from
+// LDS feeds one MFMA where the tiles of prefill_tile.h (64 rows, the whole
+// register file, nothing beside them) feed two; their layouts, item maps and
+// step geometry are the ones described there.
+//  * Per 32-key step the K and V tiles reach LDS by direct-to-LDS copies issued
+//    three steps ahead into four LDS buffers, with counted waits and one barrier
+//    per step.  Steps of dense prompt keys are copied the same way from the
+//    prompt rows; steps with an invalid page id, across the history / prompt
+//    boundary, and of prompts over fp8 pages or pages of a run-time size take a
+//    synchronous register path.
 //  * The QK MFMAs of step st+1 are issued among the exponentials of step st,
 //    and the step's copies among the PV MFMAs.
 //  * The exponent offset and the row max are handled as in prefill_tile.h.
@@ -21,18 +25,29 @@ namespace {
 constexpr int kHalfRows = kPfWaves * 32;  // M-rows (token, head) per workgroup
 
 // One query tile: rows [row0, row0 + nrows) of sequence s (nrows <= tokens
-// per tile), query heads h0 .. h0+15 of kv head kvh; every key from pages.
-template <int DT, int HD, int TPP, bool KV8>
+// per tile), query heads h0 .. h0+15 of kv head kvh.  PROMPT: the
+// uniform-prompt mode (keys below the history length from pages, the rest
+// from the dense prompt rows of sequence s); otherwise every key from pages.
+template <int DT, int HD, int TPP, bool PROMPT, bool KV8>
 __device__ __forceinline__ void half_tile(const PrefillParams& p, int row0, int nrows, int64_t s, int kvh, int h0,
                                              uint16_t* k_lds_base, uint16_t* v_lds_base, uint16_t* junk_lds,
                                              uint32_t* pid_lds, int* lim_lds, float* scl_lds) {
+  // TPP 0: the page size is p.tokens_per_page, known at run time (a
+  // multiple of 8; the reference prefill takes any, paged_attention_prefill.h.metal:
+  // 243-263).  Steps of history keys then take the register path, reading
+  // each key's page id from the page table; steps of dense prompt keys are
+  // copied as for the other page sizes.  LDS holds every step in the
+  // 32-key-page item order.
+  constexpr int TP = TPP == 0 ? 32 : TPP;  // page size of the LDS item order
+  const int tpp = TPP == 0 ? p.tokens_per_page : TPP;
+  static_assert(TPP != 0 || (PROMPT && !KV8), "run-time page sizes: uniform-prompt mode, 16-bit pools");
   static_assert(HD % 32 == 0, "prefill needs head_dim % 32 == 0");
   static_assert(2 * StepGeo<HD>::kLoads <= HD / 16, "a step's copies fit in its PV chunks");
   constexpr int KS = HD / 16;  // QK k-steps of 16
   constexpr int DT32 = HD / 32;  // O^T row tiles of 32 dims
   constexpr int NI = StepGeo<HD>::kItems;
   constexpr int NL = StepGeo<HD>::kLoads;
-  using IM = ItemMap<HD, TPP>;
+  using IM = ItemMap<HD, TP>;
   // fp8 pools in window mode: steps are copied as fp8 bytes (16-byte items:
   // 16 dims of one key for K, 16 keys of one row for V; 2 HD items each, in
   // item order) and converted in the operand reads, each lane reading whole
@@ -40,7 +55,7 @@ __device__ __forceinline__ void half_tile(const PrefillParams& p, int row0, int 
   // of both PV k-steps (the keys of an fp8 step are in kperm_f8 order, the
   // query operand permuted to match).  A copy instruction must stay in one
   // page: with TPP 16 that needs HD % 64 == 0 (every fp8 pool's head dim).
-  constexpr bool F8 = KV8;
+  constexpr bool F8 = KV8 && !PROMPT;
   constexpr int NI8 = 2 * HD;
   constexpr int NL8 = (NI8 + kPfThreads - 1) / kPfThreads;
   constexpr int NC = F8 ? NL8 : NL;  // copies per thread per step, K (and V)
@@ -63,10 +78,15 @@ __device__ __forceinline__ void half_tile(const PrefillParams& p, int row0, int 
   const int col = lane & 31;  // this lane's M-row within the wave
   const int half = lane >> 5;
 
-  const int64_t max_tokens = p.page_table_width * TPP;
+  const int64_t max_tokens = p.page_table_width * tpp;
+  int64_t hist = 0;  // prompt mode: keys below hist come from pages
   int64_t slen = seq_ok ? p.seq_lens[s] : 0;
   PAL_DEBUG_FLAG(slen > max_tokens, kDebugLength);
   slen = slen < 0 ? 0 : (slen > max_tokens ? max_tokens : slen);
+  if constexpr (PROMPT) {
+    hist = slen;
+    slen += p.prompt_len;
+  }
 
   // Loads that need nothing but the tile's coordinates go out first, so
   // their latency overlaps the row-limit round trip: the query operand and
@@ -113,7 +133,7 @@ __device__ __forceinline__ void half_tile(const PrefillParams& p, int row0, int 
     const bool live = tid < nrows && tid < qt;
     int lim = 0;
     if (live) {
-      int64_t off = p.q_offset[row0 + tid];
+      int64_t off = PROMPT ? hist + (row0 + tid - s * p.prompt_len) + 1 : p.q_offset[row0 + tid];
       off = off < 0 ? 0 : off;
       lim = static_cast<int>(off < slen ? off : slen);
     }
@@ -151,13 +171,18 @@ __device__ __forceinline__ void half_tile(const PrefillParams& p, int row0, int 
   min_lim = __builtin_amdgcn_readfirstlane(min_lim);
   const int my_lim = row_ok ? lim_lds[my_t] : 0;
 
-  const int64_t head_block = static_cast<int64_t>(HD) * TPP;
+  const int64_t head_block = static_cast<int64_t>(HD) * tpp;
   const int64_t page_stride = head_block * p.num_kv_heads;
   const int64_t page_stride8 = page_stride;            // fp8 pools: bytes per page (one byte per element)
   const int64_t kv_head_off8 = kvh * head_block;       // and of a kv head's block
   const int64_t kv_head_off = kvh * head_block;
   const int nsteps = (max_lim + kKeys - 1) / kKeys;
-  const int n_pid = (max_lim + TPP - 1) / TPP;  // page-table entries the tile reads
+  const int64_t dense_row0 = s * p.prompt_len - hist;  // dense row of key token tok: dense_row0 + tok
+  const int64_t dense_stride = static_cast<int64_t>(p.num_kv_heads) * HD;
+  // page-table entries the tile reads: keys below max_lim, and in prompt mode
+  // only those below the history (the rest are dense) -- never past the width
+  const int paged_keys = PROMPT ? min(max_lim, static_cast<int>(hist)) : max_lim;
+  const int n_pid = TPP == 0 ? 0 : (paged_keys + TP - 1) / TP;  // run-time page size: no staged ids
 
   // Page ids live in LDS (two chunks of 512 entries, entry e in slot e % 1024):
   // reading them is an LDS broadcast, so the only vector-memory traffic in the
@@ -181,11 +206,11 @@ __device__ __forceinline__ void half_tile(const PrefillParams& p, int row0, int 
   };
 
   // Fast step: its first key below the tile's largest limit (the last step
-  // may end past it), in valid pages: one direct-to-LDS copy per
-  // item, no registers, nothing to wait for here.  Every wavefront issues exactly
+  // may end past it), in valid pages (and, in prompt mode, all 32 keys below
+  // the history, or all of them prompt keys): one direct-to-LDS copy per item, no registers, nothing to wait for here.  Every wavefront issues exactly
   // 2*NL copies (items past the step go to a junk slot), so the wait counts
   // are the same on every wavefront.
-  // Slow step (invalid pages): register loads,
+  // Slow step (invalid pages, history / prompt boundary, fp8 in prompt mode): register loads,
   // masked, then LDS stores -- synchronous, so it also drains the copies in
   // flight, which keeps the counted waits safe.
   // pg0 / pg1: the pages of the step's first and (TP 16) second 16 keys.
@@ -209,7 +234,7 @@ __device__ __forceinline__ void half_tile(const PrefillParams& p, int row0, int 
       const uint16_t* page = p.v_pool + (IM::k_page_half(ok ? ib : 0) ? off1 : off0);
       int d = 0, key = 0;
       if (ok) IM::v_item(i, d, key);
-      const uint32_t src = 2u * static_cast<uint32_t>(d * TPP + key % TPP);
+      const uint32_t src = 2u * static_cast<uint32_t>(d * TP + key % TP);
       copy_to_lds16(page, src, lds_addr(ok ? v_lds(buf) + ib * 8 : junk_lds));
     }
   };
@@ -217,7 +242,7 @@ __device__ __forceinline__ void half_tile(const PrefillParams& p, int row0, int 
   // 16c+15), key of the step; V item i: page half ph (TP 16) or 16-key half
   // of the page row (TP 32), row d.  Item i is LDS slot i.
   auto k8_item = [](int i, int& ph, int& c, int& key) {
-    if (TPP == 16) {  // page-major; page 1's keys at positions XOR 12, so a 16-lane operand read spans all banks
+    if (TP == 16) {  // page-major; page 1's keys at positions XOR 12, so a 16-lane operand read spans all banks
       ph = i / HD;
       c = (i % HD) / 16;
       key = 16 * ph + ((i % 16) ^ (ph ? 12 : 0));
@@ -228,7 +253,7 @@ __device__ __forceinline__ void half_tile(const PrefillParams& p, int row0, int 
     }
   };
   auto v8_item = [](int i, int& ph, int& d, int& kb) {  // kb: the item's first key in the step
-    ph = TPP == 16 ? i / HD : 0;
+    ph = TP == 16 ? i / HD : 0;
     d = i % HD;
     kb = 16 * (i / HD);
   };
@@ -245,12 +270,12 @@ __device__ __forceinline__ void half_tile(const PrefillParams& p, int row0, int 
     uint32_t src = 0;
     if (q < NL8) {
       if (ok) k8_item(i, ph, a, b);
-      src = static_cast<uint32_t>((a * TPP + b % TPP) * 16);
+      src = static_cast<uint32_t>((a * TP + b % TP) * 16);
     } else {
       if (ok) v8_item(i, ph, a, b);
-      src = static_cast<uint32_t>(a * TPP + b % TPP);
+      src = static_cast<uint32_t>(a * TP + b % TP);
     }
-    const int phw = (TPP == 16 && ok) ? ib / HD : 0;  // the load's page half (one page per instruction)
+    const int phw = (TP == 16 && ok) ? ib / HD : 0;  // the load's page half (one page per instruction)
     const uint8_t* page = (q < NL8 ? k8_pool : v8_pool) + (phw ? boff1 : boff0);
     copy_to_lds16(page, ok ? src : 0u, lds_addr(ok ? (q < NL8 ? k_lds(buf) : v_lds(buf)) + ib * 8 : junk_lds));
   };
@@ -271,7 +296,7 @@ __device__ __forceinline__ void half_tile(const PrefillParams& p, int row0, int 
         u32x4 val = {0u, 0u, 0u, 0u};
         if (pg < p.num_pages && k0 + key < max_lim)
           val = *reinterpret_cast<const u32x4*>(k8_pool + static_cast<int64_t>(pg) * page_stride8 +
-                                                (c * TPP + key % TPP) * 16);
+                                                (c * TP + key % TP) * 16);
         *reinterpret_cast<u32x4*>(k_lds(buf) + i * 8) = val;
       }
       {
@@ -281,7 +306,7 @@ __device__ __forceinline__ void half_tile(const PrefillParams& p, int row0, int 
         u32x4 val = {0u, 0u, 0u, 0u};
         const int valid = max_lim - (k0 + kb);
         if (pg < p.num_pages && valid > 0) {
-          val = *reinterpret_cast<const u32x4*>(v8_pool + static_cast<int64_t>(pg) * page_stride8 + d * TPP + kb % TPP);
+          val = *reinterpret_cast<const u32x4*>(v8_pool + static_cast<int64_t>(pg) * page_stride8 + d * TP + kb % TP);
 #pragma unroll
           for (int e = 0; e < 4; ++e)
 #pragma unroll
@@ -293,17 +318,55 @@ __device__ __forceinline__ void half_tile(const PrefillParams& p, int row0, int 
     }
     __builtin_amdgcn_s_waitcnt(vmcnt_only(0));  // also where no load was executed
   };
-  // step j takes the fast path
+  // step j takes the fast path (fp8 pools only in window mode, as fp8 items;
+  // the 16-bit copies cannot dequantize)
   // (the tile's last step may end past max_lim: its copies then read keys
   // no row sees, from valid pages, and fix_tail clears their V entries)
   auto is_fast = [&](int j, uint32_t pg0, uint32_t pg1) {
     const int k0 = j * kKeys;
-    return k0 < max_lim && pg0 < np32 && pg1 < np32;
+    return TPP != 0 && (!KV8 || F8) && k0 < max_lim && pg0 < np32 && pg1 < np32 && (!PROMPT || k0 + kKeys <= hist);
+  };
+  // Prompt mode: a step whose 32 keys are all prompt keys below the tile's
+  // largest limit copies them from the dense prompt rows, as in prefill_tile.h
+  // (row offsets inside a step are 32 bits; longer rows take the register path).
+  const bool long_rows = PROMPT && dense_stride * 2 * kKeys > 0xFFFFFFFFll;
+  auto is_dense = [&](int j) {
+    const int k0 = j * kKeys;
+    return PROMPT && !long_rows && k0 >= hist && k0 < max_lim;
+  };
+  auto copy_dense = [&](int q, int buf, int j) {
+    const int jj = q % NL;
+    const int i = tid + jj * kPfThreads;
+    const int ib = w * kWave + jj * kPfThreads;
+    const bool ok = kAllItems || ib < NI;
+    const int64_t first = (dense_row0 + j * kKeys) * dense_stride + kvh * HD;  // key 0 of the step, this kv head
+    const int last = max_lim - 1 - j * kKeys;  // keys past it (tile's last step) read this key's row instead
+    if (q < NL) {  // K in its operand layout, as from pages
+      int c = 0, key = 0;
+      if (ok) IM::k_item(i, c, key);
+      const uint32_t src = 2u * static_cast<uint32_t>(min(key, last) * dense_stride + c * 8);
+      copy_to_lds16(p.k_dense + first, src, lds_addr(ok ? k_lds(buf) + ib * 8 : junk_lds));
+    } else {  // raw rows: slot i = (key, 8-dim chunk c ^ vd_swz(key))
+      const int key = ok ? i / (HD / 8) : 0, c = ok ? (i % (HD / 8)) ^ vd_swz<HD>(key) : 0;
+      const uint32_t src = 2u * static_cast<uint32_t>(min(key, last) * dense_stride + c * 8);
+      copy_to_lds16(p.v_dense + first, src, lds_addr(ok ? v_lds(buf) + ib * 8 : junk_lds));
+    }
+  };
+  // the page of item i, whose (first) key is tok: of the step's two pages, or
+  // with a run-time page size from the page table
+  auto page_of = [&](int i, int tok, uint32_t pg0, uint32_t pg1) {
+    if constexpr (TPP == 0) return tok < paged_keys ? pt[tok / tpp] : 0u;
+    else return IM::k_page_half(i) ? pg1 : pg0;
   };
   auto issue = [&](int j, uint32_t pg0, uint32_t pg1) {
     const int buf = j % kNBuf;
     const int k0 = j * kKeys;
-    if (TPP != 16) pg1 = pg0;
+    if (is_dense(j)) {
+#pragma unroll
+      for (int q = 0; q < 2 * NL; ++q) copy_dense(q, buf, j);
+      return;
+    }
+    if (TP != 16) pg1 = pg0;
     const bool fast = is_fast(j, pg0, pg1);
     if constexpr (F8) {
       if (fast) {
@@ -326,31 +389,73 @@ __device__ __forceinline__ void half_tile(const PrefillParams& p, int row0, int 
     for (int jj = 0; jj < NL; ++jj) {
       const int i = tid + jj * kPfThreads;
       if (i >= NI) continue;
-      const uint32_t pg = IM::k_page_half(i) ? pg1 : pg0;
-      const bool pg_ok = pg < p.num_pages;
-      PAL_DEBUG_FLAG(!pg_ok && k0 + (IM::k_page_half(i) ? 16 : 0) < max_lim, kDebugPageId);
       {  // K: stripe c, key kj of the step
         int kj, c;
         IM::k_item(i, c, kj);
+        const uint32_t pg = page_of(i, k0 + kj, pg0, pg1);
+        const bool pg_ok = pg < p.num_pages;
         u32x4 val = {0u, 0u, 0u, 0u};
-        if (pg_ok && k0 + kj < max_lim)
-          val = *reinterpret_cast<const u32x4*>(p.k_pool + static_cast<int64_t>(pg) * page_stride + kv_head_off +
-                                                IM::k_offset(i));
+        if (!PROMPT || k0 + kj < hist) {
+          if (pg_ok && k0 + kj < max_lim) {
+            if constexpr (KV8) {  // dims 8c..8c+7: half of 16-dim stripe c / 2, times the page's K scale
+              const uint8_t* kp8 = k8_pool + static_cast<int64_t>(pg) * page_stride8 + ((c >> 1) * TP + kj % TP) * 16 +
+                                   (c & 1) * 8;
+              val = fp8x8_scaled<DT>(*reinterpret_cast<const u32x2*>(kp8),
+                                     p.k_scales[static_cast<int64_t>(pg) * p.num_kv_heads + kvh]);
+            } else {
+              const int64_t off = TPP == 0 ? (static_cast<int64_t>(c) * tpp + (k0 + kj) % tpp) * 8 : IM::k_offset(i);
+              val = *reinterpret_cast<const u32x4*>(p.k_pool + static_cast<int64_t>(pg) * page_stride + kv_head_off + off);
+            }
+          }
+        } else if (k0 + kj < max_lim) {
+          val = *reinterpret_cast<const u32x4*>(p.k_dense + (dense_row0 + k0 + kj) * dense_stride + kvh * HD + c * 8);
+        }
         *reinterpret_cast<u32x4*>(k_lds(buf) + i * 8) = val;
       }
-      {  // V: row d, keys key .. key+7 of the step; those past the largest limit may hold anything
+      {  // V: row d, keys key .. key+7 of the step (they share a page: page sizes are multiples of 8)
         int d, key;
         IM::v_item(i, d, key);
+        const int tok = k0 + key;
+        const uint32_t pg = page_of(i, tok, pg0, pg1);
+        const bool pg_ok = pg < p.num_pages;
+        PAL_DEBUG_FLAG(!pg_ok && tok < paged_keys, kDebugPageId);
+        const int slot = TPP == 0 ? tok % tpp : key % TP;
+        const uint16_t* vrow = p.v_pool + static_cast<int64_t>(pg) * page_stride + kv_head_off +
+                               static_cast<int64_t>(d) * tpp + slot;
+        const uint8_t* vrow8 = v8_pool + static_cast<int64_t>(pg) * page_stride8 + d * TP + slot;
+        const float vsc = KV8 && pg_ok ? p.v_scales[static_cast<int64_t>(pg) * p.num_kv_heads + kvh] : 1.f;
         u32x4 val = {0u, 0u, 0u, 0u};
-        const int valid = max_lim - (k0 + key);
-        if (pg_ok && valid > 0) {
-          val = *reinterpret_cast<const u32x4*>(p.v_pool + static_cast<int64_t>(pg) * page_stride + kv_head_off + d * TPP +
-                                                key % TPP);
-          if (valid < 8) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-              val[e] &= (2 * e < valid ? 0x0000FFFFu : 0u) | (2 * e + 1 < valid ? 0xFFFF0000u : 0u);
+        if (!PROMPT || tok + 8 <= hist) {
+          if (pg_ok && tok < max_lim) {
+            if constexpr (KV8)
+              val = fp8x8_scaled<DT>(*reinterpret_cast<const u32x2*>(vrow8), vsc);
+            else
+              val = *reinterpret_cast<const u32x4*>(vrow);
           }
+        } else if (tok < max_lim) {  // some of the 8 keys are prompt tokens (dense, strided by row)
+          uint32_t e16[8];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const int t2 = tok + e;
+            const bool pgd = t2 < hist;
+            uint16_t x = 0;
+            if (t2 < max_lim && (!pgd || pg_ok)) {
+              if (!pgd)
+                x = p.v_dense[(dense_row0 + t2) * dense_stride + kvh * HD + d];
+              else if constexpr (KV8)
+                x = static_cast<uint16_t>(fp8x8_scaled<DT>(u32x2{vrow8[e], 0u}, vsc)[0] & 0xFFFFu);
+              else
+                x = vrow[e];
+            }
+            e16[e] = x;
+          }
+          val = {e16[0] | (e16[1] << 16), e16[2] | (e16[3] << 16), e16[4] | (e16[5] << 16), e16[6] | (e16[7] << 16)};
+        }
+        const int valid = max_lim - tok;  // keys past the largest limit may hold anything (NaN bits included)
+        if (valid < 8) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            val[e] &= (2 * e < valid ? 0x0000FFFFu : 0u) | (2 * e + 1 < valid ? 0xFFFF0000u : 0u);
         }
         *reinterpret_cast<u32x4*>(v_lds(buf) + i * 8) = val;
       }
@@ -358,8 +463,8 @@ __device__ __forceinline__ void half_tile(const PrefillParams& p, int row0, int 
     __builtin_amdgcn_s_waitcnt(vmcnt_only(0));  // also where no load was executed
   };
   // The tile's last step j, when it ends past max_lim and was copied: the
-  // keys no row sees hold whatever the pages held, and a masked probability of 0 times a NaN there
-  // would still be NaN, so their V entries are cleared.  Each thread clears
+  // keys no row sees hold whatever the pages (or, in prompt mode, the row of
+  // the last key) held, and a masked probability of 0 times a NaN there would still be NaN, so their V entries are cleared.  Each thread clears
   // its own items, after the barrier that saw the copies land and before the
   // barrier preceding the step's V reads (a slow step's entries are zero
   // already).
@@ -387,12 +492,15 @@ __device__ __forceinline__ void half_tile(const PrefillParams& p, int row0, int 
       }
       return;
     }
+    const bool dense = is_dense(j);
 #pragma unroll
     for (int jj = 0; jj < NL; ++jj) {
       const int i = tid + jj * kPfThreads;
       if (i >= NI) continue;
       u32x4* slot = reinterpret_cast<u32x4*>(vb + i * 8);
-      {  // operand layout: 8 keys key .. key+7 of row d
+      if (dense) {  // raw rows: slot i holds 8 dims of key i / (HD / 8)
+        if (i / (HD / 8) >= valid0) *slot = u32x4{0u, 0u, 0u, 0u};
+      } else {  // operand layout: 8 keys key .. key+7 of row d
         int d, key;
         IM::v_item(i, d, key);
         const int valid = valid0 - key;
@@ -413,9 +521,9 @@ __device__ __forceinline__ void half_tile(const PrefillParams& p, int row0, int 
   // step's keys past max_lim: their V bytes are cleared, and 0 x a stale
   // scale could be NaN)
   auto read_scales = [&](const float* arr, int j, float& s0, float& s1) {
-    const int e = j * kKeys / TPP;
+    const int e = j * kKeys / TP;
     s0 = e < n_pid ? arr[pid_slot(e)] : 0.f;
-    s1 = TPP == 16 ? (e + 1 < n_pid ? arr[pid_slot(e + 1)] : 0.f) : s0;
+    s1 = TP == 16 ? (e + 1 < n_pid ? arr[pid_slot(e + 1)] : 0.f) : s0;
   };
   // fp8: step j's scores times the K scale of each key's page (register r
   // holds key 16 (r / 8) + ..., so r < 8: the first page)
@@ -428,9 +536,9 @@ __device__ __forceinline__ void half_tile(const PrefillParams& p, int row0, int 
     }
   };
   auto read_pids = [&](int j) {
-    const int e = pid_slot(j * kKeys / TPP);
+    const int e = pid_slot(j * kKeys / TP);
     u32x2 v;
-    if (TPP == 16) {
+    if (TP == 16) {
       v = *reinterpret_cast<const u32x2*>(pid_lds + e);  // e is even: 8-byte aligned
     } else {
       v.x = pid_lds[e];
@@ -463,7 +571,7 @@ __device__ __forceinline__ void half_tile(const PrefillParams& p, int row0, int 
 #pragma unroll
       for (int j = 0; j < KS / 2; ++j) {
         const int c = 2 * j + half;
-        const int slot = TPP == 16 ? (key / 16) * HD + c * 16 + ((key % 16) ^ (key >= 16 ? 12 : 0)) : c * 32 + col;
+        const int slot = TP == 16 ? (key / 16) * HD + c * 16 + ((key % 16) ^ (key >= 16 ? 12 : 0)) : c * 32 + col;
         const u32x4 v = *reinterpret_cast<const u32x4*>(kb + slot * 16);
         // exact in 16 bits; the K scale goes on the scores
         ka[2 * j] = fp8x8_exact<DT>(u32x2{v.x, v.y});
@@ -576,8 +684,12 @@ __device__ __forceinline__ void half_tile(const PrefillParams& p, int row0, int 
   // the unmasked body.  The last step is always in the masked part, whose
   // mask also discards the scores of the stale buffer it reads as "next".
   const int n_main = max(0, min(nsteps, min_lim / kKeys - 1));
-  auto step = [&](auto masked, int st) {
+  // dense_v: step st's V rows were copied untransposed (a dense prompt step);
+  // each combination is its own loop body, so the operand reads carry no
+  // per-chunk branch.
+  auto step = [&](auto masked, auto dense_v, int st) {
     constexpr bool kMask = decltype(masked)::value;
+    constexpr bool vdense = decltype(dense_v)::value;
     wait_barrier(st + 2 < nsteps ? 1 : 0);  // step st+1 has landed
     const int j = st + kLeadHalf;
     const u32x2 pgv = read_pids(j);  // used after the MFMAs (in bounds whether or not step j exists)
@@ -611,7 +723,9 @@ __device__ __forceinline__ void half_tile(const PrefillParams& p, int row0, int 
 #pragma unroll
     for (int kk = 0; kk < KS; ++kk) {
       s_next = Dt<DT>::mma32x32x16(ka[kk], qv[kk], s_next);
-      if constexpr (F8) {
+      if constexpr (vdense) {
+        va[kk] = read_dense_v<HD>(v_lds(vbuf), kk / DT32, kk % DT32, col, half);
+      } else if constexpr (F8) {
         // chunk t < DT32 reads row tile t's item (half, d = col + 32 t): keys
         // 16 half .. +7 for k-step 0 (operand t), +8 .. +15 for k-step 1
         // (operand t + DT32).  Exact in 16 bits; the V scale is on P.  Each
@@ -661,8 +775,9 @@ __device__ __forceinline__ void half_tile(const PrefillParams& p, int row0, int 
     // memory pipeline (measured 3 % on config 4 against issuing them all
     // after the chunks); other steps take the synchronous path below.
     const uint32_t jp0 = __builtin_amdgcn_readfirstlane(pgv.x);
-    const uint32_t jp1 = TPP == 16 ? __builtin_amdgcn_readfirstlane(pgv.y) : jp0;
-    const bool jfast = j < nsteps && is_fast(j, jp0, jp1);
+    const uint32_t jp1 = TP == 16 ? __builtin_amdgcn_readfirstlane(pgv.y) : jp0;
+    const bool jdense = j < nsteps && (vdense || is_dense(j));  // steps after a dense one are dense
+    const bool jfast = j < nsteps && (jdense || is_fast(j, jp0, jp1));
     const int64_t joff0 = static_cast<int64_t>(jp0) * page_stride + kv_head_off;
     const int64_t joff1 = static_cast<int64_t>(jp1) * page_stride + kv_head_off;
 #pragma unroll
@@ -670,6 +785,8 @@ __device__ __forceinline__ void half_tile(const PrefillParams& p, int row0, int 
       if (jfast && m < 2 * NC) {
         if constexpr (F8)
           copy8(m, j % kNBuf, static_cast<int64_t>(jp0) * page_stride8, static_cast<int64_t>(jp1) * page_stride8);
+        else if (jdense)
+          copy_dense(m, j % kNBuf, j);
         else
           copy_one(m, j % kNBuf, joff0, joff1);
       }
@@ -685,13 +802,20 @@ __device__ __forceinline__ void half_tile(const PrefillParams& p, int row0, int 
     }
     __builtin_amdgcn_s_setprio(0);
     mb = update_max(bm);
-    if (const int chunk = pid_chunk_to_stage(st, TPP, n_pid)) stage_pids(chunk);
+    if (const int chunk = pid_chunk_to_stage(st, TP, n_pid)) stage_pids(chunk);
     if (j < nsteps && !jfast) issue(j, jp0, jp1);
     s_cur = s_next;
   };
+  // prompt mode: steps from ceil(hist / 32) on are dense (the one across the
+  // boundary, if any, is not)
+  const int fd = PROMPT && !long_rows ? min(nsteps, static_cast<int>((hist + kKeys - 1) / kKeys)) : nsteps;
   int st = 0;
-  for (; st < n_main; ++st) step(std::false_type{}, st);
-  for (; st < nsteps; ++st) step(std::true_type{}, st);
+  for (; st < min(n_main, fd); ++st) step(std::false_type{}, std::false_type{}, st);
+  if constexpr (PROMPT)
+    for (; st < n_main; ++st) step(std::false_type{}, std::true_type{}, st);
+  for (; st < fd; ++st) step(std::true_type{}, std::false_type{}, st);
+  if constexpr (PROMPT)
+    for (; st < nsteps; ++st) step(std::true_type{}, std::true_type{}, st);
 
   // ---- normalise and write: lane holds O[M-row col][32n + 8(r/4) + 4 half + r%4]
   float l;
@@ -736,10 +860,12 @@ __device__ __forceinline__ bool single_row(const uint32_t* q2seq, int64_t r, int
 }
 
 // The work of tile block b (a 1-D grid, XCD-aware): head group g = b % G (G =
-// kv heads x head chunks) and window b / G of `tokens per tile` rows, the last
-// window first; every run of rows of one sequence inside the window that is
-// not a lone decode row is computed as a tile.
-template <int DT, int HD, int TPP, bool KV8>
+// kv heads x head chunks) and work unit b / G, as in prefill_item.  Prompt
+// mode: unit = (sequence, tile), the last tile of a sequence first.  Window
+// mode: unit = window of `tokens per tile` rows, the last window first; every
+// run of rows of one sequence inside the window that is not a lone decode row
+// is computed as a tile.
+template <int DT, int HD, int TPP, bool KV8, bool kPromptMode>
 __device__ __forceinline__ void half_tile_block(const PrefillParams& p, unsigned block, HalfTileLds<HD, KV8>& L) {
   const int G = p.num_kv_heads * p.head_chunks;
   const int g = static_cast<int>(block % static_cast<unsigned>(G));
@@ -747,19 +873,28 @@ __device__ __forceinline__ void half_tile_block(const PrefillParams& p, unsigned
   const int kvh = g / p.head_chunks;
   const int h0 = (g % p.head_chunks) * 16;
   const int qt = kHalfRows / p.hg_max;
-  const int w0 = (p.num_units - 1 - unit) * qt;
-  const int w1 = static_cast<int>(min(static_cast<int64_t>(w0 + qt), p.num_rows));
-  const int tid = threadIdx.x;
-  if (tid < w1 - w0) L.run_start[tid] = (tid == 0 || p.q2seq[w0 + tid] != p.q2seq[w0 + tid - 1]) ? 1 : 0;
-  __syncthreads();
-  int cur = w0;
-  while (cur < w1) {
-    int end = cur + 1;
-    while (end < w1 && !L.run_start[end - w0]) ++end;
-    end = __builtin_amdgcn_readfirstlane(end);
-    if (end - cur > 1 || !single_row(p.q2seq, cur, p.num_rows))
-      half_tile<DT, HD, TPP, KV8>(p, cur, end - cur, p.q2seq[cur], kvh, h0, L.k, L.v, L.junk, L.pid, L.lim, L.scl);
-    cur = end;
+  if constexpr (kPromptMode) {
+    const int tps = (p.prompt_len + qt - 1) / qt;
+    const int s = unit / tps;
+    const int j = tps - 1 - (unit - s * tps);
+    half_tile<DT, HD, TPP, true, KV8>(p, s * p.prompt_len + j * qt, min(qt, p.prompt_len - j * qt), s, kvh, h0, L.k, L.v,
+                                      L.junk, L.pid, L.lim, L.scl);
+  } else {
+    const int w0 = (p.num_units - 1 - unit) * qt;
+    const int w1 = static_cast<int>(min(static_cast<int64_t>(w0 + qt), p.num_rows));
+    const int tid = threadIdx.x;
+    if (tid < w1 - w0) L.run_start[tid] = (tid == 0 || p.q2seq[w0 + tid] != p.q2seq[w0 + tid - 1]) ? 1 : 0;
+    __syncthreads();
+    int cur = w0;
+    while (cur < w1) {
+      int end = cur + 1;
+      while (end < w1 && !L.run_start[end - w0]) ++end;
+      end = __builtin_amdgcn_readfirstlane(end);
+      if (end - cur > 1 || !single_row(p.q2seq, cur, p.num_rows))
+        half_tile<DT, HD, TPP, false, KV8>(p, cur, end - cur, p.q2seq[cur], kvh, h0, L.k, L.v, L.junk, L.pid, L.lim,
+                                           L.scl);
+      cur = end;
+    }
   }
 }
 

@@ -27,10 +27,10 @@
 //    into four LDS buffers each, with counted waits and one barrier per step.
 //    Page ids come from an LDS copy of the tile's page-table slice.  Steps of
 //    dense prompt keys are copied the same way from the prompt rows (V rows
-//    untransposed, read back with transposing LDS reads); fp8 pages in window
-//    mode as fp8 bytes, converted in the operand reads.  Steps across the
-//    history / prompt boundary, with invalid page ids, or of fp8 pages in
-//    prompt mode take a synchronous register path.
+//    untransposed, read back with transposing LDS reads); fp8 pages (window
+//    mode) as fp8 bytes, converted in the operand reads.  Steps across the
+//    history / prompt boundary or with invalid page ids take a synchronous
+//    register path.
 //  * Each wavefront computes S^T = K * Q^T with v_mfma_f32_32x32x16 (A = K
 //    from LDS, B = Q^T held in registers) and O^T += V^T * P^T with the same
 //    instruction.  In the transposed products a lane owns one M-row, so the
@@ -64,7 +64,8 @@
 //
 // This header holds the device code of a tile (prefill_tile) so that both the
 // prefill kernel (prefill.hip) and the fused mixed-batch kernel (decode.hip)
-// compile it; a translation unit includes it after defining its debug-check
+// compile it (and prefill_half_tile.h the tiles that share a CU, for the calls
+// that those serve faster); a translation unit includes it after defining its debug-check
 // flag word (PAL_DEBUG_FLAGS_DEFINE).
 #pragma once
 
@@ -159,6 +160,31 @@ struct ItemMap {
   static constexpr int kVRowTile = TPP == 16 ? 64 : 128;
 };
 
+// Untransposed V rows (dense prompt steps), read back with transposing reads:
+// each 16-lane group reads 32 bytes of each of 4 consecutive keys, the other
+// group of its half-wavefront the next 32 bytes.  16-byte chunk c of key k is
+// stored at chunk c ^ vd_swz(k), which puts a 16-lane group on distinct banks in
+// a 32-bank pass and a half-wavefront on distinct banks in a 64-bank pass (HD
+// 96 rows are not swizzled).
+template <int HD>
+__device__ __forceinline__ int vd_swz(int key) {
+  const int r = key & 3;
+  return HD % 128 == 0 ? 4 * r + 2 * (r >> 1) : (HD == 64 ? 2 * r : (HD == 32 ? 2 * (r >> 1) : 0));
+}
+// The PV operand of k-step ks and row tile n from such rows.  Lane 4r + c of a
+// 16-lane group points at keys kg + 4t + r, dims d0 + 4c .. +3 (d0 = 32 n + (col
+// & 16)); the transposing read hands lane j dim d0 + j = col + 32 n of those 4 keys.
+template <int HD>
+__device__ __forceinline__ u32x4 read_dense_v(const uint16_t* rows, int ks, int n, int col, int half) {
+  const int l16 = static_cast<int>(threadIdx.x) & 15;
+  const int key = 16 * ks + 8 * half + (l16 >> 2);
+  const int d = 32 * n + (col & 16) + 4 * (l16 & 3);
+  const uint16_t* vr = rows + key * HD + (((d >> 3) ^ vd_swz<HD>(key)) << 3) + (d & 7);
+  const u32x2 lo = lds_read_tr16(vr);           // keys kg .. kg+3
+  const u32x2 hi = lds_read_tr16(vr + 4 * HD);  // keys kg+4 .. kg+7 (vd_swz(key + 4) = vd_swz(key))
+  return u32x4{lo[0], lo[1], hi[0], hi[1]};
+}
+
 // Next-item claims of the window mode.  Items 8 apart (workgroups of one XCD:
 // the same few kv heads) form a queue with a counter of its own; a workgroup
 // claims from the queue of its XCD and, when that is empty, from the others in
@@ -209,15 +235,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
                                              uint16_t* k_lds_base, uint16_t* v_lds_base, uint16_t* junk_lds,
                                              uint32_t* pid_lds, int* lim_lds, float* scl_lds, const int32_t* off_lds,
                                              Claim* claim) {
-  // TPP 0: the page size is p.tokens_per_page, known at run time (a
-  // multiple of 8; the reference prefill takes any, paged_attention_prefill.h.metal:
-  // 243-263).  Steps of history keys then take the register path, reading
-  // each key's page id from the page table; steps of dense prompt keys are
-  // copied as for the other page sizes.  LDS holds every step in the
-  // 32-key-page item order.
-  constexpr int TP = TPP == 0 ? 32 : TPP;  // page size of the LDS item order
-  const int tpp = TPP == 0 ? p.tokens_per_page : TPP;
-  static_assert(TPP != 0 || (PROMPT && !KV8), "run-time page sizes: uniform-prompt mode, 16-bit pools");
+  static_assert(!PROMPT || !KV8, "prompts over fp8 pages run on half tiles (prefill_choose_tiles)");
   static_assert(HD % 32 == 0, "prefill needs head_dim % 32 == 0");
   constexpr int kMRows = m_rows(RG);
   constexpr int KS = HD / 16;  // QK k-steps of 16
@@ -225,15 +243,15 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
   constexpr int NI = StepGeo<HD>::kItems;
   constexpr int NL = StepGeo<HD>::kLoads;
   constexpr int NCH = KS * RG;  // MFMAs (and chunks) of each product per step
-  using IM = ItemMap<HD, TP>;
+  using IM = ItemMap<HD, TPP>;
   // fp8 pools in window mode: steps are copied as fp8 bytes (16-byte items:
   // 16 dims of one key for K, 16 keys of one row for V; 2 HD items each, in
   // item order) and converted in the operand reads, each lane reading whole
   // items: a K item gives the 8 dims of two QK k-steps, a V item the 8 keys
   // of both PV k-steps (the keys of an fp8 step are in kperm_f8 order, the
   // query operand permuted to match).  A copy instruction must stay in one
-  // page: with TP 16 that needs HD % 64 == 0 (every fp8 pool's head dim).
-  constexpr bool F8 = KV8 && !PROMPT && (TP == 32 || HD % 64 == 0);
+  // page: with TPP 16 that needs HD % 64 == 0 (every fp8 pool's head dim).
+  constexpr bool F8 = KV8;
   constexpr int NI8 = 2 * HD;
   constexpr int NL8 = (NI8 + kPfThreads - 1) / kPfThreads;
   constexpr int NC = F8 ? NL8 : NL;  // copies per thread per step of K, and as many of V
@@ -258,7 +276,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
   const int col = lane & 31;  // this lane's M-row within a row group
   const int half = lane >> 5;
 
-  const int64_t max_tokens = p.page_table_width * tpp;
+  const int64_t max_tokens = p.page_table_width * TPP;
   int64_t hist = 0;  // prompt mode: keys below hist come from pages
   int64_t slen;
   if (prompt_mode) {
@@ -364,7 +382,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
 #pragma unroll
   for (int r = 0; r < RG; ++r) my_lim[r] = row_ok[r] ? lim_lds[my_t[r]] : 0;
 
-  const int64_t head_block = static_cast<int64_t>(HD) * tpp;
+  const int64_t head_block = static_cast<int64_t>(HD) * TPP;
   const int64_t page_stride = head_block * p.num_kv_heads;
   const int64_t page_stride8 = page_stride;            // fp8 pools: bytes per page (one byte per element)
   const int64_t kv_head_off8 = kvh * head_block;       // and of a kv head's block
@@ -375,7 +393,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
   // page-table entries the tile reads: keys below max_lim, and in prompt mode
   // only those below the history (the rest are dense) -- never past the width
   const int paged_keys = prompt_mode ? min(max_lim, static_cast<int>(hist)) : max_lim;
-  const int n_pid = TPP == 0 ? 0 : (paged_keys + TP - 1) / TP;  // runtime page size: no staged ids
+  const int n_pid = (paged_keys + TPP - 1) / TPP;
 
   // Page ids live in LDS (two chunks of 512 entries, entry e in slot e % 1024):
   // reading them is an LDS broadcast, so the only vector-memory traffic in the
@@ -405,10 +423,10 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
   // item, no registers, nothing to wait for here.  Every wavefront issues exactly
   // NC copies of K and NC of V (items past the step go to a junk slot), so the
   // wait counts are the same on every wavefront.
-  // Slow step (invalid pages, history / prompt boundary, fp8 in prompt mode): register loads,
+  // Slow step (invalid pages, history / prompt boundary): register loads,
   // masked, then LDS stores -- synchronous, and it drains the copies in
   // flight, which keeps the counted waits safe.
-  // pg0 / pg1: the pages of the step's first and (TP 16) second 16 keys.
+  // pg0 / pg1: the pages of the step's first and (TPP 16) second 16 keys.
   constexpr bool kAllItems = (F8 ? NI8 : NI) % kPfThreads == 0;  // no wavefront has a padding copy
   __builtin_assume(w >= 0 && w < kPfWaves);
   // The copies take a page's (a prompt row's) stride as 32 bits; longer ones go
@@ -418,11 +436,11 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
   // page ids >= 2^32 - 1 cannot occur with fewer pages; such an id takes the slow path
   const uint32_t np32 =
       long_pages ? 0u : (p.num_pages > 0xFFFFFFFFll ? 0xFFFFFFFFu : static_cast<uint32_t>(p.num_pages));
-  // fp8 items.  K item i: page half ph (TP 16), stripe c (dims 16c ..
-  // 16c+15), key of the step; V item i: page half ph (TP 16) or 16-key half
-  // of the page row (TP 32), row d.  Item i is LDS slot i.
+  // fp8 items.  K item i: page half ph (TPP 16), stripe c (dims 16c ..
+  // 16c+15), key of the step; V item i: page half ph (TPP 16) or 16-key half
+  // of the page row (TPP 32), row d.  Item i is LDS slot i.
   auto k8_item = [](int i, int& ph, int& c, int& key) {
-    if (TP == 16) {  // page-major; page 1's keys at positions XOR 12, so a 16-lane operand read spans all banks
+    if (TPP == 16) {  // page-major; page 1's keys at positions XOR 12, so a 16-lane operand read spans all banks
       ph = i / HD;
       c = (i % HD) / 16;
       key = 16 * ph + ((i % 16) ^ (ph ? 12 : 0));
@@ -433,7 +451,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
     }
   };
   auto v8_item = [](int i, int& ph, int& d, int& kb) {  // kb: the item's first key in the step
-    ph = TP == 16 ? i / HD : 0;
+    ph = TPP == 16 ? i / HD : 0;
     d = i % HD;
     kb = 16 * (i / HD);
   };
@@ -450,7 +468,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
     if constexpr (F8) {
       int ph, c, key;
       k8_item(i, ph, c, key);
-      return reinterpret_cast<uint64_t>(k8_pool) + static_cast<uint32_t>((c * TP + key % TP) * 16);
+      return reinterpret_cast<uint64_t>(k8_pool) + static_cast<uint32_t>((c * TPP + key % TPP) * 16);
     } else {
       return reinterpret_cast<uint64_t>(p.k_pool + kv_head_off) + 2u * static_cast<uint32_t>(IM::k_offset(i));
     }
@@ -460,44 +478,37 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
     if constexpr (F8) {
       int ph, d, kb;
       v8_item(i, ph, d, kb);
-      return reinterpret_cast<uint64_t>(v8_pool) + static_cast<uint32_t>(d * TP + kb % TP);
+      return reinterpret_cast<uint64_t>(v8_pool) + static_cast<uint32_t>(d * TPP + kb % TPP);
     } else {
       int d, key;
       IM::v_item(i, d, key);
-      return reinterpret_cast<uint64_t>(p.v_pool + kv_head_off) + 2u * static_cast<uint32_t>(d * TP + key % TP);
+      return reinterpret_cast<uint64_t>(p.v_pool + kv_head_off) + 2u * static_cast<uint32_t>(d * TPP + key % TPP);
     }
   };
-  uint64_t ksrc[TPP == 0 ? 1 : NC], vsrc[TPP == 0 ? 1 : NC];
-  if constexpr (TPP != 0) {
+  uint64_t ksrc[NC], vsrc[NC];
 #pragma unroll
-    for (int q = 0; q < NC; ++q) {
-      ksrc[q] = k_src(q);
-      vsrc[q] = v_src(q);
-    }
+  for (int q = 0; q < NC; ++q) {
+    ksrc[q] = k_src(q);
+    vsrc[q] = v_src(q);
   }
-  // the page half (TP 16) a wavefront's load q reads: one page per instruction
-  auto copy_half = [&](int q) { return F8 ? (TP == 16 ? wave_item(q) / HD : 0) : IM::k_page_half(wave_item(q)); };
+  // the page half (TPP 16) a wavefront's load q reads: one page per instruction
+  auto copy_half = [&](int q) { return F8 ? (TPP == 16 ? wave_item(q) / HD : 0) : IM::k_page_half(wave_item(q)); };
   auto copy_k = [&](int q, int j, uint32_t pg0, uint32_t pg1) {
-    if constexpr (TPP != 0) {
-      const bool ok = live_copy(q);
-      const uint32_t pg = ok && copy_half(q) ? pg1 : pg0;
-      copy_row_to_lds16(ksrc[q], pg, page_bytes, lds_addr(ok ? k_lds(j) + wave_item(q) * 8 : junk_lds));
-    }
+    const bool ok = live_copy(q);
+    const uint32_t pg = ok && copy_half(q) ? pg1 : pg0;
+    copy_row_to_lds16(ksrc[q], pg, page_bytes, lds_addr(ok ? k_lds(j) + wave_item(q) * 8 : junk_lds));
   };
   auto copy_v = [&](int q, int j, uint32_t pg0, uint32_t pg1) {
-    if constexpr (TPP != 0) {
-      const bool ok = live_copy(q);
-      const uint32_t pg = ok && copy_half(q) ? pg1 : pg0;
-      copy_row_to_lds16(vsrc[q], pg, page_bytes, lds_addr(ok ? v_lds(j) + wave_item(q) * 8 : junk_lds));
-    }
+    const bool ok = live_copy(q);
+    const uint32_t pg = ok && copy_half(q) ? pg1 : pg0;
+    copy_row_to_lds16(vsrc[q], pg, page_bytes, lds_addr(ok ? v_lds(j) + wave_item(q) * 8 : junk_lds));
   };
-  // step j takes the fast path (fp8 pools only in window mode, as fp8 items;
-  // the 16-bit copies cannot dequantize)
+  // step j takes the fast path
   // (the tile's last step may end past max_lim: its copies then read keys
   // no row sees, from valid pages, and fix_tail clears their V entries)
   auto is_fast = [&](int j, uint32_t pg0, uint32_t pg1) {
     const int k0 = j * kKeys;
-    return TPP != 0 && (!KV8 || F8) && k0 < max_lim && pg0 < np32 && pg1 < np32 && (!prompt_mode || k0 + kKeys <= hist);
+    return k0 < max_lim && pg0 < np32 && pg1 < np32 && (!prompt_mode || k0 + kKeys <= hist);
   };
   // Prompt mode: a step whose 32 keys are all prompt keys below the tile's
   // largest limit copies them from the dense prompt rows (16-bit in every
@@ -507,16 +518,6 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
   auto is_dense = [&](int j) {
     const int k0 = j * kKeys;
     return PROMPT && !long_rows && k0 >= hist && k0 < max_lim;
-  };
-  // Untransposed V rows, read back with transposing reads: each 16-lane
-  // group reads 32 bytes of each of 4 consecutive keys, the other group of
-  // its half-wavefront the next 32 bytes.  16-byte chunk c of key k is stored
-  // at chunk c ^ vd_swz(k), which puts a 16-lane group on distinct banks in a
-  // 32-bank pass and a half-wavefront on distinct banks in a 64-bank pass
-  // (HD 96 rows are not swizzled).
-  auto vd_swz = [](int key) {
-    const int r = key & 3;
-    return HD % 128 == 0 ? 4 * r + 2 * (r >> 1) : (HD == 64 ? 2 * r : (HD == 32 ? 2 * (r >> 1) : 0));
   };
   // the dense row of the step's key `key` (keys past max_lim repeat the last one's row)
   auto dense_row = [&](int j, int key) {
@@ -533,7 +534,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
   auto copy_dense_v = [&](int q, int j) {  // raw rows: slot i = (key, 8-dim chunk c ^ vd_swz(key))
     const bool ok = live_copy(q);
     const int i = item_of(q);
-    const int key = ok ? i / (HD / 8) : 0, c = ok ? (i % (HD / 8)) ^ vd_swz(key) : 0;
+    const int key = ok ? i / (HD / 8) : 0, c = ok ? (i % (HD / 8)) ^ vd_swz<HD>(key) : 0;
     const uint64_t src = reinterpret_cast<uint64_t>(p.v_dense + kvh * HD + c * 8);
     copy_row_to_lds16(src, dense_row(j, key), dense_bytes, lds_addr(ok ? v_lds(j) + wave_item(q) * 8 : junk_lds));
   };
@@ -554,7 +555,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
         u32x4 val = {0u, 0u, 0u, 0u};
         if (pg < p.num_pages && k0 + key < max_lim)
           val = *reinterpret_cast<const u32x4*>(k8_pool + static_cast<int64_t>(pg) * page_stride8 +
-                                                (c * TP + key % TP) * 16);
+                                                (c * TPP + key % TPP) * 16);
         *reinterpret_cast<u32x4*>(kb + i * 8) = val;
       }
     } else {
@@ -565,30 +566,14 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
         int kj, c;
         IM::k_item(i, c, kj);
         const int tok = k0 + kj;
-        // run-time page size: each key's page from the page table
-        const uint32_t pg = TPP == 0 ? (tok < max_lim && tok < hist ? pt[tok / tpp] : 0u)
-                                     : (IM::k_page_half(i) ? pg1 : pg0);
+        const uint32_t pg = IM::k_page_half(i) ? pg1 : pg0;
         const bool pg_ok = pg < p.num_pages;
-        if constexpr (TPP == 0) {
-          PAL_DEBUG_FLAG(!pg_ok, kDebugPageId);
-        } else {
-          PAL_DEBUG_FLAG(!pg_ok && k0 + (IM::k_page_half(i) ? 16 : 0) <
-                                       (prompt_mode ? min(max_lim, static_cast<int>(hist)) : max_lim),
-                         kDebugPageId);
-        }
+        PAL_DEBUG_FLAG(!pg_ok && k0 + (IM::k_page_half(i) ? 16 : 0) < paged_keys, kDebugPageId);
         u32x4 val = {0u, 0u, 0u, 0u};
         if (!prompt_mode || tok < hist) {
-          if (pg_ok && tok < max_lim) {
-            if constexpr (KV8) {  // dims 8c..8c+7: half of 16-dim stripe c / 2, times the page's K scale
-              const uint8_t* kp8 = reinterpret_cast<const uint8_t*>(p.k_pool) + static_cast<int64_t>(pg) * page_stride8 +
-                                   kv_head_off8 + ((c >> 1) * TP + kj % TP) * 16 + (c & 1) * 8;
-              val = fp8x8_scaled<DT>(*reinterpret_cast<const u32x2*>(kp8),
-                                     p.k_scales[static_cast<int64_t>(pg) * p.num_kv_heads + kvh]);
-            } else {
-              const int64_t off = TPP == 0 ? (static_cast<int64_t>(c) * tpp + tok % tpp) * 8 : IM::k_offset(i);
-              val = *reinterpret_cast<const u32x4*>(p.k_pool + static_cast<int64_t>(pg) * page_stride + kv_head_off + off);
-            }
-          }
+          if (pg_ok && tok < max_lim)
+            val = *reinterpret_cast<const u32x4*>(p.k_pool + static_cast<int64_t>(pg) * page_stride + kv_head_off +
+                                                  IM::k_offset(i));
         } else if (tok < max_lim) {
           val = *reinterpret_cast<const u32x4*>(p.k_dense + (dense_row0 + tok) * dense_stride + kvh * HD + c * 8);
         }
@@ -611,7 +596,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
         u32x4 val = {0u, 0u, 0u, 0u};
         const int valid = max_lim - (k0 + kb);
         if (pg < p.num_pages && valid > 0) {
-          val = *reinterpret_cast<const u32x4*>(v8_pool + static_cast<int64_t>(pg) * page_stride8 + d * TP + kb % TP);
+          val = *reinterpret_cast<const u32x4*>(v8_pool + static_cast<int64_t>(pg) * page_stride8 + d * TPP + kb % TPP);
 #pragma unroll
           for (int e = 0; e < 4; ++e)
 #pragma unroll
@@ -625,27 +610,16 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
       for (int jj = 0; jj < NL; ++jj) {
         const int i = item_of(jj);
         if (i >= NI) continue;
-        // row d, keys key .. key+7 of the step (they share a page: page sizes are multiples of 8)
+        // row d, keys key .. key+7 of the step (they share a page)
         int d, key;
         IM::v_item(i, d, key);
         const int tok = k0 + key;
-        const uint32_t pg = TPP == 0 ? (tok < max_lim && tok < hist ? pt[tok / tpp] : 0u)
-                                     : (IM::k_page_half(i) ? pg1 : pg0);
+        const uint32_t pg = IM::k_page_half(i) ? pg1 : pg0;
         const bool pg_ok = pg < p.num_pages;
-        const int slot = TPP == 0 ? tok % tpp : key % TP;
-        const uint16_t* vrow = p.v_pool + static_cast<int64_t>(pg) * page_stride + kv_head_off +
-                               static_cast<int64_t>(d) * tpp + slot;
-        const uint8_t* vrow8 = reinterpret_cast<const uint8_t*>(p.v_pool) + static_cast<int64_t>(pg) * page_stride8 +
-                               kv_head_off8 + d * TP + slot;
-        const float vsc = KV8 && pg_ok ? p.v_scales[static_cast<int64_t>(pg) * p.num_kv_heads + kvh] : 1.f;
+        const uint16_t* vrow = p.v_pool + static_cast<int64_t>(pg) * page_stride + kv_head_off + d * TPP + key % TPP;
         u32x4 val = {0u, 0u, 0u, 0u};
         if (!prompt_mode || tok + 8 <= hist) {
-          if (pg_ok && tok < max_lim) {
-            if constexpr (KV8)
-              val = fp8x8_scaled<DT>(*reinterpret_cast<const u32x2*>(vrow8), vsc);
-            else
-              val = *reinterpret_cast<const u32x4*>(vrow);
-          }
+          if (pg_ok && tok < max_lim) val = *reinterpret_cast<const u32x4*>(vrow);
         } else if (tok < max_lim) {
           // some of the 8 keys are prompt tokens (dense, strided by row)
           uint32_t e16[8];
@@ -654,15 +628,8 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
             const int t2 = tok + e;
             const bool pgd = t2 < hist;
             uint16_t x = 0;
-            if (t2 < max_lim && (!pgd || pg_ok)) {
-              if (!pgd) {
-                x = p.v_dense[(dense_row0 + t2) * dense_stride + kvh * HD + d];
-              } else if constexpr (KV8) {
-                x = static_cast<uint16_t>(fp8x8_scaled<DT>(u32x2{vrow8[e], 0u}, vsc)[0] & 0xFFFFu);
-              } else {
-                x = vrow[e];
-              }
-            }
+            if (t2 < max_lim && (!pgd || pg_ok))
+              x = pgd ? vrow[e] : p.v_dense[(dense_row0 + t2) * dense_stride + kvh * HD + d];
             e16[e] = x;
           }
           val = {e16[0] | (e16[1] << 16), e16[2] | (e16[3] << 16), e16[4] | (e16[5] << 16), e16[6] | (e16[7] << 16)};
@@ -759,21 +726,21 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
     }
   };
   const bool tail_partial = max_lim % kKeys != 0;  // the last step ends past max_lim
-  // fp8: the scales of step j's first and (TP 16) second page (LDS
+  // fp8: the scales of step j's first and (TPP 16) second page (LDS
   // broadcast); 0 for a page past the tile's last staged entry (the tail
   // step's keys past max_lim: their V bytes are cleared, and 0 x a stale
   // scale could be NaN)
   auto read_scales = [&](const float* arr, int j, float& s0, float& s1) {
-    const int e = j * (kKeys / TP);  // (even with TP 16)
-    const float a0 = arr[pid_slot(e)], a1 = arr[pid_slot(e + (TP == 16))];
+    const int e = j * (kKeys / TPP);  // (even with TPP 16)
+    const float a0 = arr[pid_slot(e)], a1 = arr[pid_slot(e + (TPP == 16))];
     s0 = e < n_pid ? a0 : 0.f;
-    s1 = TP == 16 ? (e + 1 < n_pid ? a1 : 0.f) : s0;
+    s1 = TPP == 16 ? (e + 1 < n_pid ? a1 : 0.f) : s0;
   };
-  // the page ids of step j (an LDS broadcast read; TP 32: one page)
+  // the page ids of step j (an LDS broadcast read; TPP 32: one page)
   auto read_pids = [&](int j) {
-    const int e = pid_slot(j * (kKeys / TP));
+    const int e = pid_slot(j * (kKeys / TPP));
     u32x2 v;
-    if (TP == 16) {
+    if (TPP == 16) {
       v = *reinterpret_cast<const u32x2*>(pid_lds + e);  // e is even: 8-byte aligned
     } else {
       v.x = pid_lds[e];
@@ -816,7 +783,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
   auto read_k8 = [&](int j, int kj) {
     const int key = kperm_f8(col);
     const int c = 2 * kj + half;
-    const int slot = TP == 16 ? (key / 16) * HD + c * 16 + ((key % 16) ^ (key >= 16 ? 12 : 0)) : c * 32 + col;
+    const int slot = TPP == 16 ? (key / 16) * HD + c * 16 + ((key % 16) ^ (key >= 16 ? 12 : 0)) : c * 32 + col;
     return *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint8_t*>(k_lds(j)) + slot * 16);
   };
   // V^T operand bases: k-step kk takes keys 16kk + 8 half .. +7; row tile n
@@ -929,12 +896,12 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
     for (int kk = 0; kk < (F8 ? KS / 2 : KS); ++kk) ka[kk] = F8 ? read_k8(j, kk) : read_k(j, kk);
   };
   // whole steps in pages that the copies can read
-  const int paged_full = (TPP != 0 && (!KV8 || F8)) && !long_pages ? paged_keys / kKeys : 0;
+  const int paged_full = !long_pages ? paged_keys / kKeys : 0;
   if (nsteps > 0) {
     auto pids = [&](int j, uint32_t& a, uint32_t& b) {
       const u32x2 v = read_pids(j);
       a = __builtin_amdgcn_readfirstlane(v.x);
-      b = TP == 16 ? __builtin_amdgcn_readfirstlane(v.y) : a;
+      b = TPP == 16 ? __builtin_amdgcn_readfirstlane(v.y) : a;
     };
     // K 0, K 1, V 0, K 2, V 1, K 3, V 2
     if (paged_full >= 4 && __builtin_amdgcn_readfirstlane(lim_lds[kBad]) == 0) {
@@ -1029,7 +996,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
     sched_fence();
     float vs0 = 1.f, vs1 = 1.f;  // fp8: V scales of step st's pages
     if constexpr (F8) read_scales(vs_lds, st, vs0, vs1);
-    const float svs = half ? vs1 : vs0;  // the lane's keys 16 half .. +15: page half (TP 32: vs1 == vs0)
+    const float svs = half ? vs1 : vs0;  // the lane's keys 16 half .. +15: page half (TPP 32: vs1 == vs0)
     f32x16 s_next[RG];
 #pragma unroll
     for (int r = 0; r < RG; ++r)
@@ -1077,17 +1044,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
       }
       if (c % RG == 0) {
         if constexpr (vdense) {
-          // raw rows: V[key][d] in chunk (d / 8) ^ vd_swz(key) of row key.  Lane
-          // 4r + c of a 16-lane group points at keys kg + 4t + r, dims d0 + 4c ..
-          // +3 (d0 = 32 (kk % DT32) + (col & 16)); the transposing read hands
-          // lane j dim d0 + j = col + 32 (kk % DT32) of those 4 keys.
-          const int l16 = lane & 15;
-          const int key = 16 * (kk / DT32) + 8 * half + (l16 >> 2);
-          const int d = 32 * (kk % DT32) + (col & 16) + 4 * (l16 & 3);
-          const uint16_t* vr = v_lds(st) + key * HD + (((d >> 3) ^ vd_swz(key)) << 3) + (d & 7);
-          const u32x2 lo = lds_read_tr16(vr);           // keys kg .. kg+3
-          const u32x2 hi = lds_read_tr16(vr + 4 * HD);  // keys kg+4 .. kg+7 (vd_swz(key + 4) = vd_swz(key))
-          va[kk] = u32x4{lo[0], lo[1], hi[0], hi[1]};
+          va[kk] = read_dense_v<HD>(v_lds(st), kk / DT32, kk % DT32, col, half);
         } else if constexpr (F8) {
           // chunk t < DT32 reads row tile t's item (half, d = col + 32 t): keys
           // 16 half .. +7 for k-step 0 (operand t), +8 .. +15 for k-step 1
@@ -1133,9 +1090,9 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
     uint32_t kp0 = 0, kp1 = 0, vp0 = 0, vp1 = 0;
     if (kMode == kAny && jv < nsteps) {
       kp0 = __builtin_amdgcn_readfirstlane(pgk.x);
-      kp1 = TP == 16 ? __builtin_amdgcn_readfirstlane(pgk.y) : kp0;
+      kp1 = TPP == 16 ? __builtin_amdgcn_readfirstlane(pgk.y) : kp0;
       vp0 = __builtin_amdgcn_readfirstlane(pgv.x);
-      vp1 = TP == 16 ? __builtin_amdgcn_readfirstlane(pgv.y) : vp0;
+      vp1 = TPP == 16 ? __builtin_amdgcn_readfirstlane(pgv.y) : vp0;
       kdn = jk < nsteps && (vdense || is_dense(jk));  // steps after a dense one are dense
       vdn = jv < nsteps && (vdense || is_dense(jv));
       kfast = jk < nsteps && (kdn || is_fast(jk, kp0, kp1));
@@ -1232,7 +1189,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
         acc_settle();
       }
       if constexpr (kMode == kAny) {
-        if (const int chunk = pid_chunk_to_stage(st, TP, n_pid)) stage_pids(chunk);
+        if (const int chunk = pid_chunk_to_stage(st, TPP, n_pid)) stage_pids(chunk);
         if (jv < nsteps) {
           if (jk < nsteps && !kfast) slow_k(jk, kp0, kp1);
           if (!vfast) slow_v(jv, vp0, vp1);
@@ -1256,7 +1213,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
   int st = 0;
   int staged_at = -2;  // the iteration that staged page ids last (its flag is read two iterations later)
   while (st < min(nsteps - 1, fd)) {
-    const int chunk_st = pid_next_staging(st, TP);
+    const int chunk_st = pid_next_staging(st, TPP);
     const int fast_end = min(min(n_main, paged_full - kLeadK), chunk_st);
     if (st < fast_end && st >= staged_at + 2 && __builtin_amdgcn_readfirstlane(lim_lds[kBad]) == 0) {
       for (; st < fast_end; ++st) step(Fast{}, no, st);

@@ -169,12 +169,14 @@ def test_prefill_query_magnitudes(dtype):
 
 @pytest.mark.parametrize("hd,tpp,dtype", [(32, 16, "bf16"), (64, 16, "f16"), (96, 8, "bf16"), (128, 16, "bf16"),
                                           (128, 32, "f16"), (256, 32, "bf16")])
-@pytest.mark.parametrize("plen", [190, 259, 520])
+@pytest.mark.parametrize("plen", [190, 240, 259, 330, 520, 1000])
 def test_prefill_tile_rounds(plen, hd, tpp, dtype):
-    """More tiles than CUs: with 64 query heads on 16 kv heads 190 rows make
+    """More tiles than CUs (256): with 64 query heads on 16 kv heads 190 rows make
     288 tiles of one row group (32 rows) or 144 of two, 259 rows 432 / 240 with
-    three rows in the last one, 520 rows 816 / 432, two rounds of the larger
-    tiles (head dims above 128 have the smaller ones only)."""
+    three rows in the last one, 520 rows 816 / 432, two rounds: two groups up to head
+    dim 64, half tiles above.  240 and 1,000 rows make tiles of two groups that are
+    alike (192, and 768 in three rounds): head dims 96 and 128 (16-token pages)
+    have them too.  330 rows make 528 / 288: half tiles."""
     _check(hd + plen, [0, 33, 150], plen, 64, 16, hd, tpp, dtype, "tile rounds")
 
 
