@@ -280,11 +280,12 @@ size_t pal_paged_attention_workspace_size(int dtype, int64_t num_query_rows, int
  * p + 1.  Rows with no visible token, or naming no sequence (s >= num_seqs),
  * yield zeros.  out: [num_query_rows, num_q_heads, head_dim].  Runs of
  * consecutive rows of one sequence go to MFMA prefill tiles, single rows to
- * split-K decode workers, in one kernel whose first workgroups are the decode
- * workers (head dims up to 128; above, the decode and prefill kernels run one
- * after the other), followed by the merge kernel; the decode workers find
- * and schedule the single rows on the device, so the call never reads row
- * metadata on the host.  The workspace (size
+ * split-K decode workers.  Head dims up to 128: one kernel, in which decode
+ * workgroups run beside the tiles or, where the batch is mostly prefill rows,
+ * each workgroup streams decode rows first and takes tiles then; above 128 the
+ * tiles' kernel, then the decode kernel.  The merge kernel follows.  The decode
+ * workers find and schedule the single rows on the device, so the call never
+ * reads row metadata on the host.  The workspace (size
  * from pal_paged_attention_workspace_size, 256-byte aligned, zero-filled
  * before its first use) must not be shared by concurrent calls.
  */

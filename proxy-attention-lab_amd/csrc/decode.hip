@@ -889,7 +889,7 @@ __device__ __forceinline__ void fused_claim_rows(const DecodeParams& p, FusedDec
   for (;;) {
     uint32_t k = 0;
     if (lane == 0) k = atomicAdd(p.claim, 1u);
-    const int64_t batch = static_cast<int64_t>(__builtin_amdgcn_readfirstlane(k) & (kClaimsTaken - 1)) * kWave;
+    const int64_t batch = static_cast<int64_t>(__builtin_amdgcn_readfirstlane(k) & (kTilesOnly - 1)) * kWave;
     if (batch >= n_rows) break;
     const int64_t r = batch + lane;
     int32_t len = 0;
@@ -929,6 +929,46 @@ __device__ __forceinline__ void fused_claim_rows(const DecodeParams& p, FusedDec
   }
 }
 
+// Is any row alone in its run (the same in every workgroup)?  Lane t of a pass
+// reads rows 4t .. 4t+3 as one 16-byte load (when the map is 16-byte aligned)
+// and their two neighbours.
+__device__ __forceinline__ bool any_lone_row(const DecodeParams& p) {
+  const int tid = threadIdx.x;
+  const int64_t n_rows = p.num_seqs;
+  bool any = false;
+  const bool vec = (reinterpret_cast<uintptr_t>(p.q2seq) & 15u) == 0;
+  constexpr int kPasses = 4;  // passes whose loads are in flight together
+  for (int64_t base = 0; base < n_rows; base += kPasses * 4 * kGroupThreads) {
+    uint32_t q[kPasses][6];
+#pragma unroll
+    for (int u = 0; u < kPasses; ++u) {
+      const int64_t r0 = base + 4 * (static_cast<int64_t>(u) * kGroupThreads + tid);
+      q[u][0] = r0 > 0 && r0 <= n_rows ? p.q2seq[r0 - 1] : 0xFFFFFFFFu;
+      if (vec && r0 + 4 <= n_rows) {
+        const u32x4 v = *reinterpret_cast<const u32x4*>(p.q2seq + r0);
+        q[u][1] = v.x;
+        q[u][2] = v.y;
+        q[u][3] = v.z;
+        q[u][4] = v.w;
+      } else {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) q[u][1 + k] = r0 + k < n_rows ? p.q2seq[r0 + k] : 0xFFFFFFFFu;
+      }
+      q[u][5] = r0 + 4 < n_rows ? p.q2seq[r0 + 4] : 0xFFFFFFFFu;
+    }
+#pragma unroll
+    for (int u = 0; u < kPasses; ++u) {
+      const int64_t r0 = base + 4 * (static_cast<int64_t>(u) * kGroupThreads + tid);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int64_t r = r0 + k;
+        if (r < n_rows && (r == 0 || q[u][k] != q[u][k + 1]) && (r + 1 == n_rows || q[u][k + 2] != q[u][k + 1])) any = true;
+      }
+    }
+  }
+  return __syncthreads_or(any);
+}
+
 template <int DT, int HD, int TPP, int PF, bool KV8>
 __device__ __forceinline__ void fused_decode_body(const DecodeParams& p, FusedDecodeLds& L) {
   const int tid = threadIdx.x;
@@ -950,45 +990,9 @@ __device__ __forceinline__ void fused_decode_body(const DecodeParams& p, FusedDe
     return len > 0;
   };
 
-  // Quick pass: is any row alone in its run?  Lane t of a pass reads rows
-  // 4t .. 4t+3 as one 16-byte load (when the map is 16-byte aligned) and
-  // their two neighbours; a batch with none (a prefill-only batch) ends here.
-  {
-    bool any = false;
-    const bool vec = (reinterpret_cast<uintptr_t>(p.q2seq) & 15u) == 0;
-    constexpr int kPasses = 4;  // passes whose loads are in flight together
-    for (int64_t base = 0; base < n_rows; base += kPasses * 4 * kGroupThreads) {
-      uint32_t q[kPasses][6];
-#pragma unroll
-      for (int u = 0; u < kPasses; ++u) {
-        const int64_t r0 = base + 4 * (static_cast<int64_t>(u) * kGroupThreads + tid);
-        q[u][0] = r0 > 0 && r0 <= n_rows ? p.q2seq[r0 - 1] : 0xFFFFFFFFu;
-        if (vec && r0 + 4 <= n_rows) {
-          const u32x4 v = *reinterpret_cast<const u32x4*>(p.q2seq + r0);
-          q[u][1] = v.x;
-          q[u][2] = v.y;
-          q[u][3] = v.z;
-          q[u][4] = v.w;
-        } else {
-#pragma unroll
-          for (int k = 0; k < 4; ++k) q[u][1 + k] = r0 + k < n_rows ? p.q2seq[r0 + k] : 0xFFFFFFFFu;
-        }
-        q[u][5] = r0 + 4 < n_rows ? p.q2seq[r0 + 4] : 0xFFFFFFFFu;
-      }
-#pragma unroll
-      for (int u = 0; u < kPasses; ++u) {
-        const int64_t r0 = base + 4 * (static_cast<int64_t>(u) * kGroupThreads + tid);
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const int64_t r = r0 + k;
-          if (r < n_rows && (r == 0 || q[u][k] != q[u][k + 1]) && (r + 1 == n_rows || q[u][k + 2] != q[u][k + 1])) any = true;
-        }
-      }
-    }
-    if (!__syncthreads_or(any)) {
-      if (blockIdx.x == 0 && tid == 0) p.hdr[0] = 0;  // nothing to merge
-      return;
-    }
+  if (!any_lone_row(p)) {  // a batch of prefill rows only
+    if (blockIdx.x == 0 && tid == 0) p.hdr[0] = 0;  // nothing to merge
+    return;
   }
 
   int64_t n_lone = 0, n_blocks = 0;  // running totals (uniform)
@@ -1051,7 +1055,7 @@ __device__ __forceinline__ void fused_decode_body(const DecodeParams& p, FusedDe
   fused_claim_rows<DT, HD, TPP, PF, KV8>(p, L, lone_row);
 }
 
-// The fused mixed batch in one launch (head dims up to 128), in two forms.
+// The fused mixed batch (head dims up to 128), in two forms.
 //
 // Side by side (fused_kernel): blocks [0, n_dec) are the decode workers of the
 // lone rows (one workgroup per CU, equal static shares of the rows' KV blocks,
@@ -1064,18 +1068,27 @@ __device__ __forceinline__ void fused_decode_body(const DecodeParams& p, FusedDe
 // started late would end late), and the tiles take the other slot, then both
 // once the decode workers are done.  The two roles share one LDS allocation.
 //
-// One after the other (fused_wide_kernel): one resident workgroup per CU first
-// streams its share of the lone rows, then takes tiles that have the whole
-// register file (prefill_tile.h).  Those tiles are 1.25 to 1.5 times as fast,
-// which wins where the decode rows are a small part of the work (fused_wide).
+// Tiles with a CU to themselves (fused_wide_kernel): one resident workgroup per
+// CU first streams its share of the lone rows, then takes tiles that have the
+// whole register file (prefill_tile.h).  Those tiles are 1.1 to 1.6 times as
+// fast, but the stream and its set-up then overlap nothing: with even one lone
+// row the form measured 1.0 to 1.5 times as slow as side by side in most of 170
+// mixed batches (head dims 64 and 128, groups 1 to 8, 1 to 16 decode rows of
+// 4,096 to 131,072 keys beside 1,024 to 4,096 prefill rows).  Only the device sees whether
+// there are lone rows, so where there may be (fused_wide_sure) both kernels are
+// launched: this one, deciding, does nothing if it finds a lone row; otherwise
+// it computes every tile and sets kTilesOnly in the claim word, and the
+// side-by-side kernel behind it ends at once.
 static_assert(kPfThreads == kGroupThreads, "decode workers and prefill tiles share the workgroup shape");
 template <int DT, int HD, int TPP, bool KV8>
 __global__ __launch_bounds__(kGroupThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void fused_kernel(const DecodeParams dp, const PrefillParams pp, const unsigned n_dec) {
+void fused_kernel(const DecodeParams dp, const PrefillParams pp, const unsigned n_dec, const bool decided) {
   __shared__ union {
     FusedDecodeLds d;
     HalfTileLds<HD, KV8> f;
   } lds;
+  // (only fused_wide_kernel, which has ended, sets the bit)
+  if (decided && (__hip_atomic_load(dp.claim, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & kTilesOnly)) return;
   if (blockIdx.x < n_dec)
     fused_decode_body<DT, HD, TPP, shared_cu_prefetch<HD>(), KV8>(dp, lds.d);
   else
@@ -1084,13 +1097,21 @@ void fused_kernel(const DecodeParams dp, const PrefillParams pp, const unsigned 
 
 template <int DT, int HD, int TPP, bool KV8, int RG>
 __global__ __launch_bounds__(kGroupThreads) PAL_ACC_KERNEL
-void fused_wide_kernel(const DecodeParams dp, const PrefillParams pp) {
+void fused_wide_kernel(const DecodeParams dp, const PrefillParams pp, const bool deciding) {
   __shared__ union {
     FusedDecodeLds d;
     PrefillLds<HD, KV8, RG> f;
   } lds;
-  fused_decode_body<DT, HD, TPP, kPrefetch, KV8>(dp, lds.d);
-  __syncthreads();  // the workgroup's decode wavefronts are done with their lists
+  if (deciding) {
+    if (any_lone_row(dp)) return;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      dp.hdr[0] = 0;  // nothing to merge
+      __hip_atomic_fetch_or(dp.claim, kTilesOnly, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  } else {
+    fused_decode_body<DT, HD, TPP, kPrefetch, KV8>(dp, lds.d);
+    __syncthreads();  // the workgroup's decode wavefronts are done with their lists
+  }
   prefill_items<DT, HD, TPP, KV8, RG, false>(pp, blockIdx.x, gridDim.x, lds.f);
 }
 
@@ -1523,42 +1544,46 @@ hipError_t dispatch_hd(const DecodeParams& p, int hd, int tpp, bool kv8, hipStre
   }
 }
 
-// One after the other instead of side by side?  The stream of the lone rows
-// then overlaps nothing, which the faster tiles pay for only if the batch is
-// mostly prefill: many (row, head) products per sequence whose keys may be
-// streamed.  Measured side by side -> one after the other, by rows * group /
-// num_seqs (head dim 128, 8 kv heads): 5,000 (16 sequences, 20,000 rows) 0.70 ->
-// 0.61 ms; 1,370 (8 decode rows, 4 chunks of 1,024) 238 -> 210 us; 1,030 (7 decode
-// rows of 30,000 keys, one chunk of 2,048) 221 -> 228 us; 820 (4 decode rows, one
-// chunk of 1,024) 69 -> 88 us; 134 (256 decode rows, 4 chunks) 0.94 -> 1.04 ms.
+// Do tiles with a CU to themselves come into question: is the batch large
+// enough, and has it prefill rows mostly?  Measured over batches of chunks alone,
+// side by side -> these, by rows * group / num_seqs: 5,120 (8 chunks of 1,280 on
+// 1,024 cached, 32 query heads on 8 kv heads, head dim 128) 331 -> 298 us; 2,048
+// (4 of 512 on 8,192) 307 -> 265 us; 1,024 (16 of 256 on 1,024) 109 -> 114 us; 256
+// (16 of 64) 21.2 -> 21.4 us.
 inline bool fused_wide(const PrefillParams& p) { return p.num_rows * p.group >= 1200 * p.num_seqs; }
+// With one sequence there are no lone rows beside the tiles (but rows that name
+// no sequence, whose zeros cost nothing).
+inline bool fused_wide_sure(const PrefillParams& p) { return p.num_seqs <= 1; }
 
-// The fused op: the fused kernel, then the merge; head dims above 128: the
-// prefill tiles, then the decode rows' kernels.
+// The fused op: one of the fused kernels (or both, see there), then the merge;
+// head dims above 128: the prefill tiles, then the decode rows' kernels.
 template <int DT, int HD, int TPP, bool KV8>
-hipError_t launch_fused_t(const DecodeParams& dp, PrefillParams pp, hipStream_t stream) {
+hipError_t launch_fused_t(const DecodeParams& dp, const PrefillParams& pp, hipStream_t stream) {
   if constexpr (shares_cu(HD)) {
     const int64_t n_dec = (static_cast<int64_t>(dp.num_workers) + kWorkersPerGroup - 1) / kWorkersPerGroup;
     const dim3 threads(kGroupThreads);
     const int64_t n_pf = static_cast<int64_t>(pp.num_units) * pp.num_kv_heads * pp.head_chunks;
     if (n_dec + n_pf > 0x7FFFFFFFll) return hipErrorInvalidValue;
-    const bool wide = fused_wide(pp);
+    const bool wide = fused_wide(pp), sure = wide && fused_wide_sure(pp);
+    hipError_t err = hipSuccess;
     if (wide) {
-      const hipError_t err = prefill_choose_tiles(pp, HD);
+      PrefillParams wp = pp;
+      err = prefill_choose_tiles(wp, HD);
+      if (err != hipSuccess) return err;
+      const dim3 grid(static_cast<unsigned>(n_dec));
+      if (wp.row_groups == 1)
+        hipLaunchKernelGGL((fused_wide_kernel<DT, HD, TPP, KV8, 1>), grid, threads, 0, stream, dp, wp, !sure);
+      else
+        hipLaunchKernelGGL((fused_wide_kernel<DT, HD, TPP, KV8, 2>), grid, threads, 0, stream, dp, wp, !sure);
+      err = hipGetLastError();
       if (err != hipSuccess) return err;
     }
-    if (!wide) {
+    if (!sure) {
       hipLaunchKernelGGL((fused_kernel<DT, HD, TPP, KV8>), dim3(static_cast<unsigned>(n_dec + n_pf)), threads, 0, stream,
-                         dp, pp, static_cast<unsigned>(n_dec));
-    } else if (pp.row_groups == 1) {
-      hipLaunchKernelGGL((fused_wide_kernel<DT, HD, TPP, KV8, 1>), dim3(static_cast<unsigned>(n_dec)), threads, 0, stream,
-                         dp, pp);
-    } else {
-      hipLaunchKernelGGL((fused_wide_kernel<DT, HD, TPP, KV8, 2>), dim3(static_cast<unsigned>(n_dec)), threads, 0, stream,
-                         dp, pp);
+                         dp, pp, static_cast<unsigned>(n_dec), wide);
+      err = hipGetLastError();
+      if (err != hipSuccess) return err;
     }
-    const hipError_t err = hipGetLastError();
-    if (err != hipSuccess) return err;
     return launch_merge<DT, HD, TPP>(dp, stream);
   } else {
     // (tiles first: the decode's merge re-arms the claim word)

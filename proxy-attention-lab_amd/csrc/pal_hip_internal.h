@@ -107,6 +107,8 @@ hipError_t launch_decode(const DecodeParams& p, int dtype, int head_dim, int tok
 // say whether the call's clearing of them has begun, and is done.  (The counter
 // below the bits counts batches of 64 rows, fewer than 2^27.)
 constexpr int kTileClaims = 16;
+// kTilesOnly: the call's prefill tiles, all its rows, have been computed.
+constexpr uint32_t kTilesOnly = 1u << 29;
 constexpr uint32_t kClaimsTaken = 1u << 30;
 constexpr uint32_t kClaimsReady = 1u << 31;
 

@@ -396,16 +396,17 @@ def test_fused_fp8_pages(dtype, hd, tpp):
 
 @pytest.mark.parametrize("hd,tpp", [(64, 16), (64, 32), (128, 16), (128, 32), (256, 16)])
 @pytest.mark.parametrize("rows", [161, 300, 401])
-def test_fused_fp8_tile_sizes(rows, hd, tpp):
-    """Prefill tiles with a CU to themselves over fp8 pages: of one row group
-    (161 rows: 168 tiles on 8 kv heads of 16 query heads), of two (300: 152
-    tiles of 16 rows; head dims above 128: one), and beyond one round (401
-    rows on twice the kv heads)."""
+@pytest.mark.parametrize("decode", [[70], []], ids=["lone-row", "whole"])
+def test_fused_fp8_tile_sizes(decode, rows, hd, tpp):
+    """Prefill tiles with a CU to themselves over fp8 pages (with a lone row: half
+    tiles up to head dim 128): of one row group (161 rows: 168 tiles on 8 kv heads
+    of 16 query heads), of two (300: 152 tiles of 16 rows; head dims above 128:
+    one), and beyond one round (401 rows on twice the kv heads)."""
     from pal_cases import make_fused_case
 
     rng = np.random.default_rng(hd + tpp + rows)
     hkv = 16 if rows > 400 else 8
-    fc = make_fused_case(hd + tpp + rows, [70], [(45, rows)], 16 * hkv, hkv, hd, tpp, "bf16", block=rows)
+    fc = make_fused_case(hd + tpp + rows, decode, [(45, rows)], 16 * hkv, hkv, hd, tpp, "bf16", block=rows)
     c = fc.case
     kc, vc, ks, vs = fp8_case(c, rng)
     announce(f"fused fp8 tile sizes rows={rows} hd={hd} tpp={tpp}")

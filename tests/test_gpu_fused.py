@@ -189,17 +189,24 @@ def test_fused_query_magnitudes(dtype):
     assert np.isfinite(out).all()
 
 
-# (query heads, kv heads, decode lengths, chunks, block): few decode rows per
-# prefill row, so tiles have a CU to themselves from 1,200 (row, head of a group)
-# per sequence on: one side of that line and the other, tiles of one row group,
-# of two, and more tiles than CUs of either (claimed), windows that start
-# and end inside a run
+# (query heads, kv heads, decode lengths, chunks, block).  From 1,200 (row, head
+# of a group) per sequence on, tiles have a CU to themselves where no row is alone
+# in its run (found on the device if there is more than one sequence): one side of
+# that line and the other, with lone rows and without, tiles of one row group, of
+# two, and more tiles than CUs (256) of either (claimed), windows that start and
+# end inside a run
 TILE_CASES = {
     "beside-decode": (32, 8, [300], [(100, 598)], 600),            # 599 rows * 4 < 1200 * 2
-    "one-group": (32, 8, [300], [(100, 599)], 600),                # 600 rows * 4 = 1200 * 2; 152 tiles
-    "one-group-claimed": (32, 32, [], [(0, 1400)], 1400),          # 352 tiles of 128 rows
-    "two-groups": (128, 8, [], [(37, 300), (500, 1)], 300),        # 304 tiles of 8 rows, 152 of 16
-    "two-groups-claimed": (256, 16, [70], [(65, 401)], 401),       # 816 tiles of 8 rows, 416 of 16
+    "one-group": (32, 8, [300], [(100, 599)], 600),                # 600 rows * 4 = 1200 * 2, a lone row: half tiles
+    "whole-one-group": (32, 8, [], [(100, 598), (50, 2)], 600),    # 152 tiles
+    "whole-one-group-claimed": (104, 26, [], [(20, 590), (4, 12)], 590),  # 494 tiles of 32 rows, 260 of 64
+    "whole-two-groups": (128, 8, [], [(37, 300), (500, 2)], 300),  # 304 tiles of 8 rows, 152 of 16
+    "whole-two-groups-claimed": (256, 16, [], [(65, 401), (3, 5)], 401),  # 816 tiles of 8 rows, 416 of 16
+    "whole-runs": (64, 4, [], [(20, 1700), (3, 40)], 33),          # several runs to a window
+    "one-group-filled": (32, 32, [], [(0, 1400)], 1400),           # 352 tiles of 128 rows, 192 of 256: two groups
+    "one-group-claimed": (130, 130, [], [(0, 300)], 300),          # 390 tiles of 128 rows, 260 of 256: two rounds either way
+    "two-groups": (128, 8, [], [(37, 300), (500, 1)], 300),        # a lone row: half tiles
+    "two-groups-claimed": (256, 16, [70], [(65, 401)], 401),       # a lone row
     "lone-rows": (64, 4, [900] * 20 + [0], [(20, 1700), (3, 40)], 33),  # interleaved with blocks of runs
 }
 
@@ -216,11 +223,14 @@ def test_fused_tile_sizes(name, hd, tpp, dtype):
     assert np.array_equal(first, again)
 
 
-def test_fused_tile_claims_across_head_dims():
+@pytest.mark.parametrize("heads,rows", [((64, 32), 700), ((200, 100), 300)], ids=["by-place", "claimed"])
+def test_fused_tile_claims_across_head_dims(heads, rows):
     """Head dims above and up to 128 claim tiles in kernels of different launch
-    sequences, from the counters of one workspace."""
+    sequences, from the counters of one workspace.  700 rows of 32 kv heads make
+    352 tiles of one row group, which head dim 256 claims, and 192 of two, all
+    taken by place; 300 rows of 100 kv heads 500 or 300, claimed at every head dim."""
     for i, hd in enumerate([256, 64, 256, 32]):
-        _check_fused(make_fused_case(90 + i, [], [(10, 700)], 64, 32, hd, 16, "bf16", block=700), f"claims hd{hd}")
+        _check_fused(make_fused_case(90 + i, [], [(10, rows)], *heads, hd, 16, "bf16", block=rows), f"claims hd{hd}")
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
@@ -257,15 +267,18 @@ def test_fused_nan_stays_in_its_rows(decode, rows, heads, hd, tpp, dtype):
 
 
 @pytest.mark.parametrize("hd", [64, 256])
-@pytest.mark.parametrize("rows,heads", [(2200, (32, 32)), (700, (64, 16)), (2300, (128, 8))],
-                         ids=["one-group", "few", "two-groups"])
-def test_fused_workspace_contract(rows, heads, hd):
+@pytest.mark.parametrize("rows,heads,others", [(2200, (32, 32), None), (700, (64, 16), None), (2300, (128, 8), None),
+                                               (2300, (128, 8), 30), (700, (64, 16), 1), (700, (32, 32), 1)],
+                         ids=["one-group", "few", "two-groups", "two-sequences", "lone-row", "beside-decode"])
+def test_fused_workspace_contract(rows, heads, others, hd):
     """Of the workspace, the four bytes at 64 are all that has to be zero before
     a call (head dim 64: 576 tiles of one row group on 256 CUs; 352 of one, 176
-    of two; 2,304 / 1,152: claimed, all taken by place, claimed), and are zero again
-    after it."""
+    of two; 2,304 / 1,152: claimed, all taken by place, claimed; the last again with
+    a second sequence of 30 rows, so that the device decides for them, and batches
+    with a lone row above and below that line), and are zero again after it."""
     hq, hkv = heads
-    fc = make_fused_case(rows + hd, [], [(10, rows)], hq, hkv, hd, 16, "bf16", block=rows)
+    chunks = [(10, rows)] + ([(25, others)] if others else [])
+    fc = make_fused_case(rows + hd, [], chunks, hq, hkv, hd, 16, "bf16", block=rows)
     c = fc.case
     announce(f"fused workspace contract rows={rows} heads={heads} HD={hd}")
     ref = host_bits(_fused_gpu(c, fc.queries, fc.q2seq, fc.q_offset))
