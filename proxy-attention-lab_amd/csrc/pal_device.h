@@ -107,6 +107,9 @@ struct Dt<kBF16> {
     return __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(__builtin_bit_cast(s16x4, a), __builtin_bit_cast(s16x4, b), c, 0, 0, 0);
   }
   static constexpr uint32_t kOnes = 0x3F803F80u;  // a packed pair of ones
+  // the values of a packed pair
+  static __device__ __forceinline__ float lo(uint32_t w) { return __uint_as_float(w << 16); }
+  static __device__ __forceinline__ float hi(uint32_t w) { return __uint_as_float(w & 0xFFFF0000u); }
   // two fp8 e4m3 values (bytes 0-1, or 2-3 when hi) of w as a packed pair;
   // exact (every e4m3 value is a bf16 value): one v_cvt_scalef32_pk_bf16_fp8
   // with scale 1
@@ -145,6 +148,8 @@ struct Dt<kF16> {
     return __builtin_amdgcn_mfma_f32_4x4x4f16(__builtin_bit_cast(f16x4, a), __builtin_bit_cast(f16x4, b), c, 0, 0, 0);
   }
   static constexpr uint32_t kOnes = 0x3C003C00u;
+  static __device__ __forceinline__ float lo(uint32_t w) { return static_cast<float>(__builtin_bit_cast(f16x2, w)[0]); }
+  static __device__ __forceinline__ float hi(uint32_t w) { return static_cast<float>(__builtin_bit_cast(f16x2, w)[1]); }
   // two fp8 e4m3 values as a packed pair; exact (e4m3's range and 3-bit
   // mantissa fit fp16, subnormals included): one v_cvt_scalef32_pk_f16_fp8
   // with scale 1
@@ -397,16 +402,15 @@ __device__ __forceinline__ u32x2 lds_read_tr16(const uint16_t* p) {
   return __builtin_bit_cast(u32x2, r);
 }
 
-// acc + the lane's own 8 packed values p, in every register of acc: two 4x4x4
-// products of 16 blocks, against an A of ones (block l / 4, column l % 4 is
-// lane l's, so a NaN or infinity in one lane reaches no other lane's sum).  They
-// hold the matrix pipe for 16 cycles together; as many v_dot2c of one pair each
-// would take 64, and adds of the unrounded values 8 vector instructions.
+// acc + the lane's own 4 packed values p, in every register of acc: a 4x4x4
+// product of 16 blocks, against an A of ones (block l / 4, column l % 4 is lane
+// l's, so a NaN or infinity in one lane reaches no other lane's sum).  It holds
+// the matrix pipe for 8 cycles; two v_dot2c of one pair each would take 32, and
+// adds of the unrounded values 4 vector instructions.  Two on one accumulator
+// stand apart (each waits for the previous one's result).
 template <int DT>
-__device__ __forceinline__ f32x4 lane_sum8(u32x4 p, f32x4 acc) {
-  constexpr u32x2 ones = {Dt<DT>::kOnes, Dt<DT>::kOnes};
-  acc = Dt<DT>::mma4x4x4(ones, u32x2{p.x, p.y}, acc);
-  return Dt<DT>::mma4x4x4(ones, u32x2{p.z, p.w}, acc);
+__device__ __forceinline__ f32x4 lane_sum4(u32x2 p, f32x4 acc) {
+  return Dt<DT>::mma4x4x4(u32x2{Dt<DT>::kOnes, Dt<DT>::kOnes}, p, acc);
 }
 
 // Scheduling fence: the compiler's instruction scheduler moves nothing

@@ -791,8 +791,11 @@ __device__ __forceinline__ void half_tile(const PrefillParams& p, int row0, int 
           copy_one(m, j % kNBuf, joff0, joff1);
       }
       o[m % DT32] = Dt<DT>::mma32x32x16(va[m], pb[m / DT32], o[m % DT32]);
-      if constexpr (!F8)
-        if (m % DT32 == 0) l_sum = lane_sum8<DT>(pb[m / DT32], l_sum);
+      if constexpr (!F8) {  // 4 of the lane's 8 values each in the first two chunks of a k-step
+        const u32x4 pv = pb[m / DT32];
+        if (m % DT32 == 0) l_sum = lane_sum4<DT>(u32x2{pv.x, pv.y}, l_sum);
+        if (m % DT32 == (DT32 > 1 ? 1 : 0)) l_sum = lane_sum4<DT>(u32x2{pv.z, pv.w}, l_sum);
+      }
 #pragma unroll
       for (int r = m * 16 / KS; r < (m + 1) * 16 / KS; ++r) {
         if (kMask) mask_score(s_next, r, st + 1);

@@ -36,8 +36,8 @@
 //    instruction.  In the transposed products a lane owns one M-row, so the
 //    softmax max needs one cross-half exchange (v_permlane32_swap) and the
 //    probabilities go into the PV MFMA without leaving the lane.  The sum of
-//    the rounded probabilities comes from MFMAs with ones, each lane's own
-//    (v_dot2 holds the matrix pipe for 16 cycles each).  K is stored in the QK operand's row
+//    the rounded probabilities is each lane's own, from MFMAs with ones (v_dot2
+//    holds the matrix pipe for 16 cycles each) or from vector adds.  K is stored in the QK operand's row
 //    order and V rows are swizzled, so every operand read is one conflict-free
 //    16-byte LDS access.
 //  * Steps are software-pipelined inside a wavefront: the QK MFMAs of step
@@ -753,9 +753,14 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
   // row's first score above -inf: with it the exponent of -inf is -inf, and that
   // of any other score so far past the headroom that the max moves to it.
   float mb[RG];
-  // this lane's share of the exp-sum: of the probabilities as rounded for the
-  // PV product, by MFMA (register 0; fp8: of the probabilities before the V scale)
-  f32x4 l_sum[F8 ? 1 : RG];
+  // this lane's share of the exp-sum: of the probabilities as rounded for the PV
+  // product, by MFMA (l_sum, register 0) or, in the longest steps, whose matrix
+  // pipe is the busier one, by unpacking and adding (l_run; two row groups at head
+  // dim 128, 16 x 1,024 prompt rows on 1,024 cached: 436 -> 425 us; at head dim 64 280 ->
+  // 304, one row group 70.4 -> 71.3); over fp8 pages of the probabilities before
+  // the V scale (l_run)
+  constexpr bool kMmaSum = !F8 && !(RG == 2 && HD >= 128);
+  f32x4 l_sum[kMmaSum ? RG : 1];
   float l_run[RG];
   // O^T of row group r, row tile n (dims 32 n ..): accumulator r * DT32 + n
   static_assert(RG * DT32 <= 8, "eight accumulators");
@@ -765,7 +770,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
   for (int r = 0; r < RG; ++r) {
     mb[r] = 0.f;
     l_run[r] = 0.f;
-    if constexpr (!F8) l_sum[r] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if constexpr (kMmaSum) l_sum[r] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
 
   // Key order inside a 32-key step.  The QK product's A operand takes key
@@ -1025,10 +1030,11 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
       if (i % 4 == 3) asm volatile("" : "+v"(pp[r][i / 4]));
     };
     auto pair_sum = [&](int q) {
-      if constexpr (!F8) return;
+      if constexpr (kMmaSum) return;
       const int r = q / 8, i = q % 8;
-      l_run[r] += e_cur[r][2 * i];
-      l_run[r] += e_cur[r][2 * i + 1];
+      const uint32_t w = pp[r][i / 4][i % 4];
+      l_run[r] += F8 ? e_cur[r][2 * i] : Dt<DT>::lo(w);
+      l_run[r] += F8 ? e_cur[r][2 * i + 1] : Dt<DT>::hi(w);
     };
     constexpr int kPairs = 8 * RG;
     // row group 0's share of the exp-sum goes beside the QK MFMAs, row group
@@ -1131,11 +1137,18 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
           if (q < kSumA) pair_sum(q);
         }
       }
-      if constexpr (!F8) {  // the exp-sum's MFMAs, a pair per row group and PV k-step
+      if constexpr (kMmaSum) {  // the exp-sum's MFMAs: a quarter of each row group's probabilities per chunk
         constexpr int kAt = NCH >= 8 ? 2 : 0;  // (every probability is packed by the end of chunk 0)
-        if (c >= kAt && c < kAt + 2 * RG) {
-          const int x = c - kAt;
-          l_sum[x % RG] = lane_sum8<DT>(pp[x % RG][x / RG], l_sum[x % RG]);
+        constexpr int kIn = NCH - kAt < 4 ? NCH - kAt : 4;
+        if (c >= kAt && c < kAt + kIn) {
+#pragma unroll
+          for (int q = (c - kAt) * 4 / kIn; q < (c - kAt + 1) * 4 / kIn; ++q) {
+#pragma unroll
+            for (int x = 0; x < RG; ++x) {
+              const u32x4 pv = pp[x][q / 2];
+              l_sum[x] = lane_sum4<DT>(q % 2 ? u32x2{pv.z, pv.w} : u32x2{pv.x, pv.y}, l_sum[x]);
+            }
+          }
         }
       }
       if constexpr (RG == 2) {  // before chunk kFirst + (NCH - kFirst) / 2
@@ -1179,8 +1192,8 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
           scale[r] = __builtin_amdgcn_exp2f(m_new - mb[r]);
           mb[r] = m_new;
           exponents(r, st + 1, kMode == kAny, s_next[r], sc);
-          if constexpr (F8) l_run[r] *= scale[r];
-          else l_sum[r][0] *= scale[r];
+          if constexpr (kMmaSum) l_sum[r][0] *= scale[r];
+          else l_run[r] *= scale[r];
         }
         static_for<RG * DT32 * 16>([&](auto x) {
           constexpr int X = decltype(x)::value;
@@ -1253,8 +1266,8 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
     constexpr int r = decltype(rc)::value;
     uint16_t* region = k_lds_base + (w * RG + r) * 32 * HD;  // K buffers, then V buffers: 8 regions of 32 rows
     float l;
-    if constexpr (F8) l = sum_xor32(l_run[r]);
-    else l = sum_xor32(l_sum[r][0]);
+    if constexpr (kMmaSum) l = sum_xor32(l_sum[r][0]);
+    else l = sum_xor32(l_run[r]);
     const float inv = l > 0.f ? 1.f / l : 0.f;
     static_for<DT32 * 4>([&](auto qc) {
       constexpr int c = decltype(qc)::value, n = c / 4, q4 = c % 4;
