@@ -36,7 +36,7 @@
 //    instruction.  In the transposed products a lane owns one M-row, so the
 //    softmax max needs one cross-half exchange (v_permlane32_swap) and the
 //    probabilities go into the PV MFMA without leaving the lane.  The sum of
-//    the rounded probabilities is each lane's own, from MFMAs with ones (v_dot2
+//    the rounded probabilities comes from two MFMAs with ones per step (v_dot2
 //    holds the matrix pipe for 16 cycles each) or from vector adds.  K is stored in the QK operand's row
 //    order and V rows are swizzled, so every operand read is one conflict-free
 //    16-byte LDS access.
@@ -753,15 +753,16 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
   // row's first score above -inf: with it the exponent of -inf is -inf, and that
   // of any other score so far past the headroom that the max moves to it.
   float mb[RG];
-  // this lane's share of the exp-sum: of the probabilities as rounded for the PV
-  // product, by MFMA (l_sum, register 0) or, in the longest steps, whose matrix
-  // pipe is the busier one, by unpacking and adding (l_run; two row groups at head
-  // dim 128, 16 x 1,024 prompt rows on 1,024 cached: 436 -> 425 us; at head dim 64 280 ->
-  // 304, one row group 70.4 -> 71.3); over fp8 pages of the probabilities before
-  // the V scale (l_run)
+  // exp-sum: of the probabilities as rounded for the PV product, by MFMA (kMmaSum:
+  // the whole row's, in every lane) or by unpacking and adding; over fp8 pages of
+  // the probabilities before the V scale (both: this lane's share).  Adds where the
+  // steps are longest and the matrix pipe is the busier one: two row groups at
+  // head dim 128, 16 x 1,024 prompt rows on 1,024 cached 436 -> 425 us; at head dim 64
+  // 275 -> 304, one row group 67 -> 71.
   constexpr bool kMmaSum = !F8 && !(RG == 2 && HD >= 128);
-  f32x4 l_sum[kMmaSum ? RG : 1];
   float l_run[RG];
+  // kMmaSum: the last step's, not yet in l_run, of M-rows 0 .. 15 and 16 .. 31 of the group
+  float step_lo[RG], step_hi[RG];
   // O^T of row group r, row tile n (dims 32 n ..): accumulator r * DT32 + n
   static_assert(RG * DT32 <= 8, "eight accumulators");
   acc_reserve();
@@ -769,8 +770,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
 #pragma unroll
   for (int r = 0; r < RG; ++r) {
     mb[r] = 0.f;
-    l_run[r] = 0.f;
-    if constexpr (kMmaSum) l_sum[r] = f32x4{0.f, 0.f, 0.f, 0.f};
+    l_run[r] = step_lo[r] = step_hi[r] = 0.f;
   }
 
   // Key order inside a 32-key step.  The QK product's A operand takes key
@@ -974,6 +974,15 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
       exponents(r, 0, min_lim < kKeys, s0[r], sc);
     }
   }
+  auto take_sums = [&] {  // the last step's exp-sums into the running ones
+    if constexpr (kMmaSum) {
+#pragma unroll
+      for (int r = 0; r < RG; ++r) {
+        l_run[r] += (lane & 16) ? step_hi[r] : step_lo[r];
+        step_lo[r] = step_hi[r] = 0.f;
+      }
+    }
+  };
   // One iteration.  kFast: step st+1 needs no mask and the iteration's copies
   // are plain (pages known to be valid, or whole dense steps): no test of a
   // page id and no branch in the body.  Otherwise scores are masked and each
@@ -992,6 +1001,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
     } else {
       wait_top(st);
     }
+    take_sums();
     const int jk = st + kLeadK, jv = st + kLeadV;
     const u32x2 pgk = read_pids(jk), pgv = read_pids(jv);  // used in the second half (in bounds whether or not the steps exist)
     if (kMode == kAny && st + 2 == nsteps && tail_partial) fix_tail(st + 1);
@@ -1137,20 +1147,6 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
           if (q < kSumA) pair_sum(q);
         }
       }
-      if constexpr (kMmaSum) {  // the exp-sum's MFMAs: a quarter of each row group's probabilities per chunk
-        constexpr int kAt = NCH >= 8 ? 2 : 0;  // (every probability is packed by the end of chunk 0)
-        constexpr int kIn = NCH - kAt < 4 ? NCH - kAt : 4;
-        if (c >= kAt && c < kAt + kIn) {
-#pragma unroll
-          for (int q = (c - kAt) * 4 / kIn; q < (c - kAt + 1) * 4 / kIn; ++q) {
-#pragma unroll
-            for (int x = 0; x < RG; ++x) {
-              const u32x4 pv = pp[x][q / 2];
-              l_sum[x] = lane_sum4<DT>(q % 2 ? u32x2{pv.z, pv.w} : u32x2{pv.x, pv.y}, l_sum[x]);
-            }
-          }
-        }
-      }
       if constexpr (RG == 2) {  // before chunk kFirst + (NCH - kFirst) / 2
 #pragma unroll
         for (int q = c * 8 / (NCH / 2); q < (c + 1) * 8 / (NCH / 2); ++q)
@@ -1173,6 +1169,27 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
       }
       sched_fence();
     }
+    if constexpr (kMmaSum) {
+      // The step's exp-sums, the probabilities' registers being free now: the
+      // 16-lane groups of the two k-steps are exchanged so that one operand holds
+      // all of M-rows 0 .. 15 and the other of 16 .. 31, each four k-groups of a
+      // column of its own.  (Without the exchange a column would hold two rows,
+      // kept apart by zeros, and a NaN in one would reach the other.)
+#pragma unroll
+      for (int r = 0; r < RG; ++r) {
+        u32x4 lo = pp[r][0], hi = pp[r][1];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const auto t = __builtin_amdgcn_permlane16_swap(lo[i], hi[i], false, false);
+          lo[i] = t[0];
+          hi[i] = t[1];
+        }
+        constexpr u32x4 ones = {Dt<DT>::kOnes, Dt<DT>::kOnes, Dt<DT>::kOnes, Dt<DT>::kOnes};
+        const f32x4 none = {0.f, 0.f, 0.f, 0.f};
+        step_lo[r] = Dt<DT>::mma16x16x32(ones, lo, none)[0];
+        step_hi[r] = Dt<DT>::mma16x16x32(ones, hi, none)[0];
+      }
+    }
     if constexpr (kMode == kLast) {
       acc_settle();
     } else {
@@ -1192,9 +1209,10 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
           scale[r] = __builtin_amdgcn_exp2f(m_new - mb[r]);
           mb[r] = m_new;
           exponents(r, st + 1, kMode == kAny, s_next[r], sc);
-          if constexpr (kMmaSum) l_sum[r][0] *= scale[r];
-          else l_run[r] *= scale[r];
         }
+        take_sums();
+#pragma unroll
+        for (int r = 0; r < RG; ++r) l_run[r] *= scale[r];
         static_for<RG * DT32 * 16>([&](auto x) {
           constexpr int X = decltype(x)::value;
           acc_put<X>(acc_get<X>() * scale[X / (DT32 * 16)]);
@@ -1255,6 +1273,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
   // region per row group, 16-byte chunk c of row i at chunk c ^ i, so that both
   // sides spread over the banks) and out as whole rows, 16 bytes per lane,
   // non-temporally (nothing here reads them again).
+  take_sums();
   if (nsteps == 0) {
     acc_zero();
     acc_settle();
@@ -1266,7 +1285,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int row0, i
     constexpr int r = decltype(rc)::value;
     uint16_t* region = k_lds_base + (w * RG + r) * 32 * HD;  // K buffers, then V buffers: 8 regions of 32 rows
     float l;
-    if constexpr (kMmaSum) l = sum_xor32(l_sum[r][0]);
+    if constexpr (kMmaSum) l = l_run[r];
     else l = sum_xor32(l_run[r]);
     const float inv = l > 0.f ? 1.f / l : 0.f;
     static_for<DT32 * 4>([&](auto qc) {
