@@ -42,8 +42,9 @@
 //    16-byte LDS access.
 //  * Steps are software-pipelined inside a wavefront: the QK MFMAs of step
 //    st+1 are issued among the exponentials of step st, the row max of step
-//    st+1 and the step's copies among the PV MFMAs.  A whole unmasked step of
-//    128 dims takes 1,470 cycles with RG = 2, 1,050 of them MFMA.
+//    st+1 and the step's copies among the PV MFMAs.  Over ragged chunks a
+//    step of 128 dims takes 2,090 cycles of a wavefront with RG = 2, masked
+//    steps, tile set-up and waits included, 1,024 of them MFMA.
 //  * Online softmax in log2 units, scale and max folded into one fma per score,
 //    with a lazy rescale: the running max is only moved when a score exceeds
 //    it by more than 2^8, so O is rescaled rarely.
@@ -52,9 +53,9 @@
 //  * The output leaves through LDS as whole rows of 16-byte stores.
 //  * Measured (bf16, 32 query heads on 8 kv heads, head dim 128), against 32
 //    rows per wavefront and two workgroups per CU: 16 sequences of 1,280 rows
-//    on 1,024 cached 0.76 -> 0.62 ms (0.90 PFLOP/s over the keys seen); one
-//    prompt of 768 rows 32.4 -> 19.5 us (RG 1).  Under this load
-//    the card's clock falls to about 1.9 GHz.
+//    on 1,024 cached 670 -> 570 us (0.98 PFLOP/s over the keys seen); one prompt
+//    of 777 rows 29.6 -> 19.2 us (RG 1).  Under this load the card's clock falls
+//    to about 1.9 GHz.
 //  * Two ways to name the work, both without a planning pass: the reference
 //    prefill's uniform prompt (S sequences x P prompt rows; tiles are pure
 //    arithmetic; keys [0, hist[s]) come from pages and keys hist[s] + i from
@@ -1432,9 +1433,7 @@ __device__ __forceinline__ void prefill_item(const PrefillParams& p, unsigned it
 }
 
 // The prefill's items on a resident grid, one workgroup per CU: a workgroup
-// that starts on a CU pays several us before its first load (measured: 6.5 us
-// between a workgroup's end and its successor's first instruction on the same
-// CU, tiles of 30-60 us).
+// that starts on a CU pays several us before its first load (tiles take 30 to 60).
 //  * Window mode: items are claimed, the first by place (workgroup b starts on
 //    item b).  Lengths differ by item, and a static share left CUs idle for up
 //    to a fifth of the time (16 sequences of 512 to 2,048 rows on 0 to 2,048

@@ -117,9 +117,9 @@ def _workspace(kind: str, nbytes: int, device: torch.device, stream_handle: int)
     """Zero-initialised workspace per (operator, device, stream), kept for the
     streams used most recently.
 
-    The decode kernels keep a work-claim counter in it that must read zero
-    when a call starts; every call leaves it zero again, so the buffer is
-    reused as is by the next call of the same operator on the same stream
+    The kernels keep a claim word in it (a counter, and two bits for the fused
+    op's tile counters) that must read zero when a call starts; every call
+    leaves it zero again, so the buffer is reused as is by the next call of the same operator on the same stream
     (calls on one stream never overlap).  A larger request replaces it with a
     new zeroed buffer.  At most ``_WORKSPACES_PER_DEVICE`` streams keep one
     per (operator, device); the least recently used is dropped beyond that.
