@@ -127,6 +127,14 @@ def test_prefill_long_history_page_id_chunks(tpp, hist):
     _check(31 + tpp, hist, 48, 32, 8, 128, tpp, "bf16", f"long history tpp{tpp}")
 
 
+@pytest.mark.parametrize("hd,heads,tpp,hist,dtype", [(256, (8, 2), 16, [26000, 9000], "bf16"), (256, (4, 1), 32, [40000, 300], "f16"),
+                                                     (96, (300, 300), 16, [17000], "bf16")])
+def test_prefill_half_tiles_long_history(hd, heads, tpp, hist, dtype):
+    """The same for half tiles: head dim 256, and 300 kv heads (300 tiles of one row
+    group on 256 CUs, more than one round)."""
+    _check(hd + tpp, hist, 40, *heads, hd, tpp, dtype, f"half tiles, long history hd{hd} tpp{tpp}")
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("hd", [32, 64, 96, 128, 256])
 def test_prefill_dense_prompt_steps(hd, dtype):
